@@ -29,8 +29,9 @@
  *
  * Ordering: every call enqueues on the caller's hipStream_t and returns
  * without synchronising.  A context is not thread-safe: use one per host
- * thread, or serialise.  A context owns scratch memory that its GEMM calls
- * write and read on the device (the split-K partial sums, the int8 route's
+ * thread, or serialise.  A context owns scratch memory that its GEMM and
+ * attention calls write and read on the device (the split-K partial sums,
+ * the partial outputs of attention split over the keys, the int8 route's
  * codes and scales, the dequant expansion), so ALL calls on one context
  * must be ordered on ONE stream (or otherwise ordered by the caller, e.g.
  * with events): two calls on one context queued on unordered streams race
@@ -317,7 +318,11 @@ u15h_status u15h_build_rope_tables(const int32_t* pos_t, const int32_t* pos_h,
  *   query head h reads kv head h / (hq / hkv)  (the GQA group size)
  *   softmax(q.k / sqrt(d)) . v, f32 accumulation; causal: key j attends
  *   iff j <= q_offset + i (queries sit at q_offset within the keys).
- * d in {32, 64, 128}; hq % hkv == 0; tk <= cap. */
+ * d in {32, 64, 128}; hq % hkv == 0; tk <= cap.
+ * A few queries over many keys (decode, a line of text after cached images)
+ * split the keys over workgroups, whose f32 partial outputs go to the
+ * context's scratch (32 MiB, allocated by u15h_create; without it, or with
+ * env U15H_ATTN_SPLIT=0, no call splits). */
 u15h_status u15h_sdpa(u15h_ctx* ctx, u15h_stream stream, const u15h_bf16* q,
                       const u15h_bf16* k, const u15h_bf16* v, u15h_bf16* out,
                       int hq, int hkv, int tq, int tk, int d, int cap,

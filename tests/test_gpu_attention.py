@@ -298,3 +298,88 @@ def test_token_major_masked_matches_head_major(ops, mode):
     torch.cuda.synchronize()
     assert torch.equal(ot.view(tq, hq, d).transpose(0, 1).contiguous().view(torch.int16),
                        out.view(torch.int16))
+
+
+def ctx_with(value):
+    """A context created with U15H_ATTN_SPLIT=value (read at create)."""
+    import os
+    old = os.environ.get("U15H_ATTN_SPLIT")
+    os.environ["U15H_ATTN_SPLIT"] = str(value)
+    try:
+        return u15h.Ops(0)
+    finally:
+        if old is None:
+            del os.environ["U15H_ATTN_SPLIT"]
+        else:
+            os.environ["U15H_ATTN_SPLIT"] = old
+
+
+# (hq, hkv, d, tq, prefix, mode, shares): rows = tq * hq / hkv at the edges
+# of the 1-, 2- and 4-wave builds and of a 32-row group; more shares than a
+# causal block has tiles (empty shares); one tile per share; up to 8 and
+# above 8 shares (the combine's two builds); a group of 3 and of 1 heads.
+SPLIT_CASES = [
+    (4, 1, 128, 1, 700, "causal", 11), (8, 2, 128, 8, 130, "bidirectional", 3),
+    (8, 2, 128, 9, 257, "block_causal", 5), (8, 2, 128, 16, 300, "causal", 9),
+    (6, 2, 128, 22, 191, "block_causal", 4), (8, 2, 128, 33, 400, "bidirectional", 2),
+    (4, 1, 64, 41, 640, "causal", 7), (4, 4, 64, 200, 64, "block_causal", 4),
+    (4, 2, 32, 65, 200, "causal", 5), (2, 1, 32, 3, 1000, "bidirectional", 40),
+    (4, 1, 128, 130, 0, "causal", 4), (4, 1, 128, 1, 0, "causal", 2),
+]
+
+
+@pytest.mark.parametrize("hq,hkv,d,tq,prefix,mode,shares", SPLIT_CASES)
+def test_keys_split_over_workgroups(hq, hkv, d, tq, prefix, mode, shares):
+    """The split kernel against the oracle at the reference's bar, with a
+    NaN-filled cache tail; head-major and token-major calls agree bit for
+    bit, and a repeat gives the same bits (the shares are added in one
+    order)."""
+    rng = np.random.default_rng(hq + d + tq + prefix)
+    tk = prefix + tq
+    cap = tk + 70
+
+    def bits(*shape):
+        return oracle.f32_to_bf16(rng.standard_normal(shape).astype(np.float32))
+    qb = bits(hq, tq, d)
+    kb = bf16_cache(widen(bits(hkv, tk, d)), cap, np.nan)
+    vb = bf16_cache(widen(bits(hkv, tk, d)), cap, np.nan)
+    t_idx = np.arange(tk, dtype=np.int32)
+    at = prefix + tq // 3
+    t_idx[at:] = at                                  # an image block to the end
+    q, k, v = dev_bf16(qb), dev_bf16(kb), dev_bf16(vb)
+    t = torch.from_numpy(t_idx).cuda()
+    qt = q.transpose(0, 1).contiguous().view(tq, hq * d)
+    ops = ctx_with(shares)
+    code = {"bidirectional": 0, "causal": 1, "block_causal": 2}[mode]
+    outs = []
+    for _ in range(2):
+        out = torch.full_like(qt, 7.0)
+        ops.attention_token_major(qt, k, v, out, hq, hkv, tk, code, t, prefix)
+        outs.append(out)
+    head = torch.full_like(q, 7.0)
+    if mode == "block_causal":
+        ops.sdpa_block_causal(q, k, v, head, t, hkv, tk, prefix)
+    else:
+        ops.sdpa(q, k, v, head, hkv, tk, mode == "causal", prefix)
+    torch.cuda.synchronize()
+    ops.close()
+    assert torch.equal(outs[0], outs[1])
+    assert torch.equal(head.transpose(0, 1).contiguous().view(tq, hq * d), outs[0])
+    ref = oracle.attention(widen(qb), widen(kb)[:, :tk].copy(), widen(vb)[:, :tk].copy(), hkv,
+                           tk, mode, t_idx, q_offset=prefix)
+    assert rel_l2(host_f32(head), ref) < BAR
+
+
+@pytest.mark.parametrize("hq,tq", [(4, 1), (4, 127), (4, 128), (4, 129), (4, 257),
+                                   (256, 255), (128, 257)])
+def test_bidirectional_workgroup_sizes(ops, hq, tq):
+    """Both workgroup sizes of the bidirectional mask around their query
+    tiles' edges: four waves where the eight-wave grid leaves CUs idle (4
+    heads), eight where it fills them."""
+    hkv, d, tk = hq // 2, 32, 70
+    rng = np.random.default_rng(tq)
+    qb, kb, vb = (oracle.f32_to_bf16(rng.standard_normal((h, n, d)).astype(np.float32))
+                  for h, n in ((hq, tq), (hkv, tk), (hkv, tk)))
+    got = run_sdpa(ops, qb, kb, vb, hkv, tk)
+    ref = oracle.attention(widen(qb), widen(kb), widen(vb), hkv, tk, "bidirectional")
+    assert rel_l2(got, ref) < BAR

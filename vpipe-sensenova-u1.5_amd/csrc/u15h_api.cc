@@ -49,6 +49,12 @@ struct u15h_ctx {
   // lookup failed, with the HIP error kept for the message).
   void* noalloc_ws = nullptr;
   hipError_t noalloc_err = hipSuccess;
+  // Split attention's partial results (attn_split_ws_bytes; allocated at
+  // create so that no attention call allocates, null if that failed: then
+  // no call splits) and env U15H_ATTN_SPLIT: -1 the planner's key shares,
+  // 0 none, n >= 2 that many.
+  void* attn_ws = nullptr;
+  int attn_split = -1;
   bool i8_on = false;
   int i8_min_m = 1024;
   // Grow-only scratch of the int8 route of u15h_linear: activation and
@@ -167,6 +173,9 @@ empty_batch(int kbytes)
   b.split = 1;
   return b;
 }
+
+// Scratch of split attention calls, per context.
+constexpr size_t kAttnWsBytes = (size_t)32 << 20;
 
 // Fewest K stages a split share may have.
 constexpr int kMinStagesPerShare = 4;
@@ -512,8 +521,10 @@ u15h_create(int device, u15h_ctx** out)
   void* noalloc_ws = nullptr;
   const hipError_t noalloc_err = ok ? u15h::noalloc_scratch(device, &noalloc_ws)
                                     : hipErrorNotReady;
-  if (prev >= 0 && prev != device) { (void)hipSetDevice(prev); }
-  if (!ok) { return U15H_ENODEV; }
+  if (!ok) {
+    if (prev >= 0 && prev != device) { (void)hipSetDevice(prev); }
+    return U15H_ENODEV;
+  }
   u15h_ctx* ctx = new u15h_ctx;
   ctx->device = device;
   ctx->noalloc_ws = noalloc_ws;
@@ -532,6 +543,12 @@ u15h_create(int device, u15h_ctx** out)
   ctx->gemm.cus = env_int("U15H_PERSIST", 1) != 0 ? ctx->gemm_cus : 0;
   ctx->gemm.mfma16 = std::max(-1, std::min(1, env_int("U15H_MFMA16", 1)));
   ctx->i8_min_m = std::max(1, env_int("U15H_I8_MIN_M", 1024));
+  ctx->attn_split = env_int("U15H_ATTN_SPLIT", -1);
+  if (ctx->attn_split != 0 && hipMalloc(&ctx->attn_ws, kAttnWsBytes) != hipSuccess) {
+    ctx->attn_ws = nullptr;
+    (void)hipGetLastError();
+  }
+  if (prev >= 0 && prev != device) { (void)hipSetDevice(prev); }
   *out = ctx;
   return U15H_OK;
 }
@@ -548,6 +565,10 @@ u15h_destroy(u15h_ctx* ctx)
   if (ctx->split_ws != nullptr) {
     (void)hipDeviceSynchronize();
     (void)hipFree(ctx->split_ws);
+  }
+  if (ctx->attn_ws != nullptr) {
+    (void)hipDeviceSynchronize();
+    (void)hipFree(ctx->attn_ws);
   }
   delete ctx;
 }
@@ -1265,6 +1286,42 @@ u15h_repack_affine_i8(u15h_ctx* ctx, u15h_stream stream,
                   "repack_affine_i8");
 }
 
+// Key shares of an attention call (1: not split).  The unsplit kernel takes
+// ~0.94 us per 64-key tile on a workgroup that has its CU to itself, so a
+// few queries over a long cache leave the GPU idle; a split call pays ~6 us
+// of fixed cost more (two launches, the partial sums' round trip).  Lines
+// from measured calls (32 query heads over 8, d = 128, us in a graph, not
+// split / split): 1 query over 200 keys 8.8 / 9.4, over 1500 27.5 / 10.1,
+// over 4000 63.5 / 11.4; 41 over 2345 40.2 / 16.3; 128 over 3128 52.5 /
+// 25.1; 333 over 2333 42.5 / 30.4; 512 over 512 causal 15.0 / 21.3; 700
+// over 1700 50.4 / 48.1.
+//  - at least 12 key tiles (of the mean query, for the causal masks);
+//  - unsplit workgroups on at most 3/4 of the CUs;
+//  - shares of 1 tile or more (one-wave workgroups, at most 32 shares), 3
+//    (two waves) or 4 (four), two workgroups per CU at most.
+static int
+attention_shares(const u15h_ctx* ctx, u15h::AttnArgs a)
+{
+  if (ctx->attn_ws == nullptr || (long long)a.hq * a.tq > (1 << 20)) { return 1; }
+  const int rows = a.tq * (a.hq / a.hkv);
+  const int waves = u15h::attn_split_waves(rows);
+  const long long blocks = (long long)a.hkv * ((rows + 32 * waves - 1) / (32 * waves));
+  long long S = ctx->attn_split;
+  if (S < 0) {
+    const long long seen = a.mode == 0 ? a.tk : std::min<long long>(a.tk, a.q_offset + a.tq / 2);
+    const long long tiles = (seen + 63) / 64;
+    if (tiles < 12 || 4LL * a.hq * ((a.tq + 127) / 128) > 3LL * ctx->num_cu) { return 1; }
+    S = std::min(waves == 1 ? std::min(tiles, 32LL) : tiles / (waves == 2 ? 3 : 4),
+                 2LL * ctx->num_cu / blocks);
+  }
+  S = std::min<long long>(S, (a.tk + 63) / 64);
+  for (; S > 1; --S) {
+    a.shares = (int)S;
+    if (u15h::attn_split_ws_bytes(a) <= kAttnWsBytes) { return (int)S; }
+  }
+  return 1;
+}
+
 static u15h_status
 attention_call(u15h_ctx* ctx, u15h_stream stream, const u15h_bf16* q,
                const u15h_bf16* k, const u15h_bf16* v, u15h_bf16* out,
@@ -1312,6 +1369,9 @@ attention_call(u15h_ctx* ctx, u15h_stream stream, const u15h_bf16* q,
   a.q_offset = q_offset;
   a.d = d;
   a.mode = mode;
+  a.shares = attention_shares(ctx, a);
+  a.ws = ctx->attn_ws;
+  a.cus = ctx->num_cu;
   return launched(ctx, u15h::launch_attention(a, as_stream(stream)), what);
 }
 

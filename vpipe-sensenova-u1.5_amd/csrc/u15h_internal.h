@@ -192,7 +192,23 @@ struct AttnArgs {
   const int32_t* t_index;
   long long q_head, q_tok, o_head, o_tok;
   int hq, hkv, tq, tk, cap, q_offset, d, mode;
+  // > 1: the keys are split over that many workgroups per row block, whose
+  // f32 partial results go to ws (attn_split_ws_bytes of it)
+  int shares;
+  void* ws;
+  int cus;                // compute units (the workgroup size's rule)
 };
+// Split attention: rows (query heads of a kv head's group x tokens) per
+// workgroup in units of 32, and the scratch of one share of 32 rows (f32
+// output, running max and sum) and of a whole call.
+constexpr int attn_split_waves(int rows) { return rows <= 32 ? 1 : rows <= 64 ? 2 : 4; }
+constexpr size_t attn_split_bytes(int d) { return (size_t)32 * d * 4 + 32 * 8; }
+inline size_t attn_split_ws_bytes(const AttnArgs& a)
+{
+  const int rows = a.tq * (a.hq / a.hkv), per = 32 * attn_split_waves(rows);
+  return (size_t)a.hkv * ((rows + per - 1) / per) * (per / 32) * a.shares *
+         attn_split_bytes(a.d);
+}
 hipError_t launch_attention(const AttnArgs& a, hipStream_t s);
 // The attention prologue of a two-group pass in one launch: q normed and
 // rotated in place, k normed and rotated into its cache, v copied into its

@@ -2068,8 +2068,8 @@ f16_to_bf16_kernel(const uint2* __restrict__ src, uint2* __restrict__ dst,
 
 // ---- flash attention ------------------------------------------------------
 // Grouped-query attention over a K/V cache, one workgroup per 32 * NWV
-// queries of one head (NWV waves of 32: 8 bidirectional, 4 causal), keys
-// streamed in tiles of 64.
+// queries of one head (NWV waves of 32: attn_waves), keys streamed in tiles
+// of 64.
 //
 // The score tile is computed TRANSPOSED, S^T = K Q^T, with the key
 // fragment as the MFMA's first operand: a lane then holds 32 scores (two
@@ -2129,15 +2129,24 @@ sum_halves(float v)
 
 constexpr float kLazy = 8.0f;
 
-// Waves (32 queries each) per attention workgroup.  Bidirectional: 8, so
-// each K/V tile copied into LDS serves 256 queries (the generation pass
-// 0.295-0.302 ms against 0.309-0.311 with 4).  The causal masks keep 4:
+// Waves (32 queries each) per attention workgroup.  The causal masks run 4:
 // a workgroup runs to the last key its last query sees, and 256-query
 // workgroups waste more masked keys (causal 12% slower with 8).
-template <int MODE>
-constexpr int attn_waves()
+// Bidirectional, a K/V tile in LDS serves 256 queries with 8 waves (one
+// workgroup per CU) and 128 with 4 (two per CU).  A pair of 4-wave
+// workgroups takes ~1.06 times an 8-wave one's time, a 4-wave one alone on
+// its CU ~0.77 times, so the rounds decide (us, 32 heads, d = 128, queries
+// over queries + 128 keys, 8 / 4 waves): 1024 34.5 / 26.0, 1500 46.5 /
+// 50.3, 2048 72.1 / 74.3, 3000 169.8 / 152.1, 4096 256.1 / 262.4.
+inline int
+attn_waves(int mode, int hq, int tq, int cus)
 {
-  return MODE == 0 ? 8 : 4;
+  if (mode != 0) { return 4; }
+  const long long n8 = (long long)hq * ((tq + 255) / 256), n4 = (long long)hq * ((tq + 127) / 128);
+  const long long r4 = n4 % (2 * cus);
+  const double t8 = (double)((n8 + cus - 1) / cus);
+  const double t4 = 1.06 * (double)(n4 / (2 * cus)) + (r4 == 0 ? 0.0 : r4 <= cus ? 0.77 : 1.06);
+  return t4 < t8 ? 4 : 8;
 }
 
 // 64-byte block swizzle of V row r: four consecutive rows at one block
@@ -2149,11 +2158,33 @@ vswz(int r)
   return (r * (D / 32) / 4) % (D / 32);
 }
 
+// One share's partial results of 32 rows (row group rg) in the split
+// attention's scratch: O as [D / 8][64 lanes] float4, then the rows' running
+// max and sum.
+struct SplitRows {
+  f32x4_t* o;
+  float2* ml;
+};
+__device__ __forceinline__ SplitRows
+split_rows(void* ws, int rg, int share, int shares, int d)
+{
+  char* p = static_cast<char*>(ws) +
+            (size_t)(rg * shares + share) * attn_split_bytes(d);
+  return {reinterpret_cast<f32x4_t*>(p), reinterpret_cast<float2*>(p + 32 * d * 4)};
+}
+
 typedef short i16x4_t __attribute__((ext_vector_type(4)));
 typedef short i16x2_t __attribute__((ext_vector_type(2)));
 
-template <int D, int MODE, int NWV>
-__global__ __launch_bounds__(64 * NWV, 8 / NWV) void
+// Keys split over workgroups (SPLIT), for query sets too short to fill the
+// GPU: a workgroup computes 32 * NWV ROWS of one kv head over a share of
+// its key tiles, a row being one of the G = hq / hkv query heads of one
+// token (row r: token r / G, head kvh * G + r % G), so every K/V tile is
+// read once for all of the group's heads.  It leaves its rows' output
+// unnormalised in f32, with the running max and sum, in A.ws (SplitRows);
+// attention_combine_kernel adds the shares.
+template <int D, int MODE, int NWV, bool SPLIT = false>
+__global__ __launch_bounds__(64 * NWV, NWV < 4 ? 1 : 8 / NWV) void
 attention_kernel(const AttnArgs A)
 {
   constexpr int BK = 64;
@@ -2180,24 +2211,33 @@ attention_kernel(const AttnArgs A)
   // Work item: (query head, 128-query tile), ordered kv head first, so
   // that cutting the list into 8 runs (one per XCD, workgroups b, b+8, ...
   // run on XCD b % 8) keeps each kv head's keys in one XCD's L2.
-  const int ntq = (A.tq + QT - 1) / QT;
-  const int items = A.hq * ntq;
+  // (SPLIT: kv head, row block, share of the keys.)
+  const int G = SPLIT ? A.hq / A.hkv : 1;
+  const int nrows = A.tq * G;
+  const int ntq = (nrows + QT - 1) / QT;
+  const int items = SPLIT ? A.hkv * ntq * A.shares : A.hq * ntq;
   const int b = blockIdx.x;
   const int item = (items % 8 == 0) ? (b % 8) * (items / 8) + b / 8 : b;
-  const int h = item / ntq;
+  const int share = SPLIT ? item % A.shares : 0;
+  const int block = SPLIT ? item / A.shares : item;
   // With a mask, later query tiles see more keys: they are dealt first, so
   // the long workgroups start early instead of forming the tail.
-  const int qt = MODE == 0 ? item % ntq : ntq - 1 - item % ntq;
-  const int kvh = h / (A.hq / A.hkv);
+  const int qt = MODE == 0 ? block % ntq : ntq - 1 - block % ntq;
+  const int kvh = SPLIT ? block / ntq : (block / ntq) / (A.hq / A.hkv);
 
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform
   const int lane = tid & 63;
   const int lq = lane & 31;
   const int half = lane >> 5;
-  const int qrow = qt * QT + wave * 32 + lq;      // this lane's query
+  const int row = qt * QT + wave * 32 + lq;
+  const int h = SPLIT ? kvh * G + row % G : block / ntq;
+  const int qrow = SPLIT ? row / G : row;         // this lane's query
   const bool qvalid = qrow < A.tq;
   const int qpos = A.q_offset + qrow;
+  const int tok0 = SPLIT ? qt * QT / G : qt * QT; // the workgroup's queries
+  const int tok1 = SPLIT ? (min(nrows, qt * QT + QT) - 1) / G
+                         : min(A.tq, qt * QT + QT) - 1;
   const float scale = 1.4426950408889634f * rsqrtf((float)D);
   const float lazy = kLazy / scale;               // in raw score units
 
@@ -2221,26 +2261,27 @@ attention_kernel(const AttnArgs A)
   const uint16_t* vbase = A.v + (long long)kvh * A.cap * D;
   // (vectors, not arrays: a lambda capturing a local array of template-
   // dependent size loses the kernel's host-side launch stub)
-  static_assert(CPW <= 4, "copy offsets hold four instructions");
+  // (the swizzles repeat after four instructions, which cover 4 KiB)
   i32x4_t koffs = {}, voffs = {};
 #pragma unroll
-  for (int i = 0; i < CPW; ++i) {
+  for (int i = 0; i < (CPW < 4 ? CPW : 4); ++i) {
     const int idx = (wave * CPW + i) * 64 + lane;     // landing chunk
     const int r = idx / KCH;
     koffs[i] = (r * D + (((idx % KCH) ^ (r % KCH)) << 3)) * 2;
     voffs[i] = (r * D + (((idx % KCH) ^ (4 * vswz<D>(r))) << 3)) * 2;
   }
   int32_t tr = 0;
+  int kstop = A.tk;          // the copies' range: [0, kstop)
   auto copy_k = [&](int j0, uint16_t* dst_tile) {
-    const int left = max(A.tk - j0, 0);
+    const int left = max(kstop - j0, 0);
     const __amdgpu_buffer_rsrc_t rs = make_rsrc(kbase + (long long)j0 * D, left * D * 2);
     char* dst = reinterpret_cast<char*>(dst_tile) + wave * CPW * 1024;
     if (kCopyWaves == NWV || wave < kCopyWaves) {
 #pragma unroll
       for (int i = 0; i < CPW; ++i) {
         __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            rs, (__attribute__((address_space(3))) void*)(dst + i * 1024), 16, koffs[i],
-            0, 0, 0);
+            rs, (__attribute__((address_space(3))) void*)(dst + i * 1024), 16,
+            koffs[i & 3] + (i >> 2) * 4096, 0, 0, 0);
       }
     }
     if constexpr (MODE == 2) {
@@ -2249,15 +2290,15 @@ attention_kernel(const AttnArgs A)
     }
   };
   auto copy_v = [&](int j0, uint16_t* dst_tile) {
-    const int left = max(A.tk - j0, 0);
+    const int left = max(kstop - j0, 0);
     const __amdgpu_buffer_rsrc_t rs = make_rsrc(vbase + (long long)j0 * D, left * D * 2);
     char* dst = reinterpret_cast<char*>(dst_tile) + wave * CPW * 1024;
     if (kCopyWaves == NWV || wave < kCopyWaves) {
 #pragma unroll
       for (int i = 0; i < CPW; ++i) {
         __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            rs, (__attribute__((address_space(3))) void*)(dst + i * 1024), 16, voffs[i],
-            0, 0, 0);
+            rs, (__attribute__((address_space(3))) void*)(dst + i * 1024), 16,
+            voffs[i & 3] + (i >> 2) * 4096, 0, 0, 0);
       }
     }
   };
@@ -2286,12 +2327,12 @@ attention_kernel(const AttnArgs A)
   f32x16_t sc[2];           // scores of the current tile
   float mb = -INFINITY;     // their max over the row (both halves)
 
-  const int q_first = A.q_offset + qt * QT;       // workgroup's first query
+  const int q_first = A.q_offset + tok0;          // workgroup's first query
   // One past the last key any of the workgroup's queries sees; the tiles
   // after it are fully masked and would add exactly 0.
   int kend = A.tk;
   if constexpr (MODE != 0) {
-    const int q_last = A.q_offset + min(A.tq, qt * QT + QT) - 1;
+    const int q_last = A.q_offset + tok1;
     kend = min(A.tk, q_last + 1);
   }
   if constexpr (MODE == 2) {
@@ -2300,7 +2341,7 @@ attention_kernel(const AttnArgs A)
     // [tmin, tmax] (a superset of the visible keys; the mask is exact).
     __shared__ int kred[3][NWV];
     int tmin = INT_MAX, tmax = INT_MIN;
-    if (tid < QT && qt * QT + tid < A.tq) {
+    if (tid < QT && tok0 + tid <= tok1) {
       const int tv = A.t_index[q_first + tid];
       tmin = tv;
       tmax = tv;
@@ -2335,7 +2376,15 @@ attention_kernel(const AttnArgs A)
     for (int w = 1; w < NWV; ++w) { jm = max(jm, kred[2][w]); }
     kend = jm + 1;
   }
-  const int ntiles = (kend + BK - 1) / BK;
+  // this workgroup's key tiles [tbeg, ntiles)
+  int tbeg = 0;
+  int ntiles = (kend + BK - 1) / BK;
+  if constexpr (SPLIT) {
+    const int all = ntiles;
+    tbeg = (int)((long long)share * all / A.shares);
+    ntiles = (int)((long long)(share + 1) * all / A.shares);
+    kstop = min(A.tk, ntiles * BK);
+  }
 
   // -inf for the scores of tile j0 that the mode hides; a no-op for a tile
   // whose keys are all below tk and (causal masks) the first query
@@ -2461,7 +2510,7 @@ attention_kernel(const AttnArgs A)
       __builtin_amdgcn_sched_group_barrier(0x002, 6 * EPB / 4, 0);    // VALU
     }
     // ---- C --------------------------------------------------------------
-    mask(sn, j0 + BK, (t + 1) % 3);
+    mask(sn, j0 + BK, (t - tbeg + 1) % 3);
     float mx = -INFINITY;
 #pragma unroll
     for (int k4 = 2; k4 < 4; ++k4) {
@@ -2482,20 +2531,20 @@ attention_kernel(const AttnArgs A)
     }
     mb = max_halves(mx);
     l += ps;
-    store_t((t + 2) % 3);
+    store_t((t - tbeg + 2) % 3);
     __syncthreads();
     sc[0] = sn[0];
     sc[1] = sn[1];
   };
 
-  if (ntiles > 0) {
+  if (tbeg < ntiles) {
     // K and t of tiles 0 and 1, V of tile 0; the scores of tile 0, read
     // by every wave before the first iteration refills ks0
-    copy_k(0, ks0);
+    copy_k(tbeg * BK, ks0);
     store_t(0);
-    copy_k(BK, ks1);
+    copy_k(tbeg * BK + BK, ks1);
     store_t(1);
-    copy_v(0, vs0);
+    copy_v(tbeg * BK, vs0);
     __syncthreads();
     sc[0] = f32x16_t{};
     sc[1] = f32x16_t{};
@@ -2506,19 +2555,32 @@ attention_kernel(const AttnArgs A)
       sc[1] = MmaBf16::run(*reinterpret_cast<const i32x4_t*>(ks0 + 32 * D + off),
                            qf[ds], sc[1]);
     }
-    mask(sc, 0, 0);
+    mask(sc, tbeg * BK, 0);
     float mx = sc[0][0];
 #pragma unroll
     for (int r = 1; r < 32; ++r) { mx = fmaxf(mx, sc[r >> 4][r & 15]); }
     mb = max_halves(mx);
     __syncthreads();
   }
-  for (int t = 0; t < ntiles; t += 2) {
+  for (int t = tbeg; t < ntiles; t += 2) {
     iteration(t, ks1, ks0, vs0, vs1);
     if (t + 1 < ntiles) { iteration(t + 1, ks0, ks1, vs1, vs0); }
   }
 
   l = sum_halves(l);
+  if constexpr (SPLIT) {
+    // lane-major: every store writes 1 KiB of consecutive bytes
+    const SplitRows ws = split_rows(A.ws, (kvh * ntq + qt) * NWV + wave, share, A.shares, D);
+    if (half == 0) { ws.ml[lq] = make_float2(m, l); }
+    if (!qvalid || l == 0.0f) { return; }
+#pragma unroll
+    for (int i = 0; i < D / 8; ++i) {
+      const int g = 4 * (i & 3);
+      ws.o[i * 64 + lane] = f32x4_t{o[i >> 2][g], o[i >> 2][g + 1], o[i >> 2][g + 2],
+                                    o[i >> 2][g + 3]};
+    }
+    return;
+  }
   if (!qvalid) { return; }
   const float inv = l > 0.0f ? 1.0f / l : 0.0f;
   uint16_t* op = A.out + (long long)h * A.o_head + (long long)qrow * A.o_tok;
@@ -2534,6 +2596,87 @@ attention_kernel(const AttnArgs A)
       *reinterpret_cast<u32x2_t*>(op + c) = w;
     }
   }
+}
+
+// Adds the key shares of attention_kernel<.., SPLIT>: W waves sum 8 columns
+// (chunk i of D / 8) of the 32 rows of one row group, lane (half, lq)
+// holding columns 8 i + 4 half .. + 3 of row lq as the kernel's accumulators
+// do.  out = sum_s w_s O_s / sum_s w_s l_s, w_s = exp2((m_s - max m) *
+// scale).  A share that saw no key of a row (l = 0) left no output for it.
+// The partials come from the other XCDs' writes, a round trip past L2 each,
+// so the shares are dealt over the W waves (up to kCombineAhead each), whose
+// loads all go out before the first is used; the waves' sums meet in LDS.
+constexpr int kCombineAhead = 8;
+
+template <int D, int W>
+__global__ __launch_bounds__(256) void
+attention_combine_kernel(const AttnArgs A, int groups_per_head)
+{
+  constexpr int NC = D / 8;
+  constexpr int kUnits = 4 / W;             // (row group, chunk) per workgroup
+  __shared__ f32x4_t so[4][64];
+  __shared__ float2 sml[4][64];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lq = lane & 31;
+  const int half = lane >> 5;
+  const int unit = blockIdx.x * kUnits + wave / W;
+  const int part = wave % W;
+  const int rg = unit / NC;                 // D / 8 is a multiple of kUnits
+  const int i = unit % NC;
+  const int G = A.hq / A.hkv;
+  const int kvh = rg / groups_per_head;
+  const int row = (rg % groups_per_head) * 32 + lq;
+  const int tok = row / G;
+  const bool valid = tok < A.tq;
+  const float scale = 1.4426950408889634f * rsqrtf((float)D);
+  // adds (m1, l1, o1) to (m, l, o); a share without keys has l = 0
+  auto add = [&](float& m, float& l, f32x4_t& o, float m1, float l1, f32x4_t o1) {
+    if (l1 == 0.0f) { return; }
+    const float mx = l == 0.0f ? m1 : fmaxf(m, m1);
+    const float w0 = l == 0.0f ? 0.0f : __builtin_amdgcn_exp2f((m - mx) * scale);
+    const float w1 = __builtin_amdgcn_exp2f((m1 - mx) * scale);
+    l = l * w0 + l1 * w1;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) { o[e] = o[e] * w0 + o1[e] * w1; }
+    m = mx;
+  };
+  float m = -INFINITY, l = 0.0f;
+  f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
+  for (int s0 = part; s0 < A.shares; s0 += kCombineAhead * W) {
+    float2 ml[kCombineAhead];
+    f32x4_t o[kCombineAhead];
+#pragma unroll
+    for (int j = 0; j < kCombineAhead; ++j) {
+      const int s = s0 + j * W;
+      ml[j] = make_float2(0.0f, 0.0f);
+      o[j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+      if (s < A.shares && valid) {
+        const SplitRows ws = split_rows(A.ws, rg, s, A.shares, D);
+        ml[j] = ws.ml[lq];
+        o[j] = ws.o[i * 64 + lane];
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < kCombineAhead; ++j) { add(m, l, acc, ml[j].x, ml[j].y, o[j]); }
+  }
+  if constexpr (W > 1) {
+    so[wave][lane] = acc;
+    sml[wave][lane] = make_float2(m, l);
+    __syncthreads();
+    if (part != 0) { return; }
+#pragma unroll
+    for (int w = 1; w < W; ++w) {
+      add(m, l, acc, sml[wave + w][lane].x, sml[wave + w][lane].y, so[wave + w][lane]);
+    }
+  }
+  if (!valid) { return; }
+  const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+  uint16_t* op = A.out + (long long)(kvh * G + row % G) * A.o_head +
+                 (long long)tok * A.o_tok + 8 * i + 4 * half;
+  *reinterpret_cast<u32x2_t*>(op) = u32x2_t{
+      bf16_bits(acc[0] * inv) | (bf16_bits(acc[1] * inv) << 16),
+      bf16_bits(acc[2] * inv) | (bf16_bits(acc[3] * inv) << 16)};
 }
 
 // Row re-layout of [T][H][D] data between two strided views: element
@@ -3655,14 +3798,47 @@ launch_f16_to_bf16(const uint16_t* src, int64_t n, uint16_t* dst, hipStream_t s)
   return hipGetLastError();
 }
 
+template <int D, int MODE, int NWV>
+static hipError_t
+launch_attention_split(const AttnArgs& a, hipStream_t s)
+{
+  const int rows = a.tq * (a.hq / a.hkv);
+  const int blocks = (rows + 32 * NWV - 1) / (32 * NWV);
+  hipLaunchKernelGGL((attention_kernel<D, MODE, NWV, true>), dim3(a.hkv * blocks * a.shares),
+                     dim3(64 * NWV), 0, s, a);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) { return e; }
+  const int groups = a.hkv * blocks * NWV;
+  const int units = groups * (D / 8);
+  if (a.shares <= kCombineAhead) {
+    hipLaunchKernelGGL((attention_combine_kernel<D, 1>), dim3(units / 4), dim3(256), 0, s, a,
+                       blocks * NWV);
+  } else {
+    hipLaunchKernelGGL((attention_combine_kernel<D, 4>), dim3(units), dim3(256), 0, s, a,
+                       blocks * NWV);
+  }
+  return hipGetLastError();
+}
+
 template <int D, int MODE>
 hipError_t
 launch_attention_d(const AttnArgs& a, hipStream_t s)
 {
-  constexpr int NWV = attn_waves<MODE>();
-  const int ntq = (a.tq + 32 * NWV - 1) / (32 * NWV);
-  hipLaunchKernelGGL((attention_kernel<D, MODE, NWV>), dim3(a.hq * ntq), dim3(64 * NWV),
-                     0, s, a);
+  if (a.shares > 1) {
+    const int rows = a.tq * (a.hq / a.hkv);
+    if (attn_split_waves(rows) == 1) { return launch_attention_split<D, MODE, 1>(a, s); }
+    if (attn_split_waves(rows) == 2) { return launch_attention_split<D, MODE, 2>(a, s); }
+    return launch_attention_split<D, MODE, 4>(a, s);
+  }
+  if constexpr (MODE == 0) {
+    if (attn_waves(MODE, a.hq, a.tq, a.cus) == 8) {
+      hipLaunchKernelGGL((attention_kernel<D, MODE, 8>), dim3(a.hq * ((a.tq + 255) / 256)),
+                         dim3(512), 0, s, a);
+      return hipGetLastError();
+    }
+  }
+  hipLaunchKernelGGL((attention_kernel<D, MODE, 4>), dim3(a.hq * ((a.tq + 127) / 128)),
+                     dim3(256), 0, s, a);
   return hipGetLastError();
 }
 
@@ -3780,15 +3956,51 @@ kernels_loadable()
 {
   const void* fns[] = {
       reinterpret_cast<const void*>(&f16_to_bf16_kernel),
-      reinterpret_cast<const void*>(&attention_kernel<128, 0, attn_waves<0>()>),
-      reinterpret_cast<const void*>(&attention_kernel<128, 1, attn_waves<1>()>),
-      reinterpret_cast<const void*>(&attention_kernel<128, 2, attn_waves<2>()>),
-      reinterpret_cast<const void*>(&attention_kernel<64, 0, attn_waves<0>()>),
-      reinterpret_cast<const void*>(&attention_kernel<64, 1, attn_waves<1>()>),
-      reinterpret_cast<const void*>(&attention_kernel<64, 2, attn_waves<2>()>),
-      reinterpret_cast<const void*>(&attention_kernel<32, 0, attn_waves<0>()>),
-      reinterpret_cast<const void*>(&attention_kernel<32, 1, attn_waves<1>()>),
-      reinterpret_cast<const void*>(&attention_kernel<32, 2, attn_waves<2>()>),
+      reinterpret_cast<const void*>(&attention_kernel<128, 0, 8>),
+      reinterpret_cast<const void*>(&attention_kernel<128, 0, 4>),
+      reinterpret_cast<const void*>(&attention_kernel<128, 1, 4>),
+      reinterpret_cast<const void*>(&attention_kernel<128, 2, 4>),
+      reinterpret_cast<const void*>(&attention_kernel<64, 0, 8>),
+      reinterpret_cast<const void*>(&attention_kernel<64, 0, 4>),
+      reinterpret_cast<const void*>(&attention_kernel<64, 1, 4>),
+      reinterpret_cast<const void*>(&attention_kernel<64, 2, 4>),
+      reinterpret_cast<const void*>(&attention_kernel<32, 0, 8>),
+      reinterpret_cast<const void*>(&attention_kernel<32, 0, 4>),
+      reinterpret_cast<const void*>(&attention_kernel<32, 1, 4>),
+      reinterpret_cast<const void*>(&attention_kernel<32, 2, 4>),
+      reinterpret_cast<const void*>(&attention_combine_kernel<128, 1>),
+      reinterpret_cast<const void*>(&attention_combine_kernel<128, 4>),
+      reinterpret_cast<const void*>(&attention_kernel<128, 0, 1, true>),
+      reinterpret_cast<const void*>(&attention_kernel<128, 0, 2, true>),
+      reinterpret_cast<const void*>(&attention_kernel<128, 0, 4, true>),
+      reinterpret_cast<const void*>(&attention_kernel<128, 1, 1, true>),
+      reinterpret_cast<const void*>(&attention_kernel<128, 1, 2, true>),
+      reinterpret_cast<const void*>(&attention_kernel<128, 1, 4, true>),
+      reinterpret_cast<const void*>(&attention_kernel<128, 2, 1, true>),
+      reinterpret_cast<const void*>(&attention_kernel<128, 2, 2, true>),
+      reinterpret_cast<const void*>(&attention_kernel<128, 2, 4, true>),
+      reinterpret_cast<const void*>(&attention_combine_kernel<64, 1>),
+      reinterpret_cast<const void*>(&attention_combine_kernel<64, 4>),
+      reinterpret_cast<const void*>(&attention_kernel<64, 0, 1, true>),
+      reinterpret_cast<const void*>(&attention_kernel<64, 0, 2, true>),
+      reinterpret_cast<const void*>(&attention_kernel<64, 0, 4, true>),
+      reinterpret_cast<const void*>(&attention_kernel<64, 1, 1, true>),
+      reinterpret_cast<const void*>(&attention_kernel<64, 1, 2, true>),
+      reinterpret_cast<const void*>(&attention_kernel<64, 1, 4, true>),
+      reinterpret_cast<const void*>(&attention_kernel<64, 2, 1, true>),
+      reinterpret_cast<const void*>(&attention_kernel<64, 2, 2, true>),
+      reinterpret_cast<const void*>(&attention_kernel<64, 2, 4, true>),
+      reinterpret_cast<const void*>(&attention_combine_kernel<32, 1>),
+      reinterpret_cast<const void*>(&attention_combine_kernel<32, 4>),
+      reinterpret_cast<const void*>(&attention_kernel<32, 0, 1, true>),
+      reinterpret_cast<const void*>(&attention_kernel<32, 0, 2, true>),
+      reinterpret_cast<const void*>(&attention_kernel<32, 0, 4, true>),
+      reinterpret_cast<const void*>(&attention_kernel<32, 1, 1, true>),
+      reinterpret_cast<const void*>(&attention_kernel<32, 1, 2, true>),
+      reinterpret_cast<const void*>(&attention_kernel<32, 1, 4, true>),
+      reinterpret_cast<const void*>(&attention_kernel<32, 2, 1, true>),
+      reinterpret_cast<const void*>(&attention_kernel<32, 2, 2, true>),
+      reinterpret_cast<const void*>(&attention_kernel<32, 2, 4, true>),
       reinterpret_cast<const void*>(&transpose_rows_kernel),
       reinterpret_cast<const void*>(&split_norm_rope_kernel<true, true>),
       reinterpret_cast<const void*>(&split_norm_rope_kernel<true, false>),
