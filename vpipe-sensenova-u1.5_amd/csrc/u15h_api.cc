@@ -234,38 +234,67 @@ plan_split(u15h_ctx* ctx, GemmBatch& b, bool noalloc = false)
              : fail(ctx, U15H_EINVAL, "split workspace overflow");
 }
 
-// The skinny route: a bf16 batch whose problems all have at most 128 rows
-// (und prefill, small decode-like steps) and plain [N][K] weights.  There
-// the weights are the traffic; the tiled GEMM would run its 256-row tiles
-// mostly empty.
+// The skinny route: a batch whose problems all have at most 128 rows (und
+// prefill, small decode-like steps) and plain [N][K] weights (SwiGLU: rows
+// any whole pitch apart).  There the weights are the traffic; the tiled GEMM
+// would run its 256-row tiles mostly empty.
 bool
-skinny_fits(const u15h_ctx* ctx, const GemmBatch& b)
+skinny_fits(const u15h_ctx* ctx, const GemmBatch& b, Epi epi)
 {
   if (!ctx->skinny_on || b.nprob <= 0 || b.kbytes % 128 != 0) { return false; }
   for (int i = 0; i < b.nprob; ++i) {
     const GemmProblem& p = b.p[i];
-    if (p.rows > u15h::kSkinnyMaxRows || p.wld != b.kbytes || p.n % 4 != 0) {
+    if (p.rows > u15h::kSkinnyMaxRows || (p.wld != b.kbytes && epi != Epi::kSwiglu) ||
+        p.n % 4 != 0) {
       return false;
     }
   }
   return true;
 }
 
-// Launches a batch that skinny_fits on the skinny kernels.  K shares S
-// (a power of two) are added while the workgroups stay within what the
-// CUs hold at once, each share keeps enough K-blocks to fill its waves'
-// prefetch, and the fp32 partial sums (written and read once) stay at most
-// half the weight bytes: S * rows * 8 <= K.
-// The partials go to the split-K workspace (or, with `noalloc`, the static
-// scratch); a batch whose partials would not fit takes fewer shares.
+// At most 16 rows: waves per workgroup and K shares of `cb` workgroups of 16
+// columns over nkb K-blocks of 128 bytes.  A share's partial sums cost a
+// second launch (~2.5 us), so shares come only where the columns leave most
+// CUs idle over a long K; eight waves where four would keep too few loads in
+// flight.  Measured in a graph (us, bf16 1 / 16 rows; W x S waves and shares;
+// the earlier rule took 4 waves and shares of at least 32 K-blocks):
+//   N = 1024, K = 4096   4x1 6.0 / 7.5  8x1 5.2 / 7.8  4x2 6.8 / 8.0
+//   N = 4096, K = 4096   4x1 10.5 / 10.4  8x1 9.2 / 10.5  4x2 12.0 / 12.6
+//   N = 4096, K = 12288  4x1 23.9 / 24.0  8x1 21.2 / 24.3  4x2 23.5 / 26.1
+//   N = 1024, K = 8192   8x1 7.2 / 12.1  4x2 8.1 / 10.2  4x4 8.7 / 9.4
+//   N = 1024, K = 12288  8x1 13.0 / 20.0  4x2 13.7 / 14.9  4x4 10.9 / 11.7
+//   N = 1024, K = 1024   4x1 2.9 / 3.6  8x1 3.1 / 3.8
+// 16 waves were slower than 8 at every shape.
+void
+narrow_plan(const u15h_ctx* ctx, int rows, int nkb, int cb, int* waves, int* shares)
+{
+  int S = 1;
+  while (nkb > 64 && S < 4 && nkb / S > (rows > 8 ? 48 : 64) && 2 * S * cb <= ctx->num_cu) {
+    S *= 2;
+  }
+  const bool few = 3 * cb < 4 * ctx->num_cu;
+  const bool eight = S == 1 && few && nkb >= 64 && (rows <= 4 || 8 * cb >= 5 * ctx->num_cu);
+  *waves = eight ? 8 : 4;
+  *shares = S;
+}
+
+// Launches a batch that skinny_fits on the skinny kernels.
+// At most 16 rows: narrow_plan's workgroups.
+// Above: K shares S (a power of two) are added while the
+// workgroups stay within what the CUs hold at once, each share keeps enough
+// K-blocks to fill its waves' prefetch, and the 4-byte partial sums (written
+// and read once) stay at most half the weight bytes: S * rows * 16 <= K
+// bytes.  The partials go to the split-K workspace (or, with `noalloc`, the
+// static scratch); a batch whose partials would not fit takes fewer shares.
 u15h_status
-skinny_launch(u15h_ctx* ctx, const GemmBatch& b, hipStream_t s, bool noalloc,
+skinny_launch(u15h_ctx* ctx, const GemmBatch& b, Epi epi, hipStream_t s, bool noalloc,
               const u15h::GemmEvents& ev, const u15h_qweight* q = nullptr)
 {
   u15h::SkinnyBatch k;
   std::memset(&k, 0, sizeof k);
   k.kbytes = b.kbytes;
   k.nprob = b.nprob;
+  k.swiglu = epi == Epi::kSwiglu;
   if (q != nullptr) {         // one problem whose w is the pack's codes
     k.qbits = q->bits;
     k.qgroup = q->group;
@@ -273,35 +302,37 @@ skinny_launch(u15h_ctx* ctx, const GemmBatch& b, hipStream_t s, bool noalloc,
     k.p[0].qb = static_cast<const uint16_t*>(q->biases);
   }
   for (int i = 0; i < b.nprob; ++i) { k.max_rows = std::max(k.max_rows, b.p[i].rows); }
-  const int K = b.kbytes / 2;
   const int nkb = b.kbytes / 128;
   // Resident workgroups per CU: two for the 16-column-wave builds (at most
   // 80 KiB of LDS each), one for the 32-column-wave builds (112-128 KiB).
-  // A share keeps 32 K-blocks (8 per wave) in the register kernel, 16 in
-  // the LDS kernels.
+  // A share keeps 16 K-blocks.
   auto blocks = [&](int cols) {
     int cb = 0;
     for (int i = 0; i < b.nprob; ++i) { cb += (b.p[i].n + cols - 1) / cols; }
     return cb;
   };
-  auto shares = [&](int cols, int cb, int per_cu) {
-    const int min_kb = cols == 16 ? 32 : 16;
+  auto shares = [&](int cb, int per_cu) {
     int S = 1;
     while (S < 16 && 2 * S * cb <= per_cu * ctx->num_cu &&
-           nkb / (2 * S) >= min_kb && 2 * S * k.max_rows * 8 <= K) {
+           nkb / (2 * S) >= 16 && 2 * S * k.max_rows * 16 <= b.kbytes) {
       S *= 2;
     }
     return S;
   };
   k.cols = u15h::skinny_cols(k.max_rows, k.qbits);
-  int S = shares(k.cols, blocks(k.cols), 2);
-  // Above 64 rows, bf16 weights: waves of 32 columns (each activation
-  // fragment read from LDS serves two weight fragments), with no more K
-  // shares than 16-column waves take, where that keeps at least 3/4 of the
-  // CUs busy (one such workgroup per CU)
-  if (u15h::skinny_wide_ok(k.max_rows, k.qbits)) {
+  int S = 1;
+  if (k.max_rows <= 16) {
+    narrow_plan(ctx, k.max_rows, nkb, blocks(k.cols), &k.waves, &S);
+  } else {
+    S = shares(blocks(k.cols), k.swiglu && k.max_rows > 64 ? 1 : 2);
+  }
+  // Above 64 rows, bf16 or int8 weights: waves of 32 columns (each
+  // activation fragment read from LDS serves two weight fragments; SwiGLU's
+  // waves always do), with no more K shares than 16-column waves take, where
+  // that keeps at least 3/4 of the CUs busy (one such workgroup per CU)
+  if (!k.swiglu && u15h::skinny_wide_ok(k.max_rows, k.qbits)) {
     const int cb2 = blocks(2 * k.cols);
-    const int S2 = std::min(shares(2 * k.cols, cb2, 1), S);
+    const int S2 = std::min(shares(cb2, 1), S);
     if (4 * S2 * cb2 >= 3 * ctx->num_cu) {
       k.cols *= 2;
       S = S2;
@@ -309,15 +340,19 @@ skinny_launch(u15h_ctx* ctx, const GemmBatch& b, hipStream_t s, bool noalloc,
   }
   for (int i = 0; i < b.nprob; ++i) {
     const GemmProblem& p = b.p[i];
-    u15h::SkinnyProblem& q = k.p[i];
-    q.a = p.a;
-    q.w = p.w;
-    q.y = p.y;
-    q.bias = p.bias;
-    q.rows = p.rows;
-    q.n = p.n;
-    q.ldy = p.ldy;
-    q.cb_begin = k.total_cb;
+    u15h::SkinnyProblem& d = k.p[i];
+    d.a = p.a;
+    d.w = p.w;
+    d.w2 = p.w2;
+    d.sa = p.sa;
+    d.sw = p.sw;
+    d.y = p.y;
+    d.bias = p.bias;
+    d.rows = p.rows;
+    d.n = p.n;
+    d.ldy = p.ldy;
+    d.wld = p.wld;
+    d.cb_begin = k.total_cb;
     k.total_cb += (p.n + k.cols - 1) / k.cols;
   }
   // One cap for both destinations, so u15h_mot_linear and
@@ -348,8 +383,11 @@ skinny_launch(u15h_ctx* ctx, const GemmBatch& b, hipStream_t s, bool noalloc,
     size_t off = 0;
     for (int i = 0; i < k.nprob; ++i) {
       k.p[i].ws_off = off;
-      off += (size_t)S * k.p[i].rows * k.p[i].n;
+      off += (size_t)S * k.p[i].rows * k.p[i].n * (k.swiglu ? 2 : 1);
     }
+  }
+  if (epi == Epi::kI32 || epi == Epi::kDequantBf16) {
+    return launched(ctx, u15h::launch_skinny_i8(k, epi, s, ev), "skinny_gemm_i8");
   }
   return launched(ctx, u15h::launch_skinny_bf16(k, s, ev), "skinny_gemm_bf16");
 }
@@ -457,6 +495,9 @@ linear_i8_route(u15h_ctx* ctx, hipStream_t s, const u15h_bf16* x,
   GemmBatch b = empty_batch(K);
   add_problem(b, xqp, wqp, nullptr, y, bias, sx, sw, M, N, N,
               u15h::tile_cols(Epi::kDequantBf16));
+  if (skinny_fits(ctx, b, Epi::kDequantBf16)) {
+    return skinny_launch(ctx, b, Epi::kDequantBf16, s, false, take_profile_event(ctx));
+  }
   u15h_status st = plan_split(ctx, b);
   if (st != U15H_OK) { return st; }
   return launched(ctx, u15h::launch_gemm_i8(b, Epi::kDequantBf16, ctx->gemm, s, take_profile_event(ctx)),
@@ -588,8 +629,8 @@ dense_bf16(u15h_ctx* ctx, hipStream_t s, const u15h_bf16* x,
   GemmBatch b = empty_batch(K * 2);
   add_problem(b, x, w, nullptr, y, bias, nullptr, nullptr, M, N, N,
               u15h::tile_cols(Epi::kBf16));
-  if (skinny_fits(ctx, b)) {
-    return skinny_launch(ctx, b, s, false, take_profile_event(ctx));
+  if (skinny_fits(ctx, b, Epi::kBf16)) {
+    return skinny_launch(ctx, b, Epi::kBf16, s, false, take_profile_event(ctx));
   }
   u15h_status st = plan_split(ctx, b);
   if (st != U15H_OK) { return st; }
@@ -676,8 +717,9 @@ mot_linear_impl(u15h_ctx* ctx, u15h_stream stream, const u15h_bf16* x,
                 M_und, p.N, p.N, tc);
   }
   if ((st = check_tiles(ctx, b)) != U15H_OK) { return st; }
-  if (skinny_fits(ctx, b)) {
-    return skinny_launch(ctx, b, as_stream(stream), noalloc, take_profile_event(ctx));
+  if (skinny_fits(ctx, b, Epi::kBf16)) {
+    return skinny_launch(ctx, b, Epi::kBf16, as_stream(stream), noalloc,
+                         take_profile_event(ctx));
   }
   if ((st = plan_split(ctx, b, noalloc)) != U15H_OK) { return st; }
   return launched(ctx, u15h::launch_gemm_bf16(b, Epi::kBf16, ctx->gemm, as_stream(stream), take_profile_event(ctx)),
@@ -871,6 +913,10 @@ u15h_mot_gate_up_swiglu(u15h_ctx* ctx, u15h_stream stream,
   add_problem(b, x, wg_und, wu_und, h, nullptr, nullptr, nullptr, M_und, I, I,
               tc);
   if ((st = check_tiles(ctx, b)) != U15H_OK) { return st; }
+  if (skinny_fits(ctx, b, Epi::kSwiglu)) {
+    return skinny_launch(ctx, b, Epi::kSwiglu, as_stream(stream), false,
+                         take_profile_event(ctx));
+  }
   if ((st = plan_split(ctx, b)) != U15H_OK) { return st; }
   return launched(ctx, u15h::launch_gemm_bf16(b, Epi::kSwiglu, ctx->gemm, as_stream(stream), take_profile_event(ctx)),
                   "mot_gate_up_swiglu");
@@ -1013,6 +1059,9 @@ mot_gemm_i8_common(u15h_ctx* ctx, u15h_stream stream, const int8_t* xq,
                 deq ? p.sw_und : nullptr, M_und, p.N, p.N, tc);
   }
   if ((st = check_tiles(ctx, b)) != U15H_OK) { return st; }
+  if (skinny_fits(ctx, b, epi)) {
+    return skinny_launch(ctx, b, epi, as_stream(stream), false, take_profile_event(ctx));
+  }
   if ((st = plan_split(ctx, b)) != U15H_OK) { return st; }
   return launched(ctx, u15h::launch_gemm_i8(b, epi, ctx->gemm, as_stream(stream), take_profile_event(ctx)),
                   deq ? "mot_gemm_i8" : "mot_gemm_i8_i32");
@@ -1126,8 +1175,9 @@ u15h_linear_q(u15h_ctx* ctx, u15h_stream stream, const u15h_bf16* x,
     GemmBatch b = empty_batch(K * 2);
     add_problem(b, x, w->codes, nullptr, y, bias, nullptr, nullptr, M, N, N,
                 u15h::tile_cols(Epi::kBf16));
-    if (skinny_fits(ctx, b)) {
-      return skinny_launch(ctx, b, as_stream(stream), false, take_profile_event(ctx), w);
+    if (skinny_fits(ctx, b, Epi::kBf16)) {
+      return skinny_launch(ctx, b, Epi::kBf16, as_stream(stream), false,
+                           take_profile_event(ctx), w);
     }
   }
   if ((st = ensure_deq_scratch(ctx, stream, (size_t)N * K * 2)) != U15H_OK) {
@@ -1173,6 +1223,10 @@ u15h_swiglu_fused(u15h_ctx* ctx, u15h_stream stream, const u15h_bf16* x,
               nullptr, nullptr, nullptr, M, inter, inter,
               u15h::tile_cols(Epi::kSwiglu), (int)(2 * kb));
   if ((st = check_tiles(ctx, b)) != U15H_OK) { return st; }
+  if (skinny_fits(ctx, b, Epi::kSwiglu)) {
+    return skinny_launch(ctx, b, Epi::kSwiglu, as_stream(stream), false,
+                         take_profile_event(ctx));
+  }
   if ((st = plan_split(ctx, b)) != U15H_OK) { return st; }
   return launched(ctx,
                   u15h::launch_gemm_bf16(b, Epi::kSwiglu, ctx->gemm,

@@ -108,22 +108,28 @@ constexpr int kSkinnyMaxRows = 128;
 constexpr int skinny_cols(int max_rows, int) { return max_rows <= 16 ? 16 : 64; }
 constexpr bool skinny_wide_ok(int max_rows, int qbits) { return qbits == 0 && max_rows > 64; }
 struct SkinnyProblem {
-  const void*     a;      // activation rows [rows][K] (bf16)
-  const void*     w;      // weight rows [n][K] (bf16), or the pack's codes
+  const void*     a;      // activation rows [rows][K] (bf16, or int8 codes)
+  const void*     w;      // weight rows [n][K] (bf16 or int8), or the pack's codes
+  const void*     w2;     // SwiGLU: the up rows (w the gate rows)
+  const float*    sa;     // int8 dequant: row scales [rows]
+  const float*    sw;     // int8 dequant: column scales [n]
   const uint16_t* qs;     // affine pack: scales bf16 [n][K / group]
   const uint16_t* qb;     // affine pack: biases bf16 [n][K / group]
-  void*           y;      // output rows [rows][ldy] (bf16)
+  void*           y;      // output rows [rows][ldy] (bf16, or int32)
   const uint16_t* bias;   // bf16 [n] or null
   int rows;
   int n;
   int ldy;
+  int wld;                // bytes between weight rows (not read for packs)
   int cb_begin;           // first column block of this problem
   size_t ws_off;          // floats from ws to this problem's partial sums
 };
 struct SkinnyBatch {
   SkinnyProblem p[kMaxProb];
   int nprob;
-  int kbytes;             // bytes per row of K (K * 2; a multiple of 128)
+  int kbytes;             // bytes per row of K (K * element; a multiple of 128)
+  bool swiglu;            // y = silu(a . w^T) * (a . w2^T)
+  int waves;              // waves per workgroup at <= 16 rows (4 or 8)
   int split;              // K shares per column block (S)
   int cols;               // output columns per block (skinny_cols)
   int total_cb;           // column blocks over all problems
@@ -138,7 +144,7 @@ inline size_t skinny_ws_floats(const SkinnyBatch& b)
   if (b.split <= 1) { return 0; }
   size_t f = 0;
   for (int i = 0; i < b.nprob; ++i) {
-    f += (size_t)b.split * b.p[i].rows * b.p[i].n;
+    f += (size_t)b.split * b.p[i].rows * b.p[i].n * (b.swiglu ? 2 : 1);
   }
   return f;
 }
@@ -146,6 +152,9 @@ inline size_t skinny_ws_floats(const SkinnyBatch& b)
 // pack dequantised in registers to the expansion's bf16 weights.
 hipError_t launch_skinny_bf16(const SkinnyBatch& b, hipStream_t s,
                               const GemmEvents& ev);
+// The same over int8 codes (kI32 or kDequantBf16).
+hipError_t launch_skinny_i8(const SkinnyBatch& b, Epi epi, hipStream_t s,
+                            const GemmEvents& ev);
 hipError_t launch_gemm_i8(const GemmBatch& b, Epi epi, const GemmShape& g,
                           hipStream_t s, const GemmEvents& ev);
 hipError_t launch_quant_rows_i8(const uint16_t* x, int rows, int K,

@@ -2861,6 +2861,20 @@ sk_mfma(f32x4_t& acc, i32x4_t a, i32x4_t b)
   }
 }
 
+// What the skinny kernels multiply and write: bf16 operands to bf16, or int8
+// codes (the same bytes per K-block, twice the elements) to bf16 by the
+// fused dequant or to raw int32 accumulators.
+constexpr int kElBf16 = 0, kElI8 = 1, kElI32 = 2;
+template <int EL>
+using sk_acc_t = std::conditional_t<EL == kElBf16, f32x4_t, i32x4_t>;
+
+// v_mfma_i32_16x16x64_i8, its accumulator tied as above.
+__device__ __forceinline__ void
+sk_mfma_i8(i32x4_t& acc, i32x4_t a, i32x4_t b)
+{
+  asm volatile("v_mfma_i32_16x16x64_i8 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
+}
+
 // Bias, rounding and store of 4 output columns n..n+3 of row m.
 __device__ __forceinline__ void
 skinny_store(const SkinnyProblem& P, int m, int n, f32x4_t v, uint2 bb)
@@ -2871,6 +2885,58 @@ skinny_store(const SkinnyProblem& P, int m, int n, f32x4_t v, uint2 bb)
   const float v3 = v[3] + bf16_to_f32(bb.y >> 16);
   *reinterpret_cast<uint2*>(static_cast<uint16_t*>(P.y) + (size_t)m * P.ldy + n) =
       make_uint2(pack_bf16x2(v0, v1), pack_bf16x2(v2, v3));
+}
+
+// The epilogue's operands of 4 output columns n..n+3, loaded ahead of the
+// sums they finish.
+template <int EL>
+struct SkEpi {
+  uint2 bias = make_uint2(0u, 0u);
+  float4 sw;
+};
+template <int EL, bool SW>
+__device__ __forceinline__ SkEpi<EL>
+skinny_epi(const SkinnyProblem& P, int n)
+{
+  SkEpi<EL> e;
+  if constexpr (EL == kElI8) { e.sw = *reinterpret_cast<const float4*>(P.sw + n); }
+  if constexpr (!SW && EL != kElI32) {
+    if (P.bias != nullptr) { e.bias = *reinterpret_cast<const uint2*>(P.bias + n); }
+  }
+  return e;
+}
+
+// The complete sums of 4 output columns n..n+3 of row m (with SW, v[0] the
+// gate columns and v[1] the up columns), finished by the element type's
+// epilogue and stored: the same arithmetic as the tiled GEMM's epilogues.
+template <int EL, bool SW, int CW>
+__device__ __forceinline__ void
+skinny_emit(const SkinnyProblem& P, int m, int n, const sk_acc_t<EL> (&v)[CW],
+            const SkEpi<EL>& e)
+{
+  static_assert(CW == (SW ? 2 : 1), "one accumulator per output, two for SwiGLU");
+  const size_t at = (size_t)m * P.ldy + n;
+  if constexpr (SW) {
+    *reinterpret_cast<uint2*>(static_cast<uint16_t*>(P.y) + at) = make_uint2(
+        swiglu1(v[0][0], v[1][0]) | (swiglu1(v[0][1], v[1][1]) << 16),
+        swiglu1(v[0][2], v[1][2]) | (swiglu1(v[0][3], v[1][3]) << 16));
+  } else if constexpr (EL == kElI32) {
+    *reinterpret_cast<i32x4_t*>(static_cast<int32_t*>(P.y) + at) = v[0];
+  } else if constexpr (EL == kElI8) {
+    const float sam = P.sa[m];
+    float f[4] = {((float)v[0][0] * sam) * e.sw.x, ((float)v[0][1] * sam) * e.sw.y,
+                  ((float)v[0][2] * sam) * e.sw.z, ((float)v[0][3] * sam) * e.sw.w};
+    if (P.bias != nullptr) {
+      f[0] += bf16_to_f32(e.bias.x & 0xffffu);
+      f[1] += bf16_to_f32(e.bias.x >> 16);
+      f[2] += bf16_to_f32(e.bias.y & 0xffffu);
+      f[3] += bf16_to_f32(e.bias.y >> 16);
+    }
+    *reinterpret_cast<uint2*>(static_cast<uint16_t*>(P.y) + at) =
+        make_uint2(pack_bf16x2(f[0], f[1]), pack_bf16x2(f[2], f[3]));
+  } else {
+    skinny_store(P, m, n, v[0], e.bias);
+  }
 }
 
 // Problem of a column block (uniform over the workgroup).
@@ -2885,29 +2951,50 @@ skinny_problem(const SkinnyBatch& B, int cbg)
   return pi;
 }
 
-// Rows <= 16: a workgroup computes 16 output columns
-// over a K share; its four waves take every fourth K-block each and load
-// both operands straight into registers (the activation rows are few and
-// L2-resident), with no barrier until the four partial sums meet in LDS,
-// where wave 0 adds them in wave order.
+// The K-blocks of wave w of n in the kernels for at most 16 rows: groups of
+// G consecutive blocks, dealt round robin (so a pack's line of codes is one
+// wave's).  Pairs with four waves: groups of four made the bf16 kernel 3-5%
+// slower there (N = 12288, K = 4096, 1 row: 22.5 us against 21.5; single
+// blocks 21.3), and no slower with eight.  With S K shares of NW waves each,
+// wave w of share s is wave NW s + w of NW S.
+constexpr int sk_group(int nw) { return nw == 4 ? 2 : 4; }
+template <int G>
+struct SkOrder {
+  int w, n;
+  // block j of the wave
+  __device__ __forceinline__ int kb(int j) const { return G * (w + n * (j / G)) + j % G; }
+  // how many it has (the last group may be short); n is a power of two
+  __device__ __forceinline__ int blocks(int nkb) const
+  {
+    const int groups = (nkb + G - 1) / G;
+    const int mine = groups > w ? (groups - w + n - 1) >> __builtin_ctz(n) : 0;
+    return G * mine - (((groups - 1) & (n - 1)) == w ? G * groups - nkb : 0);
+  }
+};
+
+// Rows <= 16, packs whose scales narrow_pack_kernel cannot load by dwords: a
+// workgroup computes 16 output columns; its four waves load both operands
+// straight into registers (the activation rows are few and L2-resident),
+// with no barrier until the four partial sums meet in LDS, where wave 0 adds
+// them in wave order.
 template <int MT, int QB>
 __global__ __launch_bounds__(256) void
 skinny_reg_kernel(const SkinnyBatch B)
 {
-  __shared__ f32x4_t red[4][MT][64];
+  static_assert(MT == 1, "at most 16 rows");
+  __shared__ f32x4_t red[4][64];
   const int S = B.split;
   const int cbg = blockIdx.x / S;
   const int share = blockIdx.x - cbg * S;
   const SkinnyProblem& P = B.p[skinny_problem(B, cbg)];
   const int kbytes = B.kbytes;
   const int nkb = kbytes / 128;
-  const int kb0 = share * nkb / S;
-  const int nk = (share + 1) * nkb / S - kb0;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 4, r = lane & 15;
   const int n0 = (cbg - P.cb_begin) * 16;
-  const int nw = (nk - wave + 3) / 4;              // this wave's K-blocks
+  const SkOrder<sk_group(4)> order = {share * 4 + wave, S * 4};
+  const int nw = order.blocks(nkb);                // this wave's K-blocks
 
   // weight rows [n0, n0 + 16) and activation rows [0, rows); rows past
   // either read as zero
@@ -2916,26 +3003,18 @@ skinny_reg_kernel(const SkinnyBatch B)
   const int lv = r * kbytes + g * 32;               // row r, bytes 32g..
 
   SkW<QB> wreg[kSkDepth];
-  i32x4_t xreg[kSkDepth][MT][2];
+  i32x4_t xreg[kSkDepth][2];
   auto issue = [&](int slot, int j) {
-    const int oob = j < nw ? 0 : kOobOffset;        // past the share: zeros
-    const int kb = kb0 + wave + 4 * min(j, max(nw - 1, 0));
+    const int oob = j < nw ? 0 : kOobOffset;        // past the end: zeros
+    const int kb = min(order.kb(j), nkb - 1);
     const int ko = __builtin_amdgcn_readfirstlane(kb * 128);
     sk_load_w<QB>(wreg[slot], wsrc, kb, oob, B.qgroup);
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const int v = lv + mt * 16 * kbytes + oob;
-      xreg[slot][mt][0] = __builtin_amdgcn_raw_buffer_load_b128(xr, v, ko, 0);
-      xreg[slot][mt][1] = __builtin_amdgcn_raw_buffer_load_b128(xr, v + 16, ko, 0);
-    }
+    xreg[slot][0] = __builtin_amdgcn_raw_buffer_load_b128(xr, lv + oob, ko, 0);
+    xreg[slot][1] = __builtin_amdgcn_raw_buffer_load_b128(xr, lv + 16 + oob, ko, 0);
   };
 
-  f32x4_t acc[MT];
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    acc[mt] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-    asm volatile("" : "+v"(acc[mt]));
-  }
+  f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
+  asm volatile("" : "+v"(acc));
   asm volatile("s_nop 4");
   // the loads in K order (compiler fences between the blocks)
 #pragma unroll
@@ -2949,9 +3028,7 @@ skinny_reg_kernel(const SkinnyBatch B)
     for (int d = 0; d < kSkDepth; ++d) {
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks) {
-        const i32x4_t wf = sk_frag<QB>(wreg[d], ks);
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) { sk_mfma<QB>(acc[mt], wf, xreg[d][mt][ks]); }
+        sk_mfma<QB>(acc, sk_frag<QB>(wreg[d], ks), xreg[d][ks]);
       }
       asm volatile("" ::: "memory");
       issue(d, j0 + d + kSkDepth);
@@ -2959,120 +3036,315 @@ skinny_reg_kernel(const SkinnyBatch B)
   }
   asm volatile("s_waitcnt vmcnt(0)\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7"
                ::: "memory");
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    asm volatile("" : "+v"(acc[mt]));
-    red[wave][mt][lane] = acc[mt];
-  }
+  asm volatile("" : "+v"(acc));
+  red[wave][lane] = acc;
   __syncthreads();
   if (wave != 0) { return; }
   const int n = n0 + 4 * g;
-  if (n >= P.n) { return; }
-  uint2 bb = make_uint2(0u, 0u);
-  if (S == 1 && P.bias != nullptr) { bb = *reinterpret_cast<const uint2*>(P.bias + n); }
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    const int m = mt * 16 + r;
-    if (m >= P.rows) { continue; }
-    const f32x4_t v = ((red[0][mt][lane] + red[1][mt][lane]) + red[2][mt][lane]) +
-                      red[3][mt][lane];
-    if (S == 1) {
-      skinny_store(P, m, n, v, bb);
-    } else {
-      float* ws = B.ws + P.ws_off + (size_t)share * P.rows * P.n;
-      *reinterpret_cast<f32x4_t*>(ws + (size_t)m * P.n + n) = v;
-    }
+  if (n >= P.n || r >= P.rows) { return; }
+  SkEpi<kElBf16> epi;
+  if (S == 1) { epi = skinny_epi<kElBf16, false>(P, n); }
+  const f32x4_t v[1] = {((red[0][lane] + red[1][lane]) + red[2][lane]) + red[3][lane]};
+  if (S == 1) {
+    skinny_emit<kElBf16, false, 1>(P, r, n, v, epi);
+  } else {
+    float* ws = B.ws + P.ws_off + (size_t)(share * P.rows + r) * P.n + n;
+    *reinterpret_cast<f32x4_t*>(ws) = v[0];
   }
 }
 
-// Rows <= 16 with bf16 weights: skinny_reg_kernel's work split, but each
-// wave's 16 weight rows of a K-block arrive by two whole-line direct loads
-// global -> LDS (instruction i: rows 8i .. 8i+7, 8 lanes x 16 bytes per
-// 128-byte row) into the wave's own slot of a kSkDmaDepth-stage ring, and
-// the fragments are read back in the MFMA's layout (lane (g, r): row r,
-// 16-byte chunks 2g and 2g+1, the same K order as the register kernel, so
-// the two agree bit for bit).  The register kernel's lane layout asks for
-// every 128-byte line in two half-used requests.  Chunk c of row r sits at
-// position c ^ ((r >> 1) & 7) of its row, so the 16 lanes of a fragment
-// read (16 rows, one chunk) cover the 64 banks once.  The slots are
-// private to their wave: no barrier until the partial sums meet.
-// Measured (N = 6144, K = 4096, 12 rotated weight copies, same box): 12.6
-// / 13.2 / 15.4 us per call at 1 / 8 / 16 rows against 13.6-13.9 / 15.6 /
-// 18.2 for the register kernel.
-constexpr int kSkDmaDepth = 2;    // K-blocks in flight per wave (4 measured slower)
-
-template <int MT>
-__global__ __launch_bounds__(256) void
-skinny_dma_kernel(const SkinnyBatch B)
+// Rows <= 16, affine packs: the same work split and K order as
+// skinny_dma_tile (so u15h_linear_q equals u15h_linear on the expansion bit
+// for bit), with the codes copied to LDS by 128-byte lines: a stage is KPB
+// K-blocks, 4 at 4 bits or 2 at 8 (2 at 4 bits, 64 bytes of a row, with the
+// four waves' pairs).  Loaded straight into registers (skinny_reg_kernel) a
+// K-block is a 32- or 64-byte piece of each row and three loads; here a
+// stage takes two direct loads (one for 64 bytes) and, with WIDE, one load
+// each of the scales and the biases of all its K-blocks (dwords: 4-byte
+// aligned operands, an even number of groups per row), which a lane picks
+// its own from.
+// Bound: the codes and scales from HBM (0.63 bytes per weight at 4 bits and
+// group 32), and the dequantisation's ~4 VALU operations per weight.
+template <int QB, int GRP, int NW, bool WIDE>
+__global__ __launch_bounds__(64 * NW) void
+narrow_pack_kernel(const SkinnyBatch B)
 {
-  static_assert(kSkDmaDepth == 2 || kSkDmaDepth == 4, "ring of 2 or 4 stages");
-  __shared__ f32x4_t red[4][MT][64];
-  // one __shared__ object per stage, so the compiler tells a stage's reads
-  // from the copies filling another
-  __shared__ __attribute__((aligned(1024))) char wr0[4 * 2048];
-  __shared__ __attribute__((aligned(1024))) char wr1[4 * 2048];
-  __shared__ __attribute__((aligned(1024))) char wr2[kSkDmaDepth == 4 ? 4 * 2048 : 16];
-  __shared__ __attribute__((aligned(1024))) char wr3[kSkDmaDepth == 4 ? 4 * 2048 : 16];
+  // K-blocks per stage, bytes of a row's codes in it
+  constexpr int G = sk_group(NW);
+  constexpr int KPB = 16 / QB < G ? 16 / QB : G;
+  constexpr int kRow = KPB * 8 * QB;
+  static_assert(kRow == 128 || kRow == 64, "a line of codes, or half of one");
+  constexpr int kCh = kRow / 16;                   // 16-byte chunks per row
+  constexpr int kCopies = kRow / 64;               // 1 KiB direct loads per stage
+  constexpr int kDepth = kRow == 128 ? 2 : 4;      // 4 KiB in flight per wave
+  constexpr int kDwords = KPB * 32 / GRP;          // scale dwords per stage
+  constexpr int kSlot = 1024 * kCopies;
+  __shared__ f32x4_t red[NW][64];
+  __shared__ __attribute__((aligned(1024))) char wr0[NW * kSlot];
+  __shared__ __attribute__((aligned(1024))) char wr1[NW * kSlot];
+  __shared__ __attribute__((aligned(1024))) char wr2[kDepth == 4 ? NW * kSlot : 16];
+  __shared__ __attribute__((aligned(1024))) char wr3[kDepth == 4 ? NW * kSlot : 16];
+  char* const ring[4] = {wr0, wr1, wr2, wr3};
   const int S = B.split;
   const int cbg = blockIdx.x / S;
   const int share = blockIdx.x - cbg * S;
   const SkinnyProblem& P = B.p[skinny_problem(B, cbg)];
   const int kbytes = B.kbytes;
   const int nkb = kbytes / 128;
-  const int kb0 = share * nkb / S;
-  const int nk = (share + 1) * nkb / S - kb0;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 4, r = lane & 15;
   const int n0 = (cbg - P.cb_begin) * 16;
-  const int nw = (nk - wave + 3) / 4;              // this wave's K-blocks
+  const SkOrder<G> order = {share * NW + wave, S * NW};
+  const int nst = (order.blocks(nkb) + KPB - 1) / KPB;   // stages
+
+  // rows [n0, n0 + 16) of the pack clipped to n (rows past it read zero),
+  // activation rows [0, rows)
+  const SkWSrc src = sk_wsrc<QB>(B, P, n0, lane);
+  const int cpitch = kbytes / 2 * QB / 8;
+  const __amdgpu_buffer_rsrc_t xr = make_rsrc(P.a, P.rows * kbytes);
+  const int lv = r * kbytes + g * 32;
+  const int sv = r * (kbytes / 2 / GRP) * 2;       // the row's first scale
+  // chunk c of row r sits at position c ^ key(r): the 16 rows of a fragment
+  // read at one chunk then cover the banks once
+  auto key = [](int row) { return kCh == 8 ? (row >> 1) & 7 : (row >> 2) & 3; };
+  int dv[2];
+#pragma unroll
+  for (int i = 0; i < kCopies; ++i) {
+    const int row = (64 * i + lane) / kCh;
+    dv[i] = row * cpitch + ((((lane % kCh) ^ key(row))) << 4);
+  }
+  const int slot = wave * kSlot;
+  // the lane's 16 codes of K-block b of a stage: 16 bytes at chunk 4b + g
+  // (8 bits), 8 bytes of chunk 2b + g/2 (4 bits)
+  int rdo[4];
+#pragma unroll
+  for (int b = 0; b < KPB; ++b) {
+    const int c = QB == 8 ? 4 * b + g : 2 * b + (g >> 1);
+    rdo[b] = slot + r * kRow + ((c ^ key(r)) << 4) + (QB == 4 ? (g & 1) * 8 : 0);
+  }
+
+  // (fixed sizes: a lambda capturing an array of template-dependent size
+  // loses the kernel's host-side launch stub)
+  i32x4_t xreg[4][4][2];
+  uint32_t sreg[4][4], breg[4][4];         // dwords, or one u16 per block
+  auto issue = [&](char* stage, int d, int i) {
+    const int kb = order.kb(i * KPB);
+    const bool in = i < nst;
+    const int oob = in ? 0 : kOobOffset;           // past the end: zeros
+    const int ko = __builtin_amdgcn_readfirstlane(in ? kb * 8 * QB : 0);
+#pragma unroll
+    for (int j = 0; j < kCopies; ++j) {
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          src.w, (__attribute__((address_space(3))) void*)(stage + slot + j * 1024), 16,
+          dv[j] + oob, ko, 0, 0);
+    }
+    const int so = __builtin_amdgcn_readfirstlane(in ? kb * (64 / GRP) * 2 : 0);
+    if constexpr (WIDE && kDwords == 4) {
+      const u32x4_t a = __builtin_amdgcn_raw_buffer_load_b128(src.qs, sv + oob, so, 0);
+      const u32x4_t c = __builtin_amdgcn_raw_buffer_load_b128(src.qb, sv + oob, so, 0);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) { sreg[d][e] = a[e]; breg[d][e] = c[e]; }
+    } else if constexpr (WIDE && kDwords == 2) {
+      const u32x2_t a = __builtin_amdgcn_raw_buffer_load_b64(src.qs, sv + oob, so, 0);
+      const u32x2_t c = __builtin_amdgcn_raw_buffer_load_b64(src.qb, sv + oob, so, 0);
+#pragma unroll
+      for (int e = 0; e < 2; ++e) { sreg[d][e] = a[e]; breg[d][e] = c[e]; }
+    } else if constexpr (WIDE) {
+      sreg[d][0] = __builtin_amdgcn_raw_buffer_load_b32(src.qs, sv + oob, so, 0);
+      breg[d][0] = __builtin_amdgcn_raw_buffer_load_b32(src.qb, sv + oob, so, 0);
+    } else {
+#pragma unroll
+      for (int b = 0; b < KPB; ++b) {
+        const int v = src.sv + b * (64 / GRP) * 2 + oob;
+        sreg[d][b] = __builtin_amdgcn_raw_buffer_load_b16(src.qs, v, so, 0);
+        breg[d][b] = __builtin_amdgcn_raw_buffer_load_b16(src.qb, v, so, 0);
+      }
+    }
+#pragma unroll
+    for (int b = 0; b < KPB; ++b) {
+      const int xo = __builtin_amdgcn_readfirstlane(min(kb + b, nkb - 1) * 128);
+      xreg[d][b][0] = __builtin_amdgcn_raw_buffer_load_b128(xr, lv + oob, xo, 0);
+      xreg[d][b][1] = __builtin_amdgcn_raw_buffer_load_b128(xr, lv + 16 + oob, xo, 0);
+    }
+  };
+  // K-block b's entry of the lane's 16 weights
+  auto pick = [&](const uint32_t (&v)[4], int b) {
+    if constexpr (!WIDE) { return bf16_to_f32(v[b] & 0xffffu); }
+    if constexpr (GRP == 32) {
+      return __uint_as_float(g >= 2 ? v[b] & 0xffff0000u : v[b] << 16);
+    } else {
+      return __uint_as_float(b & 1 ? v[b >> 1] & 0xffff0000u : v[b >> 1] << 16);
+    }
+  };
+
+  f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
+  asm volatile("" : "+v"(acc));
+  asm volatile("s_nop 4");
+#pragma unroll
+  for (int d = 0; d < kDepth; ++d) {
+    asm volatile("" ::: "memory");
+    issue(ring[d], d, d);
+  }
+  constexpr int kScaleLoads = WIDE ? 2 : 2 * KPB;
+  constexpr int kAfter = (kDepth - 1) * (kCopies + kScaleLoads + 2 * KPB);
+  static_assert(kAfter < 64, "vmcnt holds at most 63");
+  const int pad = (nst + kDepth - 1) / kDepth * kDepth;
+  for (int i0 = 0; i0 < pad; i0 += kDepth) {
+#pragma unroll
+    for (int d = 0; d < kDepth; ++d) {
+      // the whole stage has landed (loads complete in issue order)
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kAfter) : "memory");
+      const int kb = order.kb((i0 + d) * KPB);
+#pragma unroll
+      for (int b = 0; b < KPB; ++b) {
+        // K-blocks past K (a short last stage) hold the next row's codes
+        if (kb + b >= nkb) { continue; }
+        const float sc = pick(sreg[d], b), bi = pick(breg[d], b);
+        uint32_t codes[4];
+        if constexpr (QB == 8) {
+          const i32x4_t c = *reinterpret_cast<const i32x4_t*>(ring[d] + rdo[b]);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) { codes[e] = (uint32_t)c[e]; }
+        } else {
+          // the nibbles as bytes: even codes, then odd, of each word
+          const u32x2_t c = *reinterpret_cast<const u32x2_t*>(ring[d] + rdo[b]);
+          codes[0] = c[0] & 0x0f0f0f0fu;
+          codes[1] = (c[0] >> 4) & 0x0f0f0f0fu;
+          codes[2] = c[1] & 0x0f0f0f0fu;
+          codes[3] = (c[1] >> 4) & 0x0f0f0f0fu;
+        }
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+          i32x4_t f;
+#pragma unroll
+          for (int e = 0; e < 8; e += 2) {
+            const uint32_t w0 = QB == 8 ? codes[2 * ks + (e >> 2)] : codes[2 * ks];
+            const uint32_t w1 = QB == 8 ? w0 : codes[2 * ks + 1];
+            const int b0 = QB == 8 ? (e & 3) * 8 : (e >> 1) * 8;
+            const int b1 = QB == 8 ? b0 + 8 : b0;
+            // a multiply, then an add (not fused), as dequant_affine_kernel
+            float p0 = sc * (float)((w0 >> b0) & 0xffu);
+            float p1 = sc * (float)((w1 >> b1) & 0xffu);
+            asm("" : "+v"(p0), "+v"(p1));
+            f[e >> 1] = (int)pack_bf16x2(p0 + bi, p1 + bi);
+          }
+          sk_mfma<QB>(acc, f, xreg[d][b][ks]);
+        }
+      }
+      asm volatile("" ::: "memory");
+      issue(ring[d], d, i0 + d + kDepth);
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0)\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7"
+               ::: "memory");
+  asm volatile("" : "+v"(acc));
+  red[wave][lane] = acc;
+  __syncthreads();
+  if (wave != 0) { return; }
+  const int n = n0 + 4 * g;
+  if (n >= P.n || r >= P.rows) { return; }
+  SkEpi<kElBf16> epi;
+  if (S == 1) { epi = skinny_epi<kElBf16, false>(P, n); }
+  f32x4_t v[1] = {red[0][lane]};
+#pragma unroll
+  for (int w = 1; w < NW; ++w) { v[0] += red[w][lane]; }
+  if (S == 1) {
+    skinny_emit<kElBf16, false, 1>(P, r, n, v, epi);
+  } else {
+    float* ws = B.ws + P.ws_off + (size_t)(share * P.rows + r) * P.n + n;
+    *reinterpret_cast<f32x4_t*>(ws) = v[0];
+  }
+}
+
+// Rows <= 16 (bf16 or int8 weights): a workgroup computes 16 output columns
+// (SW: the 16 gate and the 16 up columns of 16 SwiGLU outputs) over all of
+// K or a K share.  Its NW waves take the K-blocks in SkOrder's order; a wave's 16 weight
+// rows of a K-block arrive by two whole-line direct loads global -> LDS (instruction
+// i: rows 8i .. 8i+7, 8 lanes x 16 bytes per 128-byte row) into the wave's
+// own slot of a 2-stage ring, and the fragments are read back in the MFMA's
+// layout (lane (g, r): row r, 16-byte chunks 2g and 2g+1).  The register
+// kernel's lane layout asks for every 128-byte line in two half-used
+// requests.  Chunk c of row r sits at position c ^ ((r >> 1) & 7) of its
+// row, so the 16 lanes of a fragment read (16 rows, one chunk) cover the 64
+// banks once.  The slots are private to their wave: no barrier until the NW
+// partial sums meet in LDS, where wave 0 adds them in wave order.
+// Bound: HBM, the weights, N x K read once; a call of a few MB is its chain
+// of latencies.  Few columns take eight waves of one workgroup instead of K
+// shares, whose partial sums need a second launch (N = 4096, K = 4096, 1
+// row, in a graph: 9.2 us with 8 waves, 12.2 with two shares of 4).
+// Measured with NW = 4 (N = 6144, K = 4096, 12 rotated weight copies, same
+// box): 12.6 / 13.2 / 15.4 us per call at 1 / 8 / 16 rows against 13.6-13.9
+// / 15.6 / 18.2 for the register kernel; four stages were slower.
+constexpr int kSkDmaDepth = 2;    // K-blocks in flight per wave
+
+template <int NW, bool SW, int EL>
+__device__ __forceinline__ void
+skinny_dma_tile(const SkinnyBatch& B, char* const (&ring)[kSkDmaDepth],
+                sk_acc_t<EL> (&red)[NW][SW ? 2 : 1][64])
+{
+  constexpr int CW = SW ? 2 : 1;
+  const int S = B.split;
+  const int cbg = blockIdx.x / S;
+  const int share = blockIdx.x - cbg * S;
+  const SkinnyProblem& P = B.p[skinny_problem(B, cbg)];
+  const int kbytes = B.kbytes;
+  const int nkb = kbytes / 128;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g = lane >> 4, r = lane & 15;
+  const int n0 = (cbg - P.cb_begin) * 16;
+  const SkOrder<sk_group(NW)> order = {share * NW + wave, S * NW};
+  const int nw = order.blocks(nkb);                // this wave's K-blocks
 
   // weight rows [n0, n0 + 16) and activation rows [0, rows); rows past
   // either read as zero
   const int wrows = max(0, min(16, P.n - n0));
-  const __amdgpu_buffer_rsrc_t wrs =
-      make_rsrc(static_cast<const char*>(P.w) + (size_t)min(n0, P.n) * kbytes,
-                wrows * kbytes);
+  const size_t woff = (size_t)min(n0, P.n) * P.wld;
+  __amdgpu_buffer_rsrc_t wrs[CW];
+  wrs[0] = make_rsrc(static_cast<const char*>(P.w) + woff, wrows * P.wld);
+  if constexpr (SW) {
+    wrs[CW - 1] = make_rsrc(static_cast<const char*>(P.w2) + woff, wrows * P.wld);
+  }
   const __amdgpu_buffer_rsrc_t xr = make_rsrc(P.a, P.rows * kbytes);
   const int lv = r * kbytes + g * 32;               // row r, bytes 32g..
   int dv[2];
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const int row = 8 * i + (lane >> 3);
-    dv[i] = row * kbytes + (((lane & 7) ^ ((row >> 1) & 7)) << 4);
+    dv[i] = row * P.wld + (((lane & 7) ^ ((row >> 1) & 7)) << 4);
   }
-  const int slot = wave * 2048;
+  const int slot = wave * 2048 * CW;
   int rdo[2];
 #pragma unroll
   for (int ks = 0; ks < 2; ++ks) {
     rdo[ks] = slot + r * 128 + (((2 * g + ks) ^ ((r >> 1) & 7)) << 4);
   }
 
-  i32x4_t xreg[kSkDmaDepth][MT][2];
+  i32x4_t xreg[kSkDmaDepth][2];
   auto issue = [&](char* stage, int d, int j) {
-    const int oob = j < nw ? 0 : kOobOffset;        // past the share: zeros
-    const int kb = kb0 + wave + 4 * min(j, max(nw - 1, 0));
+    const int oob = j < nw ? 0 : kOobOffset;        // past the end: zeros
+    const int kb = min(order.kb(j), nkb - 1);
     const int ko = __builtin_amdgcn_readfirstlane(kb * 128);
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          wrs, (__attribute__((address_space(3))) void*)(stage + slot + i * 1024), 16,
-          dv[i] + oob, ko, 0, 0);
-    }
+    for (int c = 0; c < CW; ++c) {
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const int v = lv + mt * 16 * kbytes + oob;
-      xreg[d][mt][0] = __builtin_amdgcn_raw_buffer_load_b128(xr, v, ko, 0);
-      xreg[d][mt][1] = __builtin_amdgcn_raw_buffer_load_b128(xr, v + 16, ko, 0);
+      for (int i = 0; i < 2; ++i) {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            wrs[c],
+            (__attribute__((address_space(3))) void*)(stage + slot + c * 2048 + i * 1024), 16,
+            dv[i] + oob, ko, 0, 0);
+      }
     }
+    xreg[d][0] = __builtin_amdgcn_raw_buffer_load_b128(xr, lv + oob, ko, 0);
+    xreg[d][1] = __builtin_amdgcn_raw_buffer_load_b128(xr, lv + 16 + oob, ko, 0);
   };
-  char* const ring[4] = {wr0, wr1, wr2, wr3};
 
-  f32x4_t acc[MT];
+  sk_acc_t<EL> acc[CW];
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    acc[mt] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-    asm volatile("" : "+v"(acc[mt]));
+  for (int c = 0; c < CW; ++c) {
+    acc[c] = sk_acc_t<EL>{};
+    asm volatile("" : "+v"(acc[c]));
   }
   asm volatile("s_nop 4");
   // the loads in K order (compiler fences between the blocks)
@@ -3085,22 +3357,31 @@ skinny_dma_kernel(const SkinnyBatch B)
   // in flight (loads complete in issue order; the compiler may order a
   // block's copies and activation loads either way, so the whole block is
   // waited for)
-  constexpr int kAfter = (kSkDmaDepth - 1) * (2 + 2 * MT);
+  constexpr int kAfter = (kSkDmaDepth - 1) * (2 * CW + 2);
   static_assert(kAfter < 64, "vmcnt holds at most 63");
   const int nw_pad = (nw + kSkDmaDepth - 1) / kSkDmaDepth * kSkDmaDepth;
   for (int j0 = 0; j0 < nw_pad; j0 += kSkDmaDepth) {
 #pragma unroll
     for (int d = 0; d < kSkDmaDepth; ++d) {
       asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kAfter) : "memory");
-      i32x4_t wf[2];
+      i32x4_t wf[CW][2];
 #pragma unroll
-      for (int ks = 0; ks < 2; ++ks) {
-        wf[ks] = *reinterpret_cast<const i32x4_t*>(ring[d] + rdo[ks]);
+      for (int c = 0; c < CW; ++c) {
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+          wf[c][ks] = *reinterpret_cast<const i32x4_t*>(ring[d] + c * 2048 + rdo[ks]);
+        }
       }
 #pragma unroll
       for (int ks = 0; ks < 2; ++ks) {
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) { sk_mfma<0>(acc[mt], wf[ks], xreg[d][mt][ks]); }
+        for (int c = 0; c < CW; ++c) {
+          if constexpr (EL == kElBf16) {
+            sk_mfma<0>(acc[c], wf[c][ks], xreg[d][ks]);
+          } else {
+            sk_mfma_i8(acc[c], wf[c][ks], xreg[d][ks]);
+          }
+        }
       }
       // the MFMAs consumed this stage's reads; its slot takes block j + depth
       asm volatile("" ::: "memory");
@@ -3110,29 +3391,59 @@ skinny_dma_kernel(const SkinnyBatch B)
   asm volatile("s_waitcnt vmcnt(0)\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7\n\ts_nop 7"
                ::: "memory");
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    asm volatile("" : "+v"(acc[mt]));
-    red[wave][mt][lane] = acc[mt];
+  for (int c = 0; c < CW; ++c) {
+    asm volatile("" : "+v"(acc[c]));
+    red[wave][c][lane] = acc[c];
   }
   __syncthreads();
   if (wave != 0) { return; }
   const int n = n0 + 4 * g;
-  if (n >= P.n) { return; }
-  uint2 bb = make_uint2(0u, 0u);
-  if (S == 1 && P.bias != nullptr) { bb = *reinterpret_cast<const uint2*>(P.bias + n); }
+  if (n >= P.n || r >= P.rows) { return; }
+  SkEpi<EL> epi;
+  if (S == 1) { epi = skinny_epi<EL, SW>(P, n); }
+  sk_acc_t<EL> v[CW];
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    const int m = mt * 16 + r;
-    if (m >= P.rows) { continue; }
-    const f32x4_t v = ((red[0][mt][lane] + red[1][mt][lane]) + red[2][mt][lane]) +
-                      red[3][mt][lane];
-    if (S == 1) {
-      skinny_store(P, m, n, v, bb);
-    } else {
-      float* ws = B.ws + P.ws_off + (size_t)share * P.rows * P.n;
-      *reinterpret_cast<f32x4_t*>(ws + (size_t)m * P.n + n) = v;
+  for (int c = 0; c < CW; ++c) {
+    v[c] = red[0][c][lane];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) { v[c] += red[w][c][lane]; }
+  }
+  if (S == 1) {
+    skinny_emit<EL, SW, CW>(P, r, n, v, epi);
+  } else {
+#pragma unroll
+    for (int c = 0; c < CW; ++c) {
+      float* ws = B.ws + P.ws_off + (size_t)((c * S + share) * P.rows + r) * P.n + n;
+      *reinterpret_cast<sk_acc_t<EL>*>(ws) = v[c];
     }
   }
+}
+
+// bf16, four waves; narrow_dma_kernel: every other build.  One __shared__
+// object per stage, so the compiler tells a stage's reads from the copies
+// filling another.
+template <int MT>
+__global__ __launch_bounds__(256) void
+skinny_dma_kernel(const SkinnyBatch B)
+{
+  static_assert(MT == 1, "at most 16 rows");
+  __shared__ f32x4_t red[4][1][64];
+  __shared__ __attribute__((aligned(1024))) char wr0[4 * 2048];
+  __shared__ __attribute__((aligned(1024))) char wr1[4 * 2048];
+  char* const ring[2] = {wr0, wr1};
+  skinny_dma_tile<4, false, kElBf16>(B, ring, red);
+}
+
+template <int NW, bool SW, int EL>
+__global__ __launch_bounds__(64 * NW) void
+narrow_dma_kernel(const SkinnyBatch B)
+{
+  constexpr int kStageBytes = NW * 2048 * (SW ? 2 : 1);
+  __shared__ sk_acc_t<EL> red[NW][SW ? 2 : 1][64];
+  __shared__ __attribute__((aligned(1024))) char wr0[kStageBytes];
+  __shared__ __attribute__((aligned(1024))) char wr1[kStageBytes];
+  char* const ring[2] = {wr0, wr1};
+  skinny_dma_tile<NW, SW, EL>(B, ring, red);
 }
 
 // Rows 17..128: a workgroup computes 64 CW output columns over a K share.
@@ -3143,10 +3454,14 @@ skinny_dma_kernel(const SkinnyBatch B)
 // __shared__ object each, so the compiler can tell a stage's DMA from
 // another stage's reads).  MT row groups of 16; with CW = 2 every
 // activation fragment read from LDS serves two weight fragments.
-template <int MT, int D, int QB, int CW>
+// SW (CW = 2): a wave's two fragments are the 16 gate and the 16 up columns
+// of its 16 SwiGLU outputs.
+template <int MT, int D, int QB, int CW, bool SW = false, int EL = kElBf16>
 __device__ __forceinline__ void
 skinny_lds_tile(const SkinnyBatch& B, char* const (&xs)[D], char* const (&wsr)[D])
 {
+  static_assert(!SW || CW == 2, "SwiGLU pairs two fragments");
+  static_assert(QB == 0 || (!SW && EL == kElBf16), "packs: plain bf16 GEMMs");
   constexpr int kXInst = MT / 2;                    // DMA loads per wave
   // bf16 weights arrive like skinny_dma_kernel's: whole-line direct loads
   // into the wave's slot of a D-stage weight ring; packs load theirs into
@@ -3163,17 +3478,24 @@ skinny_lds_tile(const SkinnyBatch& B, char* const (&xs)[D], char* const (&wsr)[D
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 4, r = lane & 15;
-  const int n0 = (cbg - P.cb_begin) * 64 * CW + wave * 16 * CW;
+  constexpr int kCols = SW ? 16 : 16 * CW;         // output columns per wave
+  const int n0 = (cbg - P.cb_begin) * 4 * kCols + wave * kCols;
 
   // weight rows [n0 + 16c, n0 + 16c + 16) clipped to n: rows past it read
   // as zero
-  SkWSrc wsrc[CW];
+  SkWSrc wsrc[kWDma ? 1 : CW];
+  if constexpr (!kWDma) {
 #pragma unroll
-  for (int c = 0; c < CW; ++c) { wsrc[c] = sk_wsrc<QB>(B, P, n0 + 16 * c, lane); }
-  // the direct loads' view: rows [n0, n0 + 16 CW) clipped to n
-  const __amdgpu_buffer_rsrc_t wdr = make_rsrc(
-      static_cast<const char*>(P.w) + (size_t)min(n0, P.n) * kbytes,
-      max(0, min(16 * CW, P.n - n0)) * kbytes);
+    for (int c = 0; c < CW; ++c) { wsrc[c] = sk_wsrc<QB>(B, P, n0 + 16 * c, lane); }
+  }
+  // the direct loads' view: rows [n0, n0 + kCols) clipped to n (SW: of the
+  // gate and of the up weights)
+  const int wld = kWDma ? P.wld : kbytes;
+  const size_t woff = (size_t)min(n0, P.n) * wld;
+  const int wbytes = max(0, min(kCols, P.n - n0)) * wld;
+  const __amdgpu_buffer_rsrc_t wdr = make_rsrc(static_cast<const char*>(P.w) + woff, wbytes);
+  const __amdgpu_buffer_rsrc_t wdr2 =
+      SW ? make_rsrc(static_cast<const char*>(P.w2) + woff, wbytes) : wdr;
   // activation rows [0, rows): rows past them read as zero
   const __amdgpu_buffer_rsrc_t xr = make_rsrc(P.a, P.rows * kbytes);
   // DMA: instruction j of wave w fills 16-byte stage slots
@@ -3210,8 +3532,8 @@ skinny_lds_tile(const SkinnyBatch& B, char* const (&xs)[D], char* const (&wsr)[D
   int dv[2 * CW], rdo[2];
 #pragma unroll
   for (int j = 0; j < 2 * CW; ++j) {
-    const int row = 8 * j + (lane >> 3);
-    dv[j] = row * kbytes + (((lane & 7) ^ ((row >> 1) & 7)) << 4);
+    const int row = 8 * (SW ? j & 1 : j) + (lane >> 3);
+    dv[j] = row * wld + (((lane & 7) ^ ((row >> 1) & 7)) << 4);
   }
 #pragma unroll
   for (int ks = 0; ks < 2; ++ks) {
@@ -3224,7 +3546,8 @@ skinny_lds_tile(const SkinnyBatch& B, char* const (&xs)[D], char* const (&wsr)[D
 #pragma unroll
       for (int j = 0; j < 2 * CW; ++j) {
         __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            wdr, (__attribute__((address_space(3))) void*)(wsr[slot] + wave * 2048 * CW + j * 1024),
+            SW && j >= 2 ? wdr2 : wdr,
+            (__attribute__((address_space(3))) void*)(wsr[slot] + wave * 2048 * CW + j * 1024),
             16, dv[j] + oob, ko, 0, 0);
       }
     } else {
@@ -3235,12 +3558,13 @@ skinny_lds_tile(const SkinnyBatch& B, char* const (&xs)[D], char* const (&wsr)[D
     }
   };
 
-  f32x4_t acc[CW][MT];
+  using acc_t = sk_acc_t<EL>;
+  acc_t acc[CW][MT];
 #pragma unroll
   for (int c = 0; c < CW; ++c) {
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
-      acc[c][mt] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+      acc[c][mt] = acc_t{};
       asm volatile("" : "+v"(acc[c][mt]));
     }
   }
@@ -3312,7 +3636,13 @@ skinny_lds_tile(const SkinnyBatch& B, char* const (&xs)[D], char* const (&wsr)[D
             wf = sk_frag<QB>(wreg[d][c], ks);
           }
 #pragma unroll
-          for (int mt = 0; mt < MT; ++mt) { sk_mfma<QB>(acc[c][mt], wf, xf[mt][ks]); }
+          for (int mt = 0; mt < MT; ++mt) {
+            if constexpr (EL == kElBf16) {
+              sk_mfma<QB>(acc[c][mt], wf, xf[mt][ks]);
+            } else {
+              sk_mfma_i8(acc[c][mt], wf, xf[mt][ks]);
+            }
+          }
         }
       }
       // (the MFMAs consumed this block's weight reads before the refill)
@@ -3330,21 +3660,28 @@ skinny_lds_tile(const SkinnyBatch& B, char* const (&xs)[D], char* const (&wsr)[D
     for (int mt = 0; mt < MT; ++mt) { asm volatile("" : "+v"(acc[c][mt])); }
   }
 
+  // (with S > 1 the gate planes of all shares, then the up planes)
+  constexpr int kOut = SW ? 1 : CW;                // outputs per lane and row
 #pragma unroll
-  for (int c = 0; c < CW; ++c) {
+  for (int c = 0; c < kOut; ++c) {
     const int n = n0 + 16 * c + 4 * g;
     if (n >= P.n) { return; }
-    uint2 bb = make_uint2(0u, 0u);
-    if (S == 1 && P.bias != nullptr) { bb = *reinterpret_cast<const uint2*>(P.bias + n); }
+    SkEpi<EL> epi;
+    if (S == 1) { epi = skinny_epi<EL, SW>(P, n); }
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
       const int m = mt * 16 + r;
       if (m >= P.rows) { continue; }
       if (S == 1) {
-        skinny_store(P, m, n, acc[c][mt], bb);
+        acc_t v[SW ? 2 : 1];
+        v[0] = acc[c][mt];
+        if constexpr (SW) { v[1] = acc[1][mt]; }
+        skinny_emit<EL, SW, SW ? 2 : 1>(P, m, n, v, epi);
       } else {
-        float* ws = B.ws + P.ws_off + (size_t)share * P.rows * P.n;
-        *reinterpret_cast<f32x4_t*>(ws + (size_t)m * P.n + n) = acc[c][mt];
+        const size_t plane = (size_t)P.rows * P.n;
+        float* ws = B.ws + P.ws_off + (size_t)m * P.n + n;
+        *reinterpret_cast<acc_t*>(ws + share * plane) = acc[c][mt];
+        if constexpr (SW) { *reinterpret_cast<acc_t*>(ws + (S + share) * plane) = acc[1][mt]; }
       }
     }
   }
@@ -3376,12 +3713,42 @@ skinny_lds_kernel(const SkinnyBatch B)
   }
 }
 
-// Sums the S partial sums of every output in share order, adds the bias
-// and rounds to bf16: one thread per 4 columns of a row; blockIdx.y is the
-// problem.
+// SwiGLU and int8 forms of the same tile (MT row groups of 16, a D-stage
+// ring, CW fragments per wave).
+template <int MT, int D, int CW, bool SW, int EL>
+__global__ __launch_bounds__(256) void
+narrow_lds_kernel(const SkinnyBatch B)
+{
+  static_assert(D == 3 || D == 4, "a ring of 3 or 4 stages");
+  constexpr int kStage = MT * 16 * 128;
+  constexpr int kWStage = 4 * 2048 * CW;
+  __shared__ __attribute__((aligned(1024))) char xs0[kStage];
+  __shared__ __attribute__((aligned(1024))) char xs1[kStage];
+  __shared__ __attribute__((aligned(1024))) char xs2[kStage];
+  __shared__ __attribute__((aligned(1024))) char xs3[D == 4 ? kStage : 16];
+  __shared__ __attribute__((aligned(1024))) char ws0[kWStage];
+  __shared__ __attribute__((aligned(1024))) char ws1[kWStage];
+  __shared__ __attribute__((aligned(1024))) char ws2[kWStage];
+  __shared__ __attribute__((aligned(1024))) char ws3[D == 4 ? kWStage : 16];
+  if constexpr (D == 4) {
+    char* const xs[4] = {xs0, xs1, xs2, xs3};
+    char* const wsr[4] = {ws0, ws1, ws2, ws3};
+    skinny_lds_tile<MT, 4, 0, CW, SW, EL>(B, xs, wsr);
+  } else {
+    char* const xs[3] = {xs0, xs1, xs2};
+    char* const wsr[3] = {ws0, ws1, ws2};
+    skinny_lds_tile<MT, 3, 0, CW, SW, EL>(B, xs, wsr);
+  }
+}
+
+// Sums the S partial sums of every output in share order and applies the
+// epilogue: one thread per 4 columns of a row; blockIdx.y is the problem.
+template <int EL, bool SW>
 __global__ __launch_bounds__(256) void
 skinny_reduce_kernel(const SkinnyBatch B)
 {
+  constexpr int CW = SW ? 2 : 1;
+  using acc_t = sk_acc_t<EL>;
   const SkinnyProblem& P = B.p[blockIdx.y];
   const int q = P.n / 4;
   const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -3390,13 +3757,16 @@ skinny_reduce_kernel(const SkinnyBatch B)
   const int n = (int)(idx - (int64_t)m * q) * 4;
   const size_t plane = (size_t)P.rows * P.n;
   const float* ws = B.ws + P.ws_off + (size_t)m * P.n + n;
-  f32x4_t v = *reinterpret_cast<const f32x4_t*>(ws);
-  for (int sh = 1; sh < B.split; ++sh) {
-    v += *reinterpret_cast<const f32x4_t*>(ws + sh * plane);
+  const SkEpi<EL> epi = skinny_epi<EL, SW>(P, n);
+  acc_t v[CW];
+#pragma unroll
+  for (int c = 0; c < CW; ++c) {
+    v[c] = *reinterpret_cast<const acc_t*>(ws + c * B.split * plane);
+    for (int sh = 1; sh < B.split; ++sh) {
+      v[c] += *reinterpret_cast<const acc_t*>(ws + (c * B.split + sh) * plane);
+    }
   }
-  uint2 bb = make_uint2(0u, 0u);
-  if (P.bias != nullptr) { bb = *reinterpret_cast<const uint2*>(P.bias + n); }
-  skinny_store(P, m, n, v, bb);
+  skinny_emit<EL, SW, CW>(P, m, n, v, epi);
 }
 
 // ---- row gather / scatter for per-token routing ------------------------
@@ -3451,11 +3821,12 @@ launch_gemm(const GemmBatch& b, int cus, hipStream_t s, const GemmEvents& ev)
   return hipGetLastError();
 }
 
-template <class F>
+template <int EL = kElBf16, bool SW = false, class F>
 hipError_t
-launch_skinny(F kernel, const SkinnyBatch& b, hipStream_t s, const GemmEvents& ev)
+launch_skinny(F kernel, const SkinnyBatch& b, hipStream_t s, const GemmEvents& ev,
+              int threads = 256)
 {
-  launch_timed(kernel, dim3(b.total_cb * b.split), dim3(256), s, ev.before,
+  launch_timed(kernel, dim3(b.total_cb * b.split), dim3(threads), s, ev.before,
                ev.after, b);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || b.split <= 1) { return e; }
@@ -3463,20 +3834,50 @@ launch_skinny(F kernel, const SkinnyBatch& b, hipStream_t s, const GemmEvents& e
   for (int i = 0; i < b.nprob; ++i) {
     most = std::max<int64_t>(most, (int64_t)b.p[i].rows * (b.p[i].n / 4));
   }
-  launch_timed(skinny_reduce_kernel, dim3((unsigned)((most + 255) / 256), b.nprob),
+  launch_timed(skinny_reduce_kernel<EL, SW>, dim3((unsigned)((most + 255) / 256), b.nprob),
                dim3(256), s, ev.red_before, ev.red_after, b);
   return hipGetLastError();
 }
 
+template <int QB, int GRP, int NW>
+hipError_t
+launch_narrow_pack_waves(const SkinnyBatch& b, bool wide, hipStream_t s, const GemmEvents& ev)
+{
+  if (wide) { return launch_skinny(narrow_pack_kernel<QB, GRP, NW, true>, b, s, ev, 64 * NW); }
+  if constexpr (NW == 4) {
+    return launch_skinny(skinny_reg_kernel<1, QB>, b, s, ev);
+  } else {
+    return launch_skinny(narrow_pack_kernel<QB, GRP, NW, false>, b, s, ev, 64 * NW);
+  }
+}
+
+// Affine packs at most 16 rows.  Scales and biases are loaded by dwords
+// where every row starts on one: 4-byte aligned, an even number of groups.
+template <int QB>
+hipError_t
+launch_narrow_pack(const SkinnyBatch& b, hipStream_t s, const GemmEvents& ev)
+{
+  const uintptr_t at = reinterpret_cast<uintptr_t>(b.p[0].qs) | reinterpret_cast<uintptr_t>(b.p[0].qb);
+  const bool wide = at % 4 == 0 && b.kbytes / 2 / b.qgroup % 2 == 0;
+  if (b.qgroup == 32) {
+    return b.waves == 4 ? launch_narrow_pack_waves<QB, 32, 4>(b, wide, s, ev)
+                        : launch_narrow_pack_waves<QB, 32, 8>(b, wide, s, ev);
+  }
+  return b.waves == 4 ? launch_narrow_pack_waves<QB, 64, 4>(b, wide, s, ev)
+                      : launch_narrow_pack_waves<QB, 64, 8>(b, wide, s, ev);
+}
+
+// bf16 weights (plain) and affine packs.
 template <int QB>
 hipError_t
 launch_skinny_q(const SkinnyBatch& b, hipStream_t s, const GemmEvents& ev)
 {
   if (b.max_rows <= 16) {
     if constexpr (QB == 0) {
-      return launch_skinny(skinny_dma_kernel<1>, b, s, ev);
+      if (b.waves == 4) { return launch_skinny(skinny_dma_kernel<1>, b, s, ev); }
+      return launch_skinny(narrow_dma_kernel<8, false, kElBf16>, b, s, ev, 512);
     } else {
-      return launch_skinny(skinny_reg_kernel<1, QB>, b, s, ev);
+      return launch_narrow_pack<QB>(b, s, ev);
     }
   }
   if (b.max_rows <= 32) { return launch_skinny(skinny_lds_kernel<2, 4, QB>, b, s, ev); }
@@ -3493,22 +3894,75 @@ launch_skinny_q(const SkinnyBatch& b, hipStream_t s, const GemmEvents& ev)
   }
 }
 
+// SwiGLU pairs (bf16; b.cols output columns of 2 weight rows each).
+hipError_t
+launch_skinny_swiglu(const SkinnyBatch& b, hipStream_t s, const GemmEvents& ev)
+{
+  constexpr int E = kElBf16;
+  if (b.max_rows <= 16) {
+    if (b.waves == 4) { return launch_skinny<E, true>(narrow_dma_kernel<4, true, E>, b, s, ev); }
+    return launch_skinny<E, true>(narrow_dma_kernel<8, true, E>, b, s, ev, 512);
+  }
+  if (b.max_rows <= 32) { return launch_skinny<E, true>(narrow_lds_kernel<2, 4, 2, true, E>, b, s, ev); }
+  if (b.max_rows <= 64) { return launch_skinny<E, true>(narrow_lds_kernel<4, 3, 2, true, E>, b, s, ev); }
+  if (b.max_rows <= 96) { return launch_skinny<E, true>(narrow_lds_kernel<6, 4, 2, true, E>, b, s, ev); }
+  return launch_skinny<E, true>(narrow_lds_kernel<8, 4, 2, true, E>, b, s, ev);
+}
+
+// int8 codes to bf16 (kElI8) or int32 (kElI32).
+template <int E>
+hipError_t
+launch_skinny_i8_el(const SkinnyBatch& b, hipStream_t s, const GemmEvents& ev)
+{
+  if (b.max_rows <= 16) {
+    if (b.waves == 4) { return launch_skinny<E>(narrow_dma_kernel<4, false, E>, b, s, ev); }
+    return launch_skinny<E>(narrow_dma_kernel<8, false, E>, b, s, ev, 512);
+  }
+  if (b.max_rows <= 32) { return launch_skinny<E>(narrow_lds_kernel<2, 4, 1, false, E>, b, s, ev); }
+  if (b.max_rows <= 64) { return launch_skinny<E>(narrow_lds_kernel<4, 4, 1, false, E>, b, s, ev); }
+  if (b.max_rows <= 96) {
+    if (b.cols == 128) { return launch_skinny<E>(narrow_lds_kernel<6, 4, 2, false, E>, b, s, ev); }
+    return launch_skinny<E>(narrow_lds_kernel<6, 4, 1, false, E>, b, s, ev);
+  }
+  if (b.cols == 128) { return launch_skinny<E>(narrow_lds_kernel<8, 4, 2, false, E>, b, s, ev); }
+  return launch_skinny<E>(narrow_lds_kernel<8, 3, 1, false, E>, b, s, ev);
+}
+
+bool
+skinny_batch_ok(const SkinnyBatch& b)
+{
+  if (b.max_rows > kSkinnyMaxRows || b.kbytes % 128 != 0) { return false; }
+  const int cols = skinny_cols(b.max_rows, b.qbits);
+  return b.cols == cols || (skinny_wide_ok(b.max_rows, b.qbits) && b.cols == 2 * cols);
+}
+
 }  // namespace
 
 hipError_t
 launch_skinny_bf16(const SkinnyBatch& b, hipStream_t s, const GemmEvents& ev)
 {
   if (b.total_cb <= 0 || b.max_rows <= 0) { return hipSuccess; }
-  if (b.max_rows > kSkinnyMaxRows || b.kbytes % 128 != 0 ||
-      (b.cols != skinny_cols(b.max_rows, b.qbits) &&
-       !(skinny_wide_ok(b.max_rows, b.qbits) && b.cols == 2 * skinny_cols(b.max_rows, b.qbits))) ||
-      (b.qbits != 0 && b.qgroup != 32 && b.qgroup != 64)) {
+  if (!skinny_batch_ok(b) || (b.qbits != 0 && b.qgroup != 32 && b.qgroup != 64) ||
+      (b.swiglu && (b.qbits != 0 || b.cols != skinny_cols(b.max_rows, 0)))) {
     return hipErrorInvalidValue;
   }
+  if (b.swiglu) { return launch_skinny_swiglu(b, s, ev); }
   switch (b.qbits) {
     case 0: return launch_skinny_q<0>(b, s, ev);
     case 4: return launch_skinny_q<4>(b, s, ev);
     case 8: return launch_skinny_q<8>(b, s, ev);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+hipError_t
+launch_skinny_i8(const SkinnyBatch& b, Epi epi, hipStream_t s, const GemmEvents& ev)
+{
+  if (b.total_cb <= 0 || b.max_rows <= 0) { return hipSuccess; }
+  if (!skinny_batch_ok(b) || b.qbits != 0 || b.swiglu) { return hipErrorInvalidValue; }
+  switch (epi) {
+    case Epi::kI32: return launch_skinny_i8_el<kElI32>(b, s, ev);
+    case Epi::kDequantBf16: return launch_skinny_i8_el<kElI8>(b, s, ev);
     default: return hipErrorInvalidValue;
   }
 }
@@ -4063,7 +4517,45 @@ kernels_loadable()
       reinterpret_cast<const void*>(&skinny_lds_kernel<4, 4, 8>),
       reinterpret_cast<const void*>(&skinny_lds_kernel<6, 4, 8>),
       reinterpret_cast<const void*>(&skinny_lds_kernel<8, 4, 8>),
-      reinterpret_cast<const void*>(&skinny_reduce_kernel),
+      reinterpret_cast<const void*>(&narrow_dma_kernel<8, false, kElBf16>),
+      reinterpret_cast<const void*>(&narrow_dma_kernel<4, true, kElBf16>),
+      reinterpret_cast<const void*>(&narrow_dma_kernel<8, true, kElBf16>),
+      reinterpret_cast<const void*>(&narrow_lds_kernel<2, 4, 2, true, kElBf16>),
+      reinterpret_cast<const void*>(&narrow_lds_kernel<4, 3, 2, true, kElBf16>),
+      reinterpret_cast<const void*>(&narrow_lds_kernel<6, 4, 2, true, kElBf16>),
+      reinterpret_cast<const void*>(&narrow_lds_kernel<8, 4, 2, true, kElBf16>),
+      reinterpret_cast<const void*>(&narrow_dma_kernel<4, false, kElI8>),
+      reinterpret_cast<const void*>(&narrow_dma_kernel<8, false, kElI8>),
+      reinterpret_cast<const void*>(&narrow_lds_kernel<2, 4, 1, false, kElI8>),
+      reinterpret_cast<const void*>(&narrow_lds_kernel<4, 4, 1, false, kElI8>),
+      reinterpret_cast<const void*>(&narrow_lds_kernel<6, 4, 1, false, kElI8>),
+      reinterpret_cast<const void*>(&narrow_lds_kernel<6, 4, 2, false, kElI8>),
+      reinterpret_cast<const void*>(&narrow_lds_kernel<8, 3, 1, false, kElI8>),
+      reinterpret_cast<const void*>(&narrow_lds_kernel<8, 4, 2, false, kElI8>),
+      reinterpret_cast<const void*>(&skinny_reduce_kernel<kElI8, false>),
+      reinterpret_cast<const void*>(&narrow_dma_kernel<4, false, kElI32>),
+      reinterpret_cast<const void*>(&narrow_dma_kernel<8, false, kElI32>),
+      reinterpret_cast<const void*>(&narrow_lds_kernel<2, 4, 1, false, kElI32>),
+      reinterpret_cast<const void*>(&narrow_lds_kernel<4, 4, 1, false, kElI32>),
+      reinterpret_cast<const void*>(&narrow_lds_kernel<6, 4, 1, false, kElI32>),
+      reinterpret_cast<const void*>(&narrow_lds_kernel<6, 4, 2, false, kElI32>),
+      reinterpret_cast<const void*>(&narrow_lds_kernel<8, 3, 1, false, kElI32>),
+      reinterpret_cast<const void*>(&narrow_lds_kernel<8, 4, 2, false, kElI32>),
+      reinterpret_cast<const void*>(&skinny_reduce_kernel<kElI32, false>),
+      reinterpret_cast<const void*>(&narrow_pack_kernel<4, 32, 4, true>),
+      reinterpret_cast<const void*>(&narrow_pack_kernel<4, 32, 8, true>),
+      reinterpret_cast<const void*>(&narrow_pack_kernel<4, 32, 8, false>),
+      reinterpret_cast<const void*>(&narrow_pack_kernel<4, 64, 4, true>),
+      reinterpret_cast<const void*>(&narrow_pack_kernel<4, 64, 8, true>),
+      reinterpret_cast<const void*>(&narrow_pack_kernel<4, 64, 8, false>),
+      reinterpret_cast<const void*>(&narrow_pack_kernel<8, 32, 4, true>),
+      reinterpret_cast<const void*>(&narrow_pack_kernel<8, 32, 8, true>),
+      reinterpret_cast<const void*>(&narrow_pack_kernel<8, 32, 8, false>),
+      reinterpret_cast<const void*>(&narrow_pack_kernel<8, 64, 4, true>),
+      reinterpret_cast<const void*>(&narrow_pack_kernel<8, 64, 8, true>),
+      reinterpret_cast<const void*>(&narrow_pack_kernel<8, 64, 8, false>),
+      reinterpret_cast<const void*>(&skinny_reduce_kernel<kElBf16, false>),
+      reinterpret_cast<const void*>(&skinny_reduce_kernel<kElBf16, true>),
   };
   for (const void* f : fns) {
     hipFuncAttributes a;
