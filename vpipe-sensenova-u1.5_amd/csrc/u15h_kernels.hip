@@ -2271,9 +2271,10 @@ attention_kernel(const AttnArgs A)
     voffs[i] = (r * D + (((idx % KCH) ^ (4 * vswz<D>(r))) << 3)) * 2;
   }
   int32_t tr = 0;
-  int kstop = A.tk;          // the copies' range: [0, kstop)
+  int kstop_split = 0;       // the copies' range: keys [0, kstop())
+  auto kstop = [&] { return SPLIT ? kstop_split : A.tk; };
   auto copy_k = [&](int j0, uint16_t* dst_tile) {
-    const int left = max(kstop - j0, 0);
+    const int left = max(kstop() - j0, 0);
     const __amdgpu_buffer_rsrc_t rs = make_rsrc(kbase + (long long)j0 * D, left * D * 2);
     char* dst = reinterpret_cast<char*>(dst_tile) + wave * CPW * 1024;
     if (kCopyWaves == NWV || wave < kCopyWaves) {
@@ -2290,7 +2291,7 @@ attention_kernel(const AttnArgs A)
     }
   };
   auto copy_v = [&](int j0, uint16_t* dst_tile) {
-    const int left = max(kstop - j0, 0);
+    const int left = max(kstop() - j0, 0);
     const __amdgpu_buffer_rsrc_t rs = make_rsrc(vbase + (long long)j0 * D, left * D * 2);
     char* dst = reinterpret_cast<char*>(dst_tile) + wave * CPW * 1024;
     if (kCopyWaves == NWV || wave < kCopyWaves) {
@@ -2332,7 +2333,7 @@ attention_kernel(const AttnArgs A)
   // after it are fully masked and would add exactly 0.
   int kend = A.tk;
   if constexpr (MODE != 0) {
-    const int q_last = A.q_offset + tok1;
+    const int q_last = A.q_offset + (SPLIT ? tok1 : min(A.tq, qt * QT + QT) - 1);
     kend = min(A.tk, q_last + 1);
   }
   if constexpr (MODE == 2) {
@@ -2341,7 +2342,7 @@ attention_kernel(const AttnArgs A)
     // [tmin, tmax] (a superset of the visible keys; the mask is exact).
     __shared__ int kred[3][NWV];
     int tmin = INT_MAX, tmax = INT_MIN;
-    if (tid < QT && tok0 + tid <= tok1) {
+    if (tid < QT && (SPLIT ? tok0 + tid <= tok1 : qt * QT + tid < A.tq)) {
       const int tv = A.t_index[q_first + tid];
       tmin = tv;
       tmax = tv;
@@ -2383,7 +2384,7 @@ attention_kernel(const AttnArgs A)
     const int all = ntiles;
     tbeg = (int)((long long)share * all / A.shares);
     ntiles = (int)((long long)(share + 1) * all / A.shares);
-    kstop = min(A.tk, ntiles * BK);
+    kstop_split = min(A.tk, ntiles * BK);
   }
 
   // -inf for the scores of tile j0 that the mode hides; a no-op for a tile
@@ -2510,7 +2511,7 @@ attention_kernel(const AttnArgs A)
       __builtin_amdgcn_sched_group_barrier(0x002, 6 * EPB / 4, 0);    // VALU
     }
     // ---- C --------------------------------------------------------------
-    mask(sn, j0 + BK, (t - tbeg + 1) % 3);
+    mask(sn, j0 + BK, ((SPLIT ? t - tbeg : t) + 1) % 3);
     float mx = -INFINITY;
 #pragma unroll
     for (int k4 = 2; k4 < 4; ++k4) {
@@ -2531,7 +2532,7 @@ attention_kernel(const AttnArgs A)
     }
     mb = max_halves(mx);
     l += ps;
-    store_t((t - tbeg + 2) % 3);
+    store_t(((SPLIT ? t - tbeg : t) + 2) % 3);
     __syncthreads();
     sc[0] = sn[0];
     sc[1] = sn[1];
