@@ -1,0 +1,97 @@
+"""The mid-size tiles (mid_gemm_kernel: 128, 192 or 256 rows x 128 weight
+rows) against the 256 x 256 tiles of a context built with U15H_MID=0: equal
+bits on operands whose sums are exact in any order, for every epilogue, at
+row and column counts around the tiles' edges, K tails, whole rounds, split
+tails, and both groups with and without bias; and the planner's choice
+against the tiled kernel and the oracle on random operands."""
+import os
+
+import numpy as np
+import pytest
+import torch
+
+import oracle
+import u15h
+from helpers import dev_bf16, host_f32, max_rel, rand_bf16_bits, rel_l2
+
+pytestmark = pytest.mark.gpu
+
+
+def ctx_with(**env):
+    old = {k: os.environ.get(k) for k in env}
+    os.environ.update({k: str(v) for k, v in env.items()})
+    try:
+        return u15h.Ops(0)
+    finally:
+        for k, v in old.items():
+            if v is None:
+                del os.environ[k]
+            else:
+                os.environ[k] = v
+
+
+@pytest.fixture(scope="module")
+def contexts():
+    made = {bm: ctx_with(U15H_MID=bm) for bm in (0, 128, 192, 256)}
+    made["one"] = ctx_with(U15H_MID=192, U15H_SPLIT=0, U15H_PERSIST=0)
+    yield made
+    torch.cuda.synchronize()
+    for o in made.values():
+        o.close()
+
+
+def ints(rng, shape, top):
+    return dev_bf16(oracle.f32_to_bf16(rng.integers(-top, top + 1, shape).astype(np.float32)))
+
+
+@pytest.mark.parametrize("Mu,Mg,K,N", [
+    (0, 129, 64, 8), (129, 0, 72, 136), (43, 157, 192, 264), (0, 333, 1088, 1000),
+    (128, 192, 640, 2056), (191, 193, 4096, 128), (257, 0, 2048, 520), (1, 1023, 256, 4104),
+    (100, 1500, 320, 264)])
+@pytest.mark.parametrize("bm", [128, 192, 256, "one"])
+def test_exact_sums_equal_the_256_tiles(contexts, bm, Mu, Mg, K, N):
+    rng = np.random.default_rng(Mu + Mg + K + N)
+    M = Mu + Mg
+    x, bias = ints(rng, (M, K), 2), [ints(rng, (N,), 3) for _ in range(2)]
+    w = [ints(rng, (N, K), 1) for _ in range(4)]
+    xq = torch.from_numpy(rng.integers(-127, 128, (M, K)).astype(np.int8)).cuda()
+    wq = [torch.from_numpy(rng.integers(-127, 128, (N, K)).astype(np.int8)).cuda()
+          for _ in range(2)]
+    sx, s0, s1 = (torch.from_numpy(rng.random(n).astype(np.float32)).cuda() for n in (M, N, N))
+
+    def run(o):
+        def out(dtype=torch.bfloat16, n=N):
+            return torch.full((M, n), 7, dtype=dtype, device="cuda")
+        ys = [out(), out(), out()]
+        o.mot_linear(x, Mu, Mg, K, [
+            dict(w_und=w[0], w_gen=w[1], bias_und=bias[0], bias_gen=bias[1], y=ys[0]),
+            dict(w_und=w[2], w_gen=w[3], y=ys[1])])
+        o.mot_gate_up_swiglu(x, Mu, Mg, K, *w, ys[2])
+        if K % 128 == 0:
+            proj = dict(wq_und=wq[0], wq_gen=wq[1], sw_und=s0, sw_gen=s1)
+            ys += [out(torch.int32), out()]
+            o.mot_gemm_i8_i32(xq, Mu, Mg, K, [dict(proj, y=ys[3])])
+            o.mot_gemm_i8(xq, sx, Mu, Mg, K, [dict(proj, y=ys[4])])
+        torch.cuda.synchronize()
+        return ys
+    for a, b in zip(run(contexts[bm]), run(contexts[0])):
+        assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+
+
+@pytest.mark.parametrize("M,K,N", [(130, 4096, 1032), (333, 4096, 4096), (1100, 1024, 2056)])
+def test_planned_tiles(ops, contexts, M, K, N):
+    """The default context's choice (a mid-size tile at these shapes) on
+    random operands, with bias, at the reference's bars."""
+    rng = np.random.default_rng(M + K + N)
+    xb, wb = rand_bf16_bits(rng, (M, K)), rand_bf16_bits(rng, (N, K), 0.02)
+    bb = rand_bf16_bits(rng, (N,), 0.5)
+    x, w, b = dev_bf16(xb), dev_bf16(wb), dev_bf16(bb)
+    y, t = (torch.full((M, N), 7.0, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    ops.linear(x, w, b, y, M, K, N)
+    contexts[0].linear(x, w, b, t, M, K, N)
+    torch.cuda.synchronize()
+    assert rel_l2(host_f32(y), host_f32(t)) < 4e-3
+    rows = np.array([0, M // 2, M - 1], np.int32)
+    ref = oracle.linear_bf16(xb, wb, bb, row_ids=rows)
+    a = host_f32(y)[rows]
+    assert max_rel(a, ref) <= 1e-2 and rel_l2(a, ref) < 4e-3

@@ -36,6 +36,8 @@ struct u15h_ctx {
   // GEMM kernel build: 8 or 4 waves per workgroup (env U15H_WAVES) and the
   // 8-wave build's MFMA shape (env U15H_MFMA16).
   u15h::GemmShape gemm = {8, 0, 1};
+  bool mid_on = true;        // the mid-size tiles (env U15H_MID)
+  int mid_bm = 0;            // nonzero: that one always
   // One-shot profiling events, bound to the next launches of a quantiser,
   // a GEMM kernel and its reduction (start and end of each); all dropped
   // when the next GEMM call has launched.
@@ -171,7 +173,26 @@ empty_batch(int kbytes)
   std::memset(&b, 0, sizeof b);
   b.kbytes = kbytes;
   b.split = 1;
+  b.bm = u15h::kBM;
+  b.bn = u15h::kBN;
   return b;
+}
+
+// Recounts the tiles of a batch for tiles of bm rows x bn weight rows.
+void
+set_tiles(GemmBatch& b, Epi epi, int bm, int bn)
+{
+  b.bm = bm;
+  b.bn = bn;
+  b.total_tiles = 0;
+  const int cols = u15h::tile_cols(epi, bn);
+  for (int i = 0; i < b.nprob; ++i) {
+    GemmProblem& p = b.p[i];
+    p.tiles_m = (p.rows + bm - 1) / bm;
+    p.tiles_n = (p.n + cols - 1) / cols;
+    p.tile_begin = b.total_tiles;
+    b.total_tiles += p.tiles_m * p.tiles_n;
+  }
 }
 
 // Scratch of split attention calls, per context.
@@ -186,7 +207,74 @@ split_ws_capacity(const u15h_ctx* ctx)
   return (size_t)ctx->num_cu * u15h::kBM * u15h::kBN * 4;
 }
 
-// Chooses the split-K tail of a batch once its tiles are known.  With T
+// K shares of a last round of `rem` tiles over C compute units.
+int
+tail_shares(const u15h_ctx* ctx, int rem, int nk)
+{
+  if (!ctx->split_on || rem == 0) { return 1; }
+  return std::max(1, std::min(ctx->gemm_cus / rem, nk / kMinStagesPerShare));
+}
+
+// Estimated time (us) of a batch on its tiles: `stage` us per K stage and
+// round, 5 us per round of prologue and epilogue, and for split tails the
+// partial sums' round trip (3.5 us + 0.3 us per MB, valid rows only).
+double
+tiles_estimate(const u15h_ctx* ctx, const GemmBatch& b, double stage)
+{
+  const int C = ctx->gemm_cus, T = b.total_tiles;
+  const int nk = (b.kbytes + u15h::kKB - 1) / u15h::kKB;
+  const int full = T / C, rem = T % C, S = tail_shares(ctx, rem, nk);
+  double rows = 0, padded = 0;
+  for (int i = 0; i < b.nprob; ++i) {
+    rows += (double)b.p[i].rows * b.p[i].tiles_n;
+    padded += (double)b.p[i].tiles_m * b.bm * b.p[i].tiles_n;
+  }
+  double us = full * (nk * stage + 5.0);
+  if (rem > 0) { us += (nk + S - 1) / S * stage + 5.0; }
+  if (S > 1) { us += 3.5 + 0.3e-6 * rem * S * b.bm * b.bn * 4.0 * (rows / padded); }
+  return us;
+}
+
+// Chooses the tile size of a batch, counted on 256 x 256 tiles: those, or the
+// mid-size kernel's where their estimate is at least 5% lower.  Stage times
+// as measured: the 256 x 256 kernel's by the share of CUs it keeps busy (1.22
+// us at 144, 1.34 at 192, 1.5 at 256), the mid-size ones' growing with K
+// (128 rows: 0.54 us at 64 stages, 0.58 at 192) and 10% longer for int8.
+// Estimated / measured, us: M = 333, K
+// = 12288, N = 4096: 256 x 256 57.5 / 55.8, 192 48.6 / 51.2, 128 63.7 / 63.9;
+// M = 1024, K = 4096, N = 12288: 256 x 256 91 / 91.2, 256 110 / 111.9; M =
+// 512, K = 4096, N = 12288: 256 x 256 66.5 / 67.9, 256 62.6 / 61.4.  The
+// 256 x 256 tiles' other builds (U15H_WAVES, U15H_MFMA16) have no mid-size
+// form and keep their tiles.
+void
+pick_tiles(const u15h_ctx* ctx, GemmBatch& b, Epi epi)
+{
+  if (!ctx->mid_on || b.total_tiles <= 0) { return; }
+  const int C = ctx->gemm_cus, T = b.total_tiles;
+  const int nk = (b.kbytes + u15h::kKB - 1) / u15h::kKB;
+  const int busy = T >= C ? C : T * tail_shares(ctx, T, nk);
+  double best = 0.95 * tiles_estimate(ctx, b, 0.85 + 0.65 * busy / C);
+  int bm = 0;
+  const struct { int bm; double stage; } mid[] = {{128, 0.525}, {192, 0.68}, {256, 0.875}};
+  const double longer = (1.0 + nk / 1920.0) *
+                        (epi == Epi::kI32 || epi == Epi::kDequantBf16 ? 1.1 : 1.0);
+  for (const auto& m : mid) {
+    if (ctx->mid_bm != 0 && ctx->mid_bm != m.bm) { continue; }
+    set_tiles(b, epi, m.bm, u15h::kMidBN);
+    const double us = tiles_estimate(ctx, b, m.stage * longer);
+    if (us < best || ctx->mid_bm != 0) {
+      best = us;
+      bm = m.bm;
+    }
+  }
+  if (bm != 0) {
+    set_tiles(b, epi, bm, u15h::kMidBN);
+  } else {
+    set_tiles(b, epi, u15h::kBM, u15h::kBN);
+  }
+}
+
+// Chooses the tiles and the split-K tail of a batch.  With T
 // tiles on C compute units, the last T % C tiles would run as a last,
 // partial round that leaves most units idle; instead each is cut into
 // S = C / (T % C) shares of its K stages (so the shares fill about one
@@ -194,8 +282,9 @@ split_ws_capacity(const u15h_ctx* ctx)
 // the context's workspace (allocated on first use), or with `noalloc` to
 // the static scratch, which allocates nothing.
 u15h_status
-plan_split(u15h_ctx* ctx, GemmBatch& b, bool noalloc = false)
+plan_split(u15h_ctx* ctx, GemmBatch& b, Epi epi, bool noalloc = false)
 {
+  pick_tiles(ctx, b, epi);
   b.split = 1;
   b.split_begin = b.total_tiles;
   b.ws = nullptr;
@@ -204,7 +293,7 @@ plan_split(u15h_ctx* ctx, GemmBatch& b, bool noalloc = false)
   const int rem = T % C;
   if (!ctx->split_on || T <= 0 || rem == 0) { return U15H_OK; }
   const int nk = (b.kbytes + u15h::kKB - 1) / u15h::kKB;
-  const int S = std::min(C / rem, nk / kMinStagesPerShare);
+  const int S = tail_shares(ctx, rem, nk);
   if (S < 2) { return U15H_OK; }
   b.split = S;
   b.split_begin = T - rem;
@@ -498,7 +587,7 @@ linear_i8_route(u15h_ctx* ctx, hipStream_t s, const u15h_bf16* x,
   if (skinny_fits(ctx, b, Epi::kDequantBf16)) {
     return skinny_launch(ctx, b, Epi::kDequantBf16, s, false, take_profile_event(ctx));
   }
-  u15h_status st = plan_split(ctx, b);
+  u15h_status st = plan_split(ctx, b, Epi::kDequantBf16);
   if (st != U15H_OK) { return st; }
   return launched(ctx, u15h::launch_gemm_i8(b, Epi::kDequantBf16, ctx->gemm, s, take_profile_event(ctx)),
                   "gemm_i8");
@@ -583,6 +672,11 @@ u15h_create(int device, u15h_ctx** out)
                                        env_int("U15H_GEMM_CUS", ctx->num_cu) / 8 * 8));
   ctx->gemm.cus = env_int("U15H_PERSIST", 1) != 0 ? ctx->gemm_cus : 0;
   ctx->gemm.mfma16 = std::max(-1, std::min(1, env_int("U15H_MFMA16", 1)));
+  // env U15H_MID: 0 keeps every batch on the 256 x 256 tiles, 128 / 192 / 256
+  // forces that mid-size tile
+  const int mid = env_int("U15H_MID", 1);
+  ctx->mid_on = mid != 0 && ctx->gemm.waves == 8 && ctx->gemm.mfma16 == 1;
+  ctx->mid_bm = mid == 128 || mid == 192 || mid == 256 ? mid : 0;
   ctx->i8_min_m = std::max(1, env_int("U15H_I8_MIN_M", 1024));
   ctx->attn_split = env_int("U15H_ATTN_SPLIT", -1);
   if (ctx->attn_split != 0 && hipMalloc(&ctx->attn_ws, kAttnWsBytes) != hipSuccess) {
@@ -632,7 +726,7 @@ dense_bf16(u15h_ctx* ctx, hipStream_t s, const u15h_bf16* x,
   if (skinny_fits(ctx, b, Epi::kBf16)) {
     return skinny_launch(ctx, b, Epi::kBf16, s, false, take_profile_event(ctx));
   }
-  u15h_status st = plan_split(ctx, b);
+  u15h_status st = plan_split(ctx, b, Epi::kBf16);
   if (st != U15H_OK) { return st; }
   return launched(ctx, u15h::launch_gemm_bf16(b, Epi::kBf16, ctx->gemm, s, take_profile_event(ctx)), "gemm_bf16");
 }
@@ -721,7 +815,7 @@ mot_linear_impl(u15h_ctx* ctx, u15h_stream stream, const u15h_bf16* x,
     return skinny_launch(ctx, b, Epi::kBf16, as_stream(stream), noalloc,
                          take_profile_event(ctx));
   }
-  if ((st = plan_split(ctx, b, noalloc)) != U15H_OK) { return st; }
+  if ((st = plan_split(ctx, b, Epi::kBf16, noalloc)) != U15H_OK) { return st; }
   return launched(ctx, u15h::launch_gemm_bf16(b, Epi::kBf16, ctx->gemm, as_stream(stream), take_profile_event(ctx)),
                   "mot_gemm_bf16");
 }
@@ -917,7 +1011,7 @@ u15h_mot_gate_up_swiglu(u15h_ctx* ctx, u15h_stream stream,
     return skinny_launch(ctx, b, Epi::kSwiglu, as_stream(stream), false,
                          take_profile_event(ctx));
   }
-  if ((st = plan_split(ctx, b)) != U15H_OK) { return st; }
+  if ((st = plan_split(ctx, b, Epi::kSwiglu)) != U15H_OK) { return st; }
   return launched(ctx, u15h::launch_gemm_bf16(b, Epi::kSwiglu, ctx->gemm, as_stream(stream), take_profile_event(ctx)),
                   "mot_gate_up_swiglu");
 }
@@ -1062,7 +1156,7 @@ mot_gemm_i8_common(u15h_ctx* ctx, u15h_stream stream, const int8_t* xq,
   if (skinny_fits(ctx, b, epi)) {
     return skinny_launch(ctx, b, epi, as_stream(stream), false, take_profile_event(ctx));
   }
-  if ((st = plan_split(ctx, b)) != U15H_OK) { return st; }
+  if ((st = plan_split(ctx, b, epi)) != U15H_OK) { return st; }
   return launched(ctx, u15h::launch_gemm_i8(b, epi, ctx->gemm, as_stream(stream), take_profile_event(ctx)),
                   deq ? "mot_gemm_i8" : "mot_gemm_i8_i32");
 }
@@ -1227,7 +1321,7 @@ u15h_swiglu_fused(u15h_ctx* ctx, u15h_stream stream, const u15h_bf16* x,
     return skinny_launch(ctx, b, Epi::kSwiglu, as_stream(stream), false,
                          take_profile_event(ctx));
   }
-  if ((st = plan_split(ctx, b)) != U15H_OK) { return st; }
+  if ((st = plan_split(ctx, b, Epi::kSwiglu)) != U15H_OK) { return st; }
   return launched(ctx,
                   u15h::launch_gemm_bf16(b, Epi::kSwiglu, ctx->gemm,
                                          as_stream(stream),

@@ -15,6 +15,7 @@ namespace u15h {
 // LDS byte layout and one load schedule; only the MFMA differs.
 constexpr int kBM = 256;          // activation rows per tile
 constexpr int kBN = 256;          // weight rows (output columns) per tile
+constexpr int kMidBN = 128;       // weight rows per tile of the mid-size kernels
 constexpr int kKB = 128;          // bytes of K per stage
 constexpr int kMaxProb = 8;       // problems (weight sets x projections) per launch
 
@@ -57,7 +58,8 @@ struct GemmBatch {
   int total_tiles;
   int split_begin;        // == total_tiles when nothing is split
   int split;              // K shares per split tile (1 = no split)
-  void* ws;               // [(tile - split_begin) * split + share][kBM][kBN]
+  int bm, bn;             // tile: 256 x 256, or 128 / 192 / 256 x kMidBN
+  void* ws;               // [(tile - split_begin) * split + share][bm][bn]
 };
 
 // Workgroups a batch launches.
@@ -68,7 +70,7 @@ __host__ __device__ inline int grid_blocks(const GemmBatch& b)
 // Bytes of partial-sum workspace a batch needs.
 inline size_t split_ws_bytes(const GemmBatch& b)
 {
-  return (size_t)(b.total_tiles - b.split_begin) * b.split * kBM * kBN * 4;
+  return (size_t)(b.total_tiles - b.split_begin) * b.split * b.bm * b.bn * 4;
 }
 
 // Kernel launchers (u15h_kernels.hip).  All are asynchronous on `s`.
@@ -270,7 +272,7 @@ hipError_t noalloc_scratch(int device, void** out);
 u15h_status set_error(u15h_ctx* ctx, u15h_status st, const char* msg);
 
 // Tile columns per tile for an epilogue (kSwiglu tiles produce half).
-constexpr int tile_cols(Epi e) { return e == Epi::kSwiglu ? kBN / 2 : kBN; }
+constexpr int tile_cols(Epi e, int bn = kBN) { return e == Epi::kSwiglu ? bn / 2 : bn; }
 
 }  // namespace u15h
 

@@ -191,9 +191,9 @@ mfma_pinned(typename Mma::acc_t& c, i32x4_t a, i32x4_t b)
 }
 
 // The accumulators of one wave: weight fragments x activation fragments
-// (the wave covers kBN / WN weight rows and 128 activation rows).
-template <class Mma, int WN>
-using acc_array_t = typename Mma::acc_t[kBN / WN / Mma::kF][128 / Mma::kF];
+// (the wave covers BN / WN weight rows and BM / 2 activation rows).
+template <class Mma, int WN, int BM = kBM, int BN = kBN>
+using acc_array_t = typename Mma::acc_t[BN / WN / Mma::kF][BM / 2 / Mma::kF];
 
 // ---- epilogue stores (shared by the GEMM and the split-K reduction) ------
 // Four consecutive output columns n..n+3 of activation row m of problem P.
@@ -286,7 +286,7 @@ find_problem(const GemmBatch& B, int tile)
 // Tile origin (first activation row, first output column) of a tile of P.
 // Grouped raster: bands of 4 row-tiles, walked column by column, so the
 // tiles that run together share activation and weight rows in L2.
-template <Epi E>
+template <Epi E, int BM = kBM, int BN = kBN>
 __device__ __forceinline__ void
 tile_origin(const GemmProblem& P, int tile, int* row0, int* col0)
 {
@@ -297,8 +297,8 @@ tile_origin(const GemmProblem& P, int tile, int* row0, int* col0)
   const int first_m = band * GM;
   const int gm = min(P.tiles_m - first_m, GM);
   const int tin = t - band * per_band;
-  *row0 = (first_m + tin % gm) * kBM;
-  *col0 = (tin / gm) * tile_cols(E);
+  *row0 = (first_m + tin % gm) * BM;
+  *col0 = (tin / gm) * tile_cols(E, BN);
 }
 
 // Which tile and which share of K a workgroup computes.
@@ -315,7 +315,7 @@ struct TileWork {
 
 // Work item w: whole tiles first, then the split tiles, `split`
 // consecutive items per tile, each a contiguous share of the `nk` K stages.
-template <Epi E>
+template <Epi E, int BM = kBM, int BN = kBN>
 __device__ __forceinline__ TileWork
 tile_work(const GemmBatch& B, int nk, int w)
 {
@@ -330,7 +330,7 @@ tile_work(const GemmBatch& B, int nk, int w)
     t.share = (w - SB) % B.split;
   }
   t.prob = find_problem(B, t.tile);
-  tile_origin<E>(B.p[t.prob], t.tile, &t.row0, &t.col0);
+  tile_origin<E, BM, BN>(B.p[t.prob], t.tile, &t.row0, &t.col0);
   t.kbeg = t.is_split ? (t.share * nk) / B.split : 0;
   const int kend = t.is_split ? ((t.share + 1) * nk) / B.split : nk;
   t.nst = kend - t.kbeg;
@@ -421,25 +421,26 @@ lds_barrier()
 // lane 4 consecutive output columns of one row per store, so direct stores
 // write every 128-byte output line in 16-byte pieces from 8 instructions.
 // Instead each wave writes its bf16 results (bias, dequant or SwiGLU
-// applied) into a [256][TC] tile in the two stage buffers (rows 0..127 in
-// ring[0], 128..255 in ring[1]; the main loop is done with them), then the
+// applied) into a [BM][TC] tile in two stage buffers (the upper half's rows
+// in ring[0], the lower's in ring[1]; the main loop is done with them), then the
 // tile is read back row-wise and 32 (or 16) lanes store one row's
 // 512 (256) contiguous bytes.  Row r's 16-byte chunk c sits at chunk
 // c ^ (r % CH) of its staged row, which spreads both the column writes (32
 // rows, one chunk) and the row reads over the bank groups.
-template <class Mma, Epi E, int WN>
+template <class Mma, Epi E, int WN, int BM = kBM, int BN = kBN>
 __device__ __forceinline__ void
 gemm_epilogue_staged(const GemmProblem& P, const TileWork& t, int wm, int wn,
-                     int lane, const acc_array_t<Mma, WN>& acc,
+                     int lane, const acc_array_t<Mma, WN, BM, BN>& acc,
                      char* const (&ring)[2], const float* scl)
 {
-  constexpr int NW = kBN / WN;
+  constexpr int NW = BN / WN;
+  constexpr int HM = BM / 2;                  // activation rows per wave
   constexpr int kF = Mma::kF;
   constexpr int FI = NW / kF;
-  constexpr int FJ = 128 / kF;
+  constexpr int FJ = HM / kF;
   constexpr int kGr = Mma::kE / 4;            // 4-column groups per fragment
   constexpr int kGs = 4 * (64 / kF);          // column stride of the groups
-  constexpr int TC = tile_cols(E);            // output columns per tile
+  constexpr int TC = tile_cols(E, BN);            // output columns per tile
   constexpr int RB = TC * 2;                  // staged bytes per row
   constexpr int CH = RB / 16;                 // 16-byte chunks per row
   const int lr = lane % kF;
@@ -460,7 +461,7 @@ gemm_epilogue_staged(const GemmProblem& P, const TileWork& t, int wm, int wn,
       const int i = c / kGr, g = c % kGr;
       const int n = min(t.col0 + wn * NW + i * kF + g * kGs + lh * 4, P.n - 4);
       if constexpr (kScaled) {
-        swn[c] = *reinterpret_cast<const float4*>(scl + kBM + wn * NW + i * kF + g * kGs +
+        swn[c] = *reinterpret_cast<const float4*>(scl + BM + wn * NW + i * kF + g * kGs +
                                                   lh * 4);
       }
       bia[c] = has_bias ? *reinterpret_cast<const uint2*>(P.bias + n) : uint2{0u, 0u};
@@ -469,7 +470,7 @@ gemm_epilogue_staged(const GemmProblem& P, const TileWork& t, int wm, int wn,
   if constexpr (kScaled) {
 #pragma unroll
     for (int j = 0; j < FJ; ++j) {
-      sam[j] = scl[wm * 128 + j * kF + lr];
+      sam[j] = scl[wm * HM + j * kF + lr];
     }
   }
   // The tile's results in bf16 (bias or SwiGLU applied) are computed
@@ -573,7 +574,7 @@ gemm_epilogue_staged(const GemmProblem& P, const TileWork& t, int wm, int wn,
   __syncthreads();
   // Read back: wave w stores tile rows [RW w, RW w + RW) (RW = 256 / waves);
   // 64 / CH rows per instruction, CH lanes per row.
-  constexpr int RW = kBM / (2 * WN);
+  constexpr int RW = BM / (2 * WN);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   constexpr int kRowsPerRead = 64 / CH;
   // The read-back addresses depend on the lane only; computed from an
@@ -583,7 +584,7 @@ gemm_epilogue_staged(const GemmProblem& P, const TileWork& t, int wm, int wn,
   int lane_o = lane;
   asm volatile("" : "+v"(lane_o));
   const int first = wave * RW;                          // first tile row
-  const char* const src = first >= 128 ? ring[1] : ring[0];
+  const char* const src = first >= HM ? ring[1] : ring[0];
   // Whole 128-byte output lines go out as non-temporal stores, so the
   // output bypasses allocation in L2 instead of evicting the activation and
   // weight rows that the tiles still running on the XCD stream through it.
@@ -593,14 +594,14 @@ gemm_epilogue_staged(const GemmProblem& P, const TileWork& t, int wm, int wn,
   // below kOobOffset).
   const __amdgpu_buffer_rsrc_t yr =
       make_rsrc(static_cast<uint16_t*>(P.y) + (size_t)t.row0 * P.ldy,
-                min(kBM, P.rows - t.row0) * P.ldy * 2);
+                min(BM, P.rows - t.row0) * P.ldy * 2);
   const int c = lane_o % CH;
   const int n = t.col0 + c * 8;
   int voff = n < P.n ? ((first + lane_o / CH) * P.ldy + n) * 2 : kOobOffset;
   const int rstep = kRowsPerRead * P.ldy * 2;
 #pragma unroll
   for (int r = 0; r < RW; r += kRowsPerRead) {
-    const int hrow = first % 128 + r + lane_o / CH;     // row within the half
+    const int hrow = first % HM + r + lane_o / CH;     // row within the half
     const u32x4_t v = *reinterpret_cast<const u32x4_t*>(
         src + hrow * RB + ((c ^ (hrow % CH)) << 4));
     __builtin_amdgcn_raw_buffer_store_b128(v, yr, voff, 0, kNonTemporal);
@@ -612,20 +613,21 @@ gemm_epilogue_staged(const GemmProblem& P, const TileWork& t, int wm, int wn,
 }
 
 // Epilogue of a tile.  acc[i][j][r] holds tile column (weight row within
-// the tile) wn*NW + i*32 + (r>>2)*8 + lh*4 + (r&3) and tile row wm*128 +
+// the tile) wn*NW + i*32 + (r>>2)*8 + lh*4 + (r&3) and tile row wm*BM/2 +
 // j*32 + lr.  A K share writes its raw accumulators to the workspace
-// [kBM][kBN] (rows past the problem are never read back); a whole tile
+// [BM][BN] (rows past the problem are never read back); a whole tile
 // applies the epilogue E.
-template <class Mma, Epi E, int WN>
+template <class Mma, Epi E, int WN, int BM = kBM, int BN = kBN>
 __device__ __forceinline__ void
 gemm_epilogue(const GemmBatch& B, const GemmProblem& P, const TileWork& t,
-              int wm, int wn, int lane, const acc_array_t<Mma, WN>& acc,
+              int wm, int wn, int lane, const acc_array_t<Mma, WN, BM, BN>& acc,
               char* const (&ring)[2], const float* scl)
 {
-  constexpr int NW = kBN / WN;
+  constexpr int NW = BN / WN;
+  constexpr int HM = BM / 2;                  // activation rows per wave
   constexpr int kF = Mma::kF;
   constexpr int FI = NW / kF;
-  constexpr int FJ = 128 / kF;
+  constexpr int FJ = HM / kF;
   constexpr int kGr = Mma::kE / 4;
   constexpr int kGs = 4 * (64 / kF);
   // Lane-derived offsets from an opaque copy of the lane: computed here,
@@ -638,10 +640,10 @@ gemm_epilogue(const GemmBatch& B, const GemmProblem& P, const TileWork& t,
   if (t.is_split) {
     int32_t* wsb = static_cast<int32_t*>(B.ws) +
                    (size_t)((t.tile - B.split_begin) * B.split + t.share) *
-                       (kBM * kBN);
+                       (BM * BN);
 #pragma unroll
     for (int j = 0; j < FJ; ++j) {
-      const int ml = wm * 128 + j * kF + lr;
+      const int ml = wm * HM + j * kF + lr;
       if (t.row0 + ml >= P.rows) { continue; }
 #pragma unroll
       for (int i = 0; i < FI; ++i) {
@@ -649,7 +651,7 @@ gemm_epilogue(const GemmBatch& B, const GemmProblem& P, const TileWork& t,
         for (int g = 0; g < kGr; ++g) {
           const int nl = wn * NW + i * kF + g * kGs + lh * 4;
           const auto& a = acc[i][j];
-          *reinterpret_cast<int4*>(wsb + ml * kBN + nl) = make_int4(
+          *reinterpret_cast<int4*>(wsb + ml * BN + nl) = make_int4(
               bits_as<int>(a[g * 4 + 0]), bits_as<int>(a[g * 4 + 1]),
               bits_as<int>(a[g * 4 + 2]), bits_as<int>(a[g * 4 + 3]));
         }
@@ -658,12 +660,12 @@ gemm_epilogue(const GemmBatch& B, const GemmProblem& P, const TileWork& t,
     return;
   }
   if constexpr (E != Epi::kI32) {
-    gemm_epilogue_staged<Mma, E, WN>(P, t, wm, wn, lane_e, acc, ring, scl);
+    gemm_epilogue_staged<Mma, E, WN, BM, BN>(P, t, wm, wn, lane_e, acc, ring, scl);
     return;
   }
 #pragma unroll
   for (int j = 0; j < FJ; ++j) {
-    const int m = t.row0 + wm * 128 + j * kF + lr;
+    const int m = t.row0 + wm * HM + j * kF + lr;
     if (m >= P.rows) { continue; }
     if constexpr (E == Epi::kSwiglu) {
 #pragma unroll
@@ -1104,6 +1106,211 @@ mot_gemm_kernel(const GemmBatch B)
   }
 }
 
+// The same GEMM on BM x 128 tiles (BM = 128, 192 or 256), for batches whose
+// 256 x 256 tiles are few or mostly padding (129 to ~2000 rows): four waves
+// of BM/2 x 64, one per SIMD, and a ring of RING stages instead of two.  A
+// stage is only BM/128 * 512 MFMA cycles per SIMD, so its loads are issued
+// RING - 1 stages ahead.  The hand-off is gemm_tile's: sub-step 0's MFMAs
+// with sub-step 1's reads between them, the wait and barrier, then sub-step
+// 1's MFMAs with the loads of stage k + RING and the next stage's first reads.
+// Bound: bytes in flight.  A stage takes 0.54 / 0.70 / 0.90 us (BM = 128 /
+// 192 / 256; its MFMAs 0.24 / 0.37 / 0.49 at 2.1 GHz): the RING - 1 stages
+// that LDS holds, over the ~1.6-2 us a load takes with every CU streaming.
+// Weights already in the Infinity Cache save 10-15% at N = 4096 and a third
+// at N = 12288, M = 256 (44 -> 30 us).  One read after each of the first
+// MFMAs instead of reads spread over the sub-step: 1-4% slower.
+// Measured against the 256 x 256 tiles in a graph, weights rotated (us, K =
+// 4096): M = 333, N = 1024 / 4096 / 12288 24.7 / 34.4 / 62.5 -> 17.5 / 28.1 /
+// 50.3; M = 1024, N = 4096 49.5 -> 39.7; M = 2048, N = 4096 72.2 -> 63.1.
+// Loads: the stage's [128 weight | BM activation] rows in blocks of 8 rows
+// (1 KiB, one instruction); wave w takes blocks w, w + 4, ..., so its first
+// four are weights and the rest activations.  SwiGLU: of each wave column's
+// 64 weight rows the first 32 are gate rows, which makes a wave's blocks 0
+// and 2 gate and 1 and 3 up.
+template <class Mma, Epi E, int BM, int RING>
+__device__ __forceinline__ void
+mid_tile(const GemmBatch& B, char* const (&ring)[RING], float* scl, int item)
+{
+  constexpr int BN = kMidBN, KB = kKB, WN = 2;
+  constexpr int kWaves = 4;
+  constexpr int HM = BM / 2, NW = BN / WN;
+  constexpr int FI = NW / Mma::kF, FJ = HM / Mma::kF;
+  constexpr int LB = (BM + BN) / 8 / kWaves;        // loads per wave and stage
+  constexpr int LW = BN / 8 / kWaves;               // the weight loads of them
+  constexpr int kSub = KB / Mma::kKBytes;
+  constexpr int kGroups = 64 / Mma::kF;
+  static_assert(Mma::kF == 16 && kSub == 2 && LW == 4, "16x16 MFMAs, two sub-steps");
+
+  const int kbytes = B.kbytes;
+  const int nk = (kbytes + KB - 1) / KB;
+  const TileWork t = tile_work<E, BM, BN>(B, nk, item);
+  const GemmProblem& P = B.p[t.prob];
+  constexpr int TC = tile_cols(E, BN);
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave / WN;
+  const int wn = wave % WN;
+
+  const int wld = P.wld;
+  const __amdgpu_buffer_rsrc_t ra =
+      make_rsrc(static_cast<const char*>(P.a) + (size_t)t.row0 * kbytes,
+                min(BM, P.rows - t.row0) * kbytes);
+  const int w_bytes = min(TC, P.n - t.col0) * wld;
+  const __amdgpu_buffer_rsrc_t rw =
+      make_rsrc(static_cast<const char*>(P.w) + (size_t)t.col0 * wld, w_bytes);
+  const __amdgpu_buffer_rsrc_t ru =
+      E == Epi::kSwiglu
+          ? make_rsrc(static_cast<const char*>(P.w2) + (size_t)t.col0 * wld, w_bytes)
+          : rw;
+
+  // lane l of a block: row l / 8, landing position l % 8, which holds chunk
+  // (l % 8) ^ key(row); the block's parity is the wave's
+  const int lrow = lane >> 3;
+  const int chunk = (lane & 7) ^ (((8 * (wave & 1) + lrow) >> 1) & 7);
+  const int tail = ((nk - 1) * KB + (chunk << 4) < kbytes) ? 0 : kOobOffset;
+  const int a_off = (8 * wave + lrow) * kbytes + (chunk << 4);
+  const int w_off = (8 * wave + lrow) * wld + (chunk << 4);
+  struct LoadArgs { int ko, va, vw; };
+  auto load_args = [&](int ktl) {
+    const int kt = t.kbeg + ktl;
+    const int oob = (kt == nk - 1 ? tail : 0) + (ktl >= t.nst ? kOobOffset : 0);
+    LoadArgs l;
+    l.ko = __builtin_amdgcn_readfirstlane(min(kt, nk - 1) * KB);
+    l.va = a_off + oob;
+    l.vw = w_off + oob;
+    return l;
+  };
+  auto load_block = [&](const LoadArgs& l, char* stage, int b) {
+    auto* dst = (__attribute__((address_space(3))) void*)(stage + (wave + kWaves * b) * 1024);
+    if (b < LW) {
+      const int row = E == Epi::kSwiglu ? (b >> 1) * 32 : b * 32;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(E == Epi::kSwiglu && (b & 1) ? ru : rw, dst, 16,
+                                               l.vw + row * wld, l.ko, 0, 0);
+    } else {
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, dst, 16, l.va + (b - LW) * 32 * kbytes, l.ko,
+                                               0, 0);
+    }
+  };
+  auto issue_loads = [&](char* stage, int ktl) {
+    const LoadArgs l = load_args(ktl);
+#pragma unroll
+    for (int b = 0; b < LB; ++b) { load_block(l, stage, b); }
+  };
+
+  const int lr = lane % Mma::kF;
+  const int lh = lane / Mma::kF;
+  int rd[kSub];
+#pragma unroll
+  for (int s = 0; s < kSub; ++s) {
+    rd[s] = lr * KB + (((kGroups * s + lh) ^ ((lr >> 1) & 7)) << 4);
+  }
+  const int wbase = wn * NW * KB;
+  const int abase = BN * KB + wm * HM * KB;
+  typename Mma::acc_t acc[FI][FJ];
+#pragma unroll
+  for (int i = 0; i < FI; ++i) {
+#pragma unroll
+    for (int j = 0; j < FJ; ++j) { acc[i][j] = typename Mma::acc_t{}; }
+  }
+  i32x4_t fa[2][FI], fb[2][FJ];
+  auto read_frags = [&](const char* base, int s, int buf) {
+#pragma unroll
+    for (int i = 0; i < FI; ++i) {
+      fa[buf][i] = *reinterpret_cast<const i32x4_t*>(base + wbase + i * 16 * KB + rd[s]);
+    }
+#pragma unroll
+    for (int j = 0; j < FJ; ++j) {
+      fb[buf][j] = *reinterpret_cast<const i32x4_t*>(base + abase + j * 16 * KB + rd[s]);
+    }
+  };
+  auto mma_step = [&](int buf) {
+#pragma unroll
+    for (int i = 0; i < FI; ++i) {
+#pragma unroll
+      for (int j = 0; j < FJ; ++j) {
+        acc[i][j] = Mma::run(fa[buf][i], fb[buf][j], acc[i][j]);
+      }
+    }
+  };
+  // past the last stage the loads fetch nothing and the reads are unused
+  auto stage = [&](char* cur, const char* nxt, int ktl) {
+    read_frags(cur, 1, 1);
+    mma_step(0);
+    interleave_reads<FI * FJ, FI + FJ>();
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((RING - 2) * LB) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    issue_loads(cur, ktl + RING);
+    read_frags(nxt, 0, 0);
+    mma_step(1);
+    interleave_loads_reads<FI * FJ, LB, FI + FJ>();
+  };
+  if constexpr (E == Epi::kDequantBf16) {
+    // the tile's row and column scales, ahead into LDS (as gemm_tile)
+    if (!t.is_split && wave < 2) {
+      const float* src = wave == 0 ? P.sa + t.row0 : P.sw + t.col0;
+      const int n = wave == 0 ? min(BM, P.rows - t.row0) : min(BN, P.n - t.col0);
+      const __amdgpu_buffer_rsrc_t rs = make_rsrc(src, n * 4);
+#pragma unroll
+      for (int i = 0; i < BM / 64; ++i) {
+        if (wave == 0 || i < BN / 64) {
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(
+              rs, (__attribute__((address_space(3))) void*)(scl + wave * BM + i * 64), 4,
+              (i * 64 + lane) * 4, 0, 0, 0);
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < RING; ++r) { issue_loads(ring[r], r); }
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"((RING - 1) * LB) : "memory");
+  lds_barrier();
+  read_frags(ring[0], 0, 0);
+  const int nst_pad = (t.nst + RING - 1) / RING * RING;
+  for (int ktl = 0; ktl < nst_pad; ktl += RING) {
+#pragma unroll
+    for (int r = 0; r < RING; ++r) { stage(ring[r], ring[(r + 1) % RING], ktl + r); }
+  }
+  // no load may still be writing LDS when the epilogue reuses it
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  char* const half[2] = {ring[0], ring[1]};
+  gemm_epilogue<Mma, E, WN, BM, BN>(B, P, t, wm, wn, lane, acc, half, scl);
+}
+
+template <class Mma, Epi E, int BM, int RING>
+__global__ __launch_bounds__(256, 1) void
+mid_gemm_kernel(const GemmBatch B)
+{
+  constexpr int kBytes = (BM + kMidBN) * kKB;
+  __shared__ __attribute__((aligned(1024))) char lds0[kBytes];
+  __shared__ __attribute__((aligned(1024))) char lds1[kBytes];
+  __shared__ __attribute__((aligned(1024))) char lds2[kBytes];
+  __shared__ __attribute__((aligned(1024))) char lds3[RING == 4 ? kBytes : 16];
+  __shared__ __attribute__((aligned(16))) float scl[E == Epi::kDequantBf16 ? BM + kMidBN : 4];
+  const int items = grid_blocks(B);
+  const int G = gridDim.x;
+  const int b = blockIdx.x;
+  for (int base = 0; base < items; base += G) {
+    const int R = min(G, items - base);
+    int w = base + b;
+    if (G % 8 == 0) {
+      const int x = b % 8, i = b / 8;
+      const int lo = x * R / 8, hi = (x + 1) * R / 8;
+      if (i >= hi - lo) { break; }
+      w = base + lo + i;
+    } else if (b >= R) {
+      break;
+    }
+    if constexpr (RING == 4) {
+      char* const ring[4] = {lds0, lds1, lds2, lds3};
+      mid_tile<Mma, E, BM, 4>(B, ring, scl, w);
+    } else {
+      char* const ring[3] = {lds0, lds1, lds2};
+      mid_tile<Mma, E, BM, 3>(B, ring, scl, w);
+    }
+  }
+}
+
 // ---- split-K reduction --------------------------------------------------
 // One workgroup per 8 rows of a split tile: sums the tile's K shares in
 // share order (fp32 adds for bf16 GEMMs, exact int32 adds for int8) and
@@ -1111,32 +1318,34 @@ mot_gemm_kernel(const GemmBatch B)
 // a 16-tile tail's reduction on all CUs: 4.6 us less per config-2 step.
 constexpr int kReduceRowsPerThread = 2;
 
-template <bool kInt, Epi E, int WN>
+template <bool kInt, Epi E, int WN, int BM = kBM, int BN = kBN>
 __global__ __launch_bounds__(256) void
 split_reduce_kernel(const GemmBatch B)
 {
-  constexpr int NW = kBN / WN;
+  constexpr int NW = BN / WN;
+  constexpr int kQuads = BN / 4;             // column quads per row
+  constexpr int kRowStep = 256 / kQuads;     // rows the workgroup covers at once
   constexpr int RPT = kReduceRowsPerThread;
-  constexpr int kRowsPerBlock = 4 * RPT;
-  const int ts = blockIdx.x / (kBM / kRowsPerBlock);
+  constexpr int kRowsPerBlock = kRowStep * RPT;
+  const int ts = blockIdx.x / (BM / kRowsPerBlock);
   const int tile = B.split_begin + ts;
   const GemmProblem& P = B.p[find_problem(B, tile)];
   int row0, col0;
-  tile_origin<E>(P, tile, &row0, &col0);
+  tile_origin<E, BM, BN>(P, tile, &row0, &col0);
   const int32_t* wsb =
-      static_cast<const int32_t*>(B.ws) + (size_t)ts * B.split * (kBM * kBN);
-  // Thread: column quad q of the tile, rows r and r+4 of the block.  The
+      static_cast<const int32_t*>(B.ws) + (size_t)ts * B.split * (BM * BN);
+  // Thread: column quad q of the tile, rows r and r + kRowStep of the block.  The
   // two rows of a share are loaded together (rows past the problem read
   // stale slot values that are never stored), and the share loop is
   // unrolled, so many loads are in flight; each sum still runs in share
   // order.
-  const int q = threadIdx.x & 63;
-  const int block_row = (blockIdx.x % (kBM / kRowsPerBlock)) * kRowsPerBlock;
+  const int q = threadIdx.x % kQuads;
+  const int block_row = (blockIdx.x % (BM / kRowsPerBlock)) * kRowsPerBlock;
   // A block whose rows all lie past the problem (the lower half of a
   // 128-row und tile) has nothing to store; its loads would only cost
   // bandwidth.
   if (row0 + block_row >= P.rows) { return; }
-  const int mlb = block_row + (threadIdx.x >> 6);
+  const int mlb = block_row + threadIdx.x / kQuads;
   const int nl = q * 4;
   constexpr int kCols = E == Epi::kSwiglu ? 2 : 1;   // gate (+ up) columns
   int col[kCols];
@@ -1160,13 +1369,13 @@ split_reduce_kernel(const GemmBatch B)
   }
 #pragma unroll 8
   for (int sh = 0; sh < B.split; ++sh) {
-    const int32_t* base = wsb + (size_t)sh * (kBM * kBN);
+    const int32_t* base = wsb + (size_t)sh * (BM * BN);
     int4 v[kCols][RPT];
 #pragma unroll
     for (int c = 0; c < kCols; ++c) {
 #pragma unroll
       for (int k = 0; k < RPT; ++k) {
-        v[c][k] = *reinterpret_cast<const int4*>(base + (mlb + 4 * k) * kBN + col[c]);
+        v[c][k] = *reinterpret_cast<const int4*>(base + (mlb + kRowStep * k) * BN + col[c]);
       }
     }
 #pragma unroll
@@ -1187,7 +1396,7 @@ split_reduce_kernel(const GemmBatch B)
   }
 #pragma unroll
   for (int k = 0; k < RPT; ++k) {
-    const int m = row0 + mlb + 4 * k;
+    const int m = row0 + mlb + kRowStep * k;
     if (m >= P.rows) { break; }
     if constexpr (E == Epi::kSwiglu) {
       const int n = col0 + (nl / NW) * (NW / 2) + (nl % NW);
@@ -3822,6 +4031,37 @@ launch_gemm(const GemmBatch& b, int cus, hipStream_t s, const GemmEvents& ev)
   return hipGetLastError();
 }
 
+// The BM x 128 tiles (b.bm); persistent as the 256 x 256 ones.
+template <class Mma, Epi E, int BM, int RING>
+hipError_t
+launch_mid(const GemmBatch& b, int cus, hipStream_t s, const GemmEvents& ev)
+{
+  const int items = grid_blocks(b);
+  const int grid = (cus > 0 && cus < items) ? cus : items;
+  launch_timed(mid_gemm_kernel<Mma, E, BM, RING>, dim3(grid), dim3(256), s, ev.before,
+               ev.after, b);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess || b.split_begin >= b.total_tiles) { return e; }
+  constexpr int kRows = 256 / (kMidBN / 4) * kReduceRowsPerThread;
+  launch_timed(split_reduce_kernel<Mma::kInt, E, 2, BM, kMidBN>,
+               dim3((b.total_tiles - b.split_begin) * (BM / kRows)), dim3(256), s,
+               ev.red_before, ev.red_after, b);
+  return hipGetLastError();
+}
+
+template <class Mma, Epi E>
+hipError_t
+launch_mid_bm(const GemmBatch& b, int cus, hipStream_t s, const GemmEvents& ev)
+{
+  if (b.total_tiles <= 0) { return hipSuccess; }
+  switch (b.bm) {
+    case 128: return launch_mid<Mma, E, 128, 4>(b, cus, s, ev);
+    case 192: return launch_mid<Mma, E, 192, 3>(b, cus, s, ev);
+    case 256: return launch_mid<Mma, E, 256, 3>(b, cus, s, ev);
+    default: return hipErrorInvalidValue;
+  }
+}
+
 template <int EL = kElBf16, bool SW = false, class F>
 hipError_t
 launch_skinny(F kernel, const SkinnyBatch& b, hipStream_t s, const GemmEvents& ev,
@@ -3975,6 +4215,7 @@ hipError_t
 launch_gemm_waves(const GemmBatch& b, const GemmShape& g, hipStream_t s,
                   const GemmEvents& ev)
 {
+  if (b.bn == kMidBN) { return launch_mid_bm<typename Mma::x16, E>(b, g.cus, s, ev); }
   // the 4-wave workgroup (one wave per SIMD, 512 registers) runs the 16x16
   // MFMAs; the 8-wave one the 32x32 MFMAs, whose fragments fit 256
   if (g.waves == 4) { return launch_gemm<typename Mma::x16, E, 2>(b, g.cus, s, ev); }
@@ -4406,6 +4647,30 @@ gemm_kernels_loadable()
 
 }  // namespace
 
+namespace {
+
+template <class Mma, Epi E, int BM, int RING>
+bool
+mid_kernel_loadable()
+{
+  hipFuncAttributes a;
+  return hipFuncGetAttributes(&a, reinterpret_cast<const void*>(
+                                      &mid_gemm_kernel<Mma, E, BM, RING>)) == hipSuccess &&
+         hipFuncGetAttributes(&a, reinterpret_cast<const void*>(
+                                      &split_reduce_kernel<Mma::kInt, E, 2, BM, kMidBN>)) ==
+             hipSuccess;
+}
+
+template <class Mma, Epi E>
+bool
+mid_kernels_loadable()
+{
+  return mid_kernel_loadable<Mma, E, 128, 4>() && mid_kernel_loadable<Mma, E, 192, 3>() &&
+         mid_kernel_loadable<Mma, E, 256, 3>();
+}
+
+}  // namespace
+
 bool
 kernels_loadable()
 {
@@ -4564,7 +4829,11 @@ kernels_loadable()
   }
   return gemm_kernels_loadable<MmaBf16x16, MmaI8x16, 2>() &&
          gemm_kernels_loadable<MmaBf16x16, MmaI8x16, 4>() &&
-         gemm_kernels_loadable<MmaBf16, MmaI8, 4>();
+         gemm_kernels_loadable<MmaBf16, MmaI8, 4>() &&
+         mid_kernels_loadable<MmaBf16x16, Epi::kBf16>() &&
+         mid_kernels_loadable<MmaBf16x16, Epi::kSwiglu>() &&
+         mid_kernels_loadable<MmaI8x16, Epi::kI32>() &&
+         mid_kernels_loadable<MmaI8x16, Epi::kDequantBf16>();
 }
 
 }  // namespace u15h
