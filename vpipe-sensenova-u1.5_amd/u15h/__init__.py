@@ -512,14 +512,24 @@ def load_matrix(ops, path, name, K):
     return "affine", (codes, scales, biases, bits, group)
 
 
+# The helpers of every call: a small GEMM takes ~5 us on the GPU, so a call
+# that costs more than that on the host is what a decode loop waits for.
+# Pointers go through ctypes as plain ints (argtypes convert them), and the
+# current stream's handle comes from torch's raw getter, which makes no
+# Stream object.
 def _ptr(t):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
+
+
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
 def _stream(stream):
     if stream is None:
+        if _raw_stream is not None and torch.cuda.is_initialized():
+            return _raw_stream(torch._C._cuda_getDevice())
         stream = torch.cuda.current_stream()
-    return ctypes.c_void_p(stream.cuda_stream)
+    return stream.cuda_stream
 
 
 def _need(t, dtype, shape, name):
@@ -527,11 +537,11 @@ def _need(t, dtype, shape, name):
         raise ValueError(f"{name} is required")
     if t.dtype != dtype:
         raise TypeError(f"{name}: dtype {t.dtype}, expected {dtype}")
-    if tuple(t.shape) != tuple(shape):
+    if t.shape != shape:
         raise ValueError(f"{name}: shape {tuple(t.shape)}, expected {tuple(shape)}")
     if not t.is_contiguous():
         raise ValueError(f"{name} must be contiguous")
-    if t.device.type != "cuda":
+    if not t.is_cuda:
         raise ValueError(f"{name} must be on the GPU")
 
 
