@@ -180,7 +180,9 @@ u15h_status u15h_dequant_affine(u15h_ctx* ctx, u15h_stream stream,
  * grow-only scratch, then u15h_linear's route on the expansion --
  * including its int8 interception when the tier is on and the shape
  * qualifies (the reference's linear_mma_q_ re-enters linear_mma_,
- * src/u15-metal-ops.cc:291-300, 393-399). */
+ * src/u15-metal-ops.cc:291-300, 393-399).  With the default floor, calls of
+ * at most 128 rows that the interception does not take still read the pack
+ * directly (the same results, faster). */
 u15h_status u15h_linear_q(u15h_ctx* ctx, u15h_stream stream,
                           const u15h_bf16* x, const u15h_qweight* w,
                           const u15h_bf16* bias, u15h_bf16* y,

@@ -179,3 +179,32 @@ def test_pack_order_equals_the_expansion(ops, bits, group, M, K, N, shift):
     assert torch.equal(torch.isnan(y), nan) and bool(nan[:, [3, 5]].all())
     assert int(nan.sum()) == 2 * M
     assert torch.equal(y.view(torch.int16)[~nan], y2.view(torch.int16)[~nan])
+
+
+@pytest.mark.parametrize("bits,group", [(8, 64), (4, 32)])
+@pytest.mark.parametrize("M", [96, 97, 128, 129])
+def test_packs_up_to_the_skinny_rows(ops, bits, group, M):
+    """96 to 128 rows read the pack directly with the default floor: bit-equal
+    to u15h_linear on the expansion, as at 129 rows and with the floor set
+    (both expand)."""
+    K, N = 1024, 520
+    rng = np.random.default_rng(M + bits)
+    codes = rng.integers(0, 1 << 32, (N, K * bits // 32), dtype=np.uint64).astype(np.uint32)
+    sc, bi = (dev_bf16(rand_bf16_bits(rng, (N, K // group), 0.01)) for _ in range(2))
+    qw = (torch.from_numpy(codes.view(np.int32)).cuda(), sc, bi, bits, group)
+    x = dev_bf16(rand_bf16_bits(rng, (M, K)))
+    os.environ["U15H_Q_MIN_M"] = "96"
+    try:
+        floor = u15h.Ops(0)
+    finally:
+        del os.environ["U15H_Q_MIN_M"]
+    w = torch.empty(N, K, dtype=torch.bfloat16, device="cuda")
+    ops.dequant_affine(qw, N, K, w)
+    ys = [torch.full((M, N), 7.0, dtype=torch.bfloat16, device="cuda") for _ in range(3)]
+    ops.linear_q(x, qw, None, ys[0], M, K, N)
+    floor.linear_q(x, qw, None, ys[1], M, K, N)
+    ops.linear(x, w, None, ys[2], M, K, N)
+    torch.cuda.synchronize()
+    floor.close()
+    assert torch.equal(ys[0].view(torch.int16), ys[2].view(torch.int16))
+    assert torch.equal(ys[1].view(torch.int16), ys[2].view(torch.int16))

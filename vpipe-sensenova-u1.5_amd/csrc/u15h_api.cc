@@ -33,6 +33,7 @@ struct u15h_ctx {
   // u15h_linear_q below this many rows reads the pack directly (the
   // reference's _mma_q_min_m, u15-metal-ops.h:502; env U15H_Q_MIN_M)
   int q_min_m = 96;
+  bool q_min_m_set = false;  // by the environment
   // GEMM kernel build: 8 or 4 waves per workgroup (env U15H_WAVES) and the
   // 8-wave build's MFMA shape (env U15H_MFMA16).
   u15h::GemmShape gemm = {8, 0, 1};
@@ -664,6 +665,8 @@ u15h_create(int device, u15h_ctx** out)
   ctx->skinny_on = env_int("U15H_SKINNY", 1) != 0;
   ctx->prologue_rpt = env_int("U15H_PROLOGUE_RPT", 2);
   ctx->q_min_m = std::max(0, std::min(u15h::kSkinnyMaxRows + 1, env_int("U15H_Q_MIN_M", 96)));
+  const char* floor = std::getenv("U15H_Q_MIN_M");
+  ctx->q_min_m_set = floor != nullptr && *floor != '\0';
   ctx->gemm.waves = env_int("U15H_WAVES", 8) == 4 ? 4 : 8;
   // env U15H_GEMM_CUS caps the tiled GEMM's persistent grid (a multiple of
   // 8, so each XCD keeps the same share), leaving CUs to work on another
@@ -1265,7 +1268,13 @@ u15h_linear_q(u15h_ctx* ctx, u15h_stream stream, const u15h_bf16* x,
   // steel qmm does (u15-metal-ops.cc:402-431): the skinny kernel
   // dequantises each weight in registers to exactly the expansion's bf16
   // value, so the product equals u15h_linear on the expansion bit for bit.
-  if (M < ctx->q_min_m) {
+  // From the floor to the skinny kernels' 128 rows it is still the faster
+  // way (128 rows, K = 4096, us in a graph, expansion / direct: w8g64 N = 4096
+  // 28.6 / 21.7, N = 12288 73.0 / 53.5; w4g32 N = 6144 34.8 / 32.0), and is
+  // taken where the expansion would go to the bf16 GEMM and the floor is the
+  // default one.
+  const bool int8 = ctx->i8_on && M >= ctx->i8_min_m && K % 128 == 0;
+  if (M < ctx->q_min_m || (!ctx->q_min_m_set && !int8)) {
     GemmBatch b = empty_batch(K * 2);
     add_problem(b, x, w->codes, nullptr, y, bias, nullptr, nullptr, M, N, N,
                 u15h::tile_cols(Epi::kBf16));
@@ -1286,9 +1295,7 @@ u15h_linear_q(u15h_ctx* ctx, u15h_stream stream, const u15h_bf16* x,
   // first step is the int8 interception (u15-metal-ops.cc:291-300,
   // 393-399: a quantized weight arrives there as the _w_deq expansion).
   hipStream_t s = as_stream(stream);
-  if (ctx->i8_on && M >= ctx->i8_min_m && K % 128 == 0) {
-    return linear_i8_route(ctx, s, x, wd, bias, y, M, K, N);
-  }
+  if (int8) { return linear_i8_route(ctx, s, x, wd, bias, y, M, K, N); }
   return dense_bf16(ctx, s, x, wd, bias, y, M, K, N);
 }
 

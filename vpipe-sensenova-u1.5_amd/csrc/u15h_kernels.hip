@@ -2169,14 +2169,15 @@ attention_prologue_kernel(const PrologueArgs a)
 {
   const int D = a.d;
   const int cpr = D >> 3;
-  const int gpb = 256 / cpr;                       // head groups per workgroup
-  const long long nq = (long long)a.tokens * (a.hq / RPT);
-  const long long nk = (long long)a.tokens * (a.hkv / RPT);
-  const long long bq = (nq + gpb - 1) / gpb;
-  const long long bk = (nk + gpb - 1) / gpb;
-  long long blk = blockIdx.x;
+  const uint32_t gpb = 256 / cpr;                  // head groups per workgroup
+  // (tokens x heads is at most 2^30: 32-bit divisions)
+  const uint32_t nq = (uint32_t)a.tokens * (a.hq / RPT);
+  const uint32_t nk = (uint32_t)a.tokens * (a.hkv / RPT);
+  const uint32_t bq = (nq + gpb - 1) / gpb;
+  const uint32_t bk = (nk + gpb - 1) / gpb;
+  uint32_t blk = blockIdx.x;
   int part;                                        // 0 q, 1 k, 2 v
-  long long ngroups;
+  uint32_t ngroups;
   if (blk < bq) {
     part = 0; ngroups = nq;
   } else if (blk < bq + bk) {
@@ -2184,13 +2185,14 @@ attention_prologue_kernel(const PrologueArgs a)
   } else {
     part = 2; ngroups = nk; blk -= bq + bk;
   }
-  const long long grp = blk * gpb + threadIdx.x / cpr;
+  const uint32_t grp = blk * gpb + threadIdx.x / cpr;
   const int c = threadIdx.x % cpr;
   const bool active = grp < ngroups;
-  const long long gg = active ? grp : 0;
+  const uint32_t gg = active ? grp : 0;
   const int H = part == 0 ? a.hq : a.hkv;
-  const long long t = gg / (H / RPT);
-  const int h0 = (int)(gg % (H / RPT)) * RPT;
+  const uint32_t t32 = gg / (uint32_t)(H / RPT);
+  const long long t = t32;
+  const int h0 = (int)(gg - t32 * (uint32_t)(H / RPT)) * RPT;
   const uint16_t* src = (part == 0 ? a.q : (part == 1 ? a.k : a.v)) +
                         (t * H + h0) * D + c * 8;
   i32x4_t raw[RPT];
@@ -3960,11 +3962,13 @@ skinny_reduce_kernel(const SkinnyBatch B)
   constexpr int CW = SW ? 2 : 1;
   using acc_t = sk_acc_t<EL>;
   const SkinnyProblem& P = B.p[blockIdx.y];
-  const int q = P.n / 4;
-  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (idx >= (int64_t)P.rows * q) { return; }
+  // 32-bit: at most 128 rows of 2^18 column quads (a 64-bit division is a
+  // long chain in a kernel that is little else)
+  const uint32_t q = (uint32_t)P.n / 4;
+  const uint32_t idx = blockIdx.x * 256 + threadIdx.x;
+  if (idx >= (uint32_t)P.rows * q) { return; }
   const int m = (int)(idx / q);
-  const int n = (int)(idx - (int64_t)m * q) * 4;
+  const int n = (int)(idx - (uint32_t)m * q) * 4;
   const size_t plane = (size_t)P.rows * P.n;
   const float* ws = B.ws + P.ws_off + (size_t)m * P.n + n;
   const SkEpi<EL> epi = skinny_epi<EL, SW>(P, n);
@@ -3972,7 +3976,8 @@ skinny_reduce_kernel(const SkinnyBatch B)
 #pragma unroll
   for (int c = 0; c < CW; ++c) {
     v[c] = *reinterpret_cast<const acc_t*>(ws + c * B.split * plane);
-    for (int sh = 1; sh < B.split; ++sh) {
+#pragma unroll 3
+    for (int sh = 1; sh < B.split; ++sh) {        // (1, 3, 7 or 15 more)
       v[c] += *reinterpret_cast<const acc_t*>(ws + (c * B.split + sh) * plane);
     }
   }
