@@ -240,11 +240,10 @@ tiles_estimate(const u15h_ctx* ctx, const GemmBatch& b, double stage)
 // mid-size kernel's where their estimate is at least 5% lower.  Stage times
 // as measured: the 256 x 256 kernel's by the share of CUs it keeps busy (1.22
 // us at 144, 1.34 at 192, 1.5 at 256), the mid-size ones' growing with K
-// (128 rows: 0.54 us at 64 stages, 0.58 at 192) and 10% longer for int8.
-// Estimated / measured, us: M = 333, K
-// = 12288, N = 4096: 256 x 256 57.5 / 55.8, 192 48.6 / 51.2, 128 63.7 / 63.9;
-// M = 1024, K = 4096, N = 12288: 256 x 256 91 / 91.2, 256 110 / 111.9; M =
-// 512, K = 4096, N = 12288: 256 x 256 66.5 / 67.9, 256 62.6 / 61.4.  The
+// (128 rows: 0.53 us at 64 stages, 0.57 at 192) and 10% longer for int8.
+// Estimated / measured, us: M = 333, K = 12288, N = 4096: 256 x 256 57.5 /
+// 55.9, 192 48.8 / 49.3; M = 512, K = 4096, N = 12288: 256 x 256 66.5 / 67.5,
+// 256 57.2 / 56.5; M = 1024, K = 4096, N = 12288: 256 x 256 91 / 87.4.  The
 // 256 x 256 tiles' other builds (U15H_WAVES, U15H_MFMA16) have no mid-size
 // form and keep their tiles.
 void
@@ -256,7 +255,7 @@ pick_tiles(const u15h_ctx* ctx, GemmBatch& b, Epi epi)
   const int busy = T >= C ? C : T * tail_shares(ctx, T, nk);
   double best = 0.95 * tiles_estimate(ctx, b, 0.85 + 0.65 * busy / C);
   int bm = 0;
-  const struct { int bm; double stage; } mid[] = {{128, 0.525}, {192, 0.68}, {256, 0.875}};
+  const struct { int bm; double stage; } mid[] = {{128, 0.515}, {192, 0.64}, {256, 0.79}};
   const double longer = (1.0 + nk / 1920.0) *
                         (epi == Epi::kI32 || epi == Epi::kDequantBf16 ? 1.1 : 1.0);
   for (const auto& m : mid) {

@@ -16,6 +16,7 @@ namespace u15h {
 constexpr int kBM = 256;          // activation rows per tile
 constexpr int kBN = 256;          // weight rows (output columns) per tile
 constexpr int kMidBN = 128;       // weight rows per tile of the mid-size kernels
+constexpr int kMidWN = 4;         // their waves along N (two along M)
 constexpr int kKB = 128;          // bytes of K per stage
 constexpr int kMaxProb = 8;       // problems (weight sets x projections) per launch
 

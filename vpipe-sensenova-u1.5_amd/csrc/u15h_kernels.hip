@@ -1107,39 +1107,41 @@ mot_gemm_kernel(const GemmBatch B)
 }
 
 // The same GEMM on BM x 128 tiles (BM = 128, 192 or 256), for batches whose
-// 256 x 256 tiles are few or mostly padding (129 to ~2000 rows): four waves
-// of BM/2 x 64, one per SIMD, and a ring of RING stages instead of two.  A
+// 256 x 256 tiles are few or mostly padding (129 to ~2000 rows): eight waves
+// of BM/2 x 32, two per SIMD, and a ring of RING stages instead of two.  A
 // stage is only BM/128 * 512 MFMA cycles per SIMD, so its loads are issued
 // RING - 1 stages ahead.  The hand-off is gemm_tile's: sub-step 0's MFMAs
 // with sub-step 1's reads between them, the wait and barrier, then sub-step
 // 1's MFMAs with the loads of stage k + RING and the next stage's first reads.
-// Bound: bytes in flight.  A stage takes 0.54 / 0.70 / 0.90 us (BM = 128 /
-// 192 / 256; its MFMAs 0.24 / 0.37 / 0.49 at 2.1 GHz): the RING - 1 stages
-// that LDS holds, over the ~1.6-2 us a load takes with every CU streaming.
-// Weights already in the Infinity Cache save 10-15% at N = 4096 and a third
-// at N = 12288, M = 256 (44 -> 30 us).  One read after each of the first
-// MFMAs instead of reads spread over the sub-step: 1-4% slower.
+// Bound: LDS and the bytes in flight.  A stage takes 0.53 / 0.66 / 0.82 us
+// (BM = 128 / 192 / 256; its MFMAs 0.24 / 0.37 / 0.49 at 2.1 GHz).  Timed
+// without its loads the 128-row tile still took 0.41 us with four waves of
+// BM/2 x 64, whose fragment reads see LDS at ~118 bytes a clock (latency);
+// eight waves (~238) made the 192- and 256-row tiles 7 and 10% faster, the
+// 128-row one 2%.  The rest is the RING - 1 stages that LDS holds over the
+// ~1.6-2 us a load takes with every CU streaming: weights already in the
+// Infinity Cache save 10-15% at N = 4096, a third at N = 12288, M = 256.
 // Measured against the 256 x 256 tiles in a graph, weights rotated (us, K =
-// 4096): M = 333, N = 1024 / 4096 / 12288 24.7 / 34.4 / 62.5 -> 17.5 / 28.1 /
-// 50.3; M = 1024, N = 4096 49.5 -> 39.7; M = 2048, N = 4096 72.2 -> 63.1.
+// 4096): M = 333, N = 1024 / 4096 / 12288 24.6 / 34.8 / 62.0 -> 17.6 / 26.7 /
+// 47.2; M = 1024, N = 4096 49.3 -> 36.7; M = 2048, N = 4096 71.4 -> 56.9;
+// int8 M = 1024, N = 4096 38.8 -> 18.7.
 // Loads: the stage's [128 weight | BM activation] rows in blocks of 8 rows
-// (1 KiB, one instruction); wave w takes blocks w, w + 4, ..., so its first
-// four are weights and the rest activations.  SwiGLU: of each wave column's
-// 64 weight rows the first 32 are gate rows, which makes a wave's blocks 0
-// and 2 gate and 1 and 3 up.
+// (1 KiB, one instruction); wave w takes blocks w, w + 8, ..., so its first
+// two are weights and the rest activations.
 template <class Mma, Epi E, int BM, int RING>
 __device__ __forceinline__ void
 mid_tile(const GemmBatch& B, char* const (&ring)[RING], float* scl, int item)
 {
-  constexpr int BN = kMidBN, KB = kKB, WN = 2;
-  constexpr int kWaves = 4;
+  constexpr int BN = kMidBN, KB = kKB, WN = kMidWN;
+  constexpr int kWaves = 2 * WN;
   constexpr int HM = BM / 2, NW = BN / WN;
   constexpr int FI = NW / Mma::kF, FJ = HM / Mma::kF;
   constexpr int LB = (BM + BN) / 8 / kWaves;        // loads per wave and stage
   constexpr int LW = BN / 8 / kWaves;               // the weight loads of them
   constexpr int kSub = KB / Mma::kKBytes;
   constexpr int kGroups = 64 / Mma::kF;
-  static_assert(Mma::kF == 16 && kSub == 2 && LW == 4, "16x16 MFMAs, two sub-steps");
+  static_assert(Mma::kF == 16 && kSub == 2 && LW == 2 && (BM + BN) % 64 == 0,
+                "16x16 MFMAs, two sub-steps, eight waves");
 
   const int kbytes = B.kbytes;
   const int nk = (kbytes + KB - 1) / KB;
@@ -1156,12 +1158,9 @@ mid_tile(const GemmBatch& B, char* const (&ring)[RING], float* scl, int item)
       make_rsrc(static_cast<const char*>(P.a) + (size_t)t.row0 * kbytes,
                 min(BM, P.rows - t.row0) * kbytes);
   const int w_bytes = min(TC, P.n - t.col0) * wld;
+  const bool up = E == Epi::kSwiglu && (wave & 2);  // this wave loads up rows
   const __amdgpu_buffer_rsrc_t rw =
-      make_rsrc(static_cast<const char*>(P.w) + (size_t)t.col0 * wld, w_bytes);
-  const __amdgpu_buffer_rsrc_t ru =
-      E == Epi::kSwiglu
-          ? make_rsrc(static_cast<const char*>(P.w2) + (size_t)t.col0 * wld, w_bytes)
-          : rw;
+      make_rsrc(static_cast<const char*>(up ? P.w2 : P.w) + (size_t)t.col0 * wld, w_bytes);
 
   // lane l of a block: row l / 8, landing position l % 8, which holds chunk
   // (l % 8) ^ key(row); the block's parity is the wave's
@@ -1169,7 +1168,9 @@ mid_tile(const GemmBatch& B, char* const (&ring)[RING], float* scl, int item)
   const int chunk = (lane & 7) ^ (((8 * (wave & 1) + lrow) >> 1) & 7);
   const int tail = ((nk - 1) * KB + (chunk << 4) < kbytes) ? 0 : kOobOffset;
   const int a_off = (8 * wave + lrow) * kbytes + (chunk << 4);
-  const int w_off = (8 * wave + lrow) * wld + (chunk << 4);
+  // SwiGLU: each wave column's 32 weight rows are 16 gate, then their 16 up
+  const int wrow = E == Epi::kSwiglu ? (wave >> 2) * 16 + 8 * (wave & 1) : 8 * wave;
+  const int w_off = (wrow + lrow) * wld + (chunk << 4);
   struct LoadArgs { int ko, va, vw; };
   auto load_args = [&](int ktl) {
     const int kt = t.kbeg + ktl;
@@ -1183,11 +1184,10 @@ mid_tile(const GemmBatch& B, char* const (&ring)[RING], float* scl, int item)
   auto load_block = [&](const LoadArgs& l, char* stage, int b) {
     auto* dst = (__attribute__((address_space(3))) void*)(stage + (wave + kWaves * b) * 1024);
     if (b < LW) {
-      const int row = E == Epi::kSwiglu ? (b >> 1) * 32 : b * 32;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(E == Epi::kSwiglu && (b & 1) ? ru : rw, dst, 16,
-                                               l.vw + row * wld, l.ko, 0, 0);
+      const int row = b * (E == Epi::kSwiglu ? 32 : 64);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, dst, 16, l.vw + row * wld, l.ko, 0, 0);
     } else {
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, dst, 16, l.va + (b - LW) * 32 * kbytes, l.ko,
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, dst, 16, l.va + (b - LW) * 64 * kbytes, l.ko,
                                                0, 0);
     }
   };
@@ -1278,7 +1278,7 @@ mid_tile(const GemmBatch& B, char* const (&ring)[RING], float* scl, int item)
 }
 
 template <class Mma, Epi E, int BM, int RING>
-__global__ __launch_bounds__(256, 1) void
+__global__ __launch_bounds__(128 * kMidWN, 1) void
 mid_gemm_kernel(const GemmBatch B)
 {
   constexpr int kBytes = (BM + kMidBN) * kKB;
@@ -4043,12 +4043,12 @@ launch_mid(const GemmBatch& b, int cus, hipStream_t s, const GemmEvents& ev)
 {
   const int items = grid_blocks(b);
   const int grid = (cus > 0 && cus < items) ? cus : items;
-  launch_timed(mid_gemm_kernel<Mma, E, BM, RING>, dim3(grid), dim3(256), s, ev.before,
+  launch_timed(mid_gemm_kernel<Mma, E, BM, RING>, dim3(grid), dim3(128 * kMidWN), s, ev.before,
                ev.after, b);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || b.split_begin >= b.total_tiles) { return e; }
   constexpr int kRows = 256 / (kMidBN / 4) * kReduceRowsPerThread;
-  launch_timed(split_reduce_kernel<Mma::kInt, E, 2, BM, kMidBN>,
+  launch_timed(split_reduce_kernel<Mma::kInt, E, kMidWN, BM, kMidBN>,
                dim3((b.total_tiles - b.split_begin) * (BM / kRows)), dim3(256), s,
                ev.red_before, ev.red_after, b);
   return hipGetLastError();
@@ -4662,7 +4662,7 @@ mid_kernel_loadable()
   return hipFuncGetAttributes(&a, reinterpret_cast<const void*>(
                                       &mid_gemm_kernel<Mma, E, BM, RING>)) == hipSuccess &&
          hipFuncGetAttributes(&a, reinterpret_cast<const void*>(
-                                      &split_reduce_kernel<Mma::kInt, E, 2, BM, kMidBN>)) ==
+                                      &split_reduce_kernel<Mma::kInt, E, kMidWN, BM, kMidBN>)) ==
              hipSuccess;
 }
 
