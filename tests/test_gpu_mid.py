@@ -95,3 +95,37 @@ def test_planned_tiles(ops, contexts, M, K, N):
     ref = oracle.linear_bf16(xb, wb, bb, row_ids=rows)
     a = host_f32(y)[rows]
     assert max_rel(a, ref) <= 1e-2 and rel_l2(a, ref) < 4e-3
+
+
+@pytest.mark.parametrize("Mu,Mg,K,N", [(128, 4096, 256, 4096), (1, 2048, 192, 8192),
+                                       (50, 4096, 320, 4096)])
+def test_few_rows_apart_from_whole_rounds(ops, contexts, Mu, Mg, K, N):
+    """A group of at most 128 rows beside one whose 256 x 256 tiles fill whole
+    rounds of 256 CUs runs in a launch of its own: equal bits on exact sums
+    to the one grouped launch, for every epilogue, and in the
+    allocation-free call."""
+    rng = np.random.default_rng(Mu + Mg + K)
+    M = Mu + Mg
+    x = ints(rng, (M, K), 2)
+    w = [ints(rng, (N, K), 1) for _ in range(4)]
+    b = [ints(rng, (N,), 3) for _ in range(2)]
+
+    def run(o, call):
+        y = torch.full((M, N), 7, dtype=torch.bfloat16, device="cuda")
+        if call == "swiglu":
+            o.mot_gate_up_swiglu(x, Mu, Mg, K, *w, y)
+        else:
+            o.mot_linear(x, Mu, Mg, K, [dict(w_und=w[0], w_gen=w[1], bias_und=b[0],
+                                             bias_gen=b[1], y=y)], noalloc=call == "noalloc")
+        torch.cuda.synchronize()
+        return y.view(torch.int16)
+    for call in ("linear", "noalloc", "swiglu"):
+        assert torch.equal(run(ops, call), run(contexts[0], call))
+    if K % 128 == 0:
+        xq, q0, q1 = (torch.from_numpy(rng.integers(-127, 128, s).astype(np.int8)).cuda()
+                      for s in ((M, K), (N, K), (N, K)))
+        ys = [torch.empty(M, N, dtype=torch.int32, device="cuda") for _ in range(2)]
+        for o, y in zip((ops, contexts[0]), ys):
+            o.mot_gemm_i8_i32(xq, Mu, Mg, K, [dict(wq_und=q0, wq_gen=q1, y=y)])
+        torch.cuda.synchronize()
+        assert torch.equal(*ys)
