@@ -129,3 +129,26 @@ def test_few_rows_apart_from_whole_rounds(ops, contexts, Mu, Mg, K, N):
             o.mot_gemm_i8_i32(xq, Mu, Mg, K, [dict(wq_und=q0, wq_gen=q1, y=y)])
         torch.cuda.synchronize()
         assert torch.equal(*ys)
+
+
+@pytest.mark.parametrize("bm", [128, 192, 256, None])
+@pytest.mark.parametrize("M,K,N", [(129, 64, 8), (191, 320, 1000), (256, 2048, 520),
+                                   (257, 192, 136), (384, 4096, 264), (385, 448, 128)])
+@pytest.mark.parametrize("bits,group", [(4, 32), (4, 64), (8, 32), (8, 64)])
+def test_packs_on_the_mid_tiles(ops, contexts, bits, group, M, K, N, bm):
+    """Packs of more than 128 rows, read by the tiles (to 256 rows at 4 bits,
+    384 at 8) or expanded, with bias: bit-equal to u15h_linear on the
+    expansion, at tile edges, one K stage, odd stage counts and splits."""
+    rng = np.random.default_rng(M + K + bits + group)
+    codes = rng.integers(0, 1 << 32, (N, K * bits // 32), dtype=np.uint64).astype(np.uint32)
+    sc, bi = (dev_bf16(rand_bf16_bits(rng, (N, K // group), 0.01)) for _ in range(2))
+    qw = (torch.from_numpy(codes.view(np.int32)).cuda(), sc, bi, bits, group)
+    x, b = dev_bf16(rand_bf16_bits(rng, (M, K))), dev_bf16(rand_bf16_bits(rng, (N,), 0.5))
+    w = torch.empty(N, K, dtype=torch.bfloat16, device="cuda")
+    o = ops if bm is None else contexts[bm]
+    o.dequant_affine(qw, N, K, w)
+    y, t = (torch.full((M, N), 7.0, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    o.linear_q(x, qw, b, y, M, K, N)
+    o.linear(x, w, b, t, M, K, N)
+    torch.cuda.synchronize()
+    assert torch.equal(y.view(torch.int16), t.view(torch.int16))

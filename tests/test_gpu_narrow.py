@@ -186,7 +186,7 @@ def test_pack_order_equals_the_expansion(ops, bits, group, M, K, N, shift):
 def test_packs_up_to_the_skinny_rows(ops, bits, group, M):
     """96 to 128 rows read the pack directly with the default floor: bit-equal
     to u15h_linear on the expansion, as at 129 rows and with the floor set
-    (both expand)."""
+    (which expands)."""
     K, N = 1024, 520
     rng = np.random.default_rng(M + bits)
     codes = rng.integers(0, 1 << 32, (N, K * bits // 32), dtype=np.uint64).astype(np.uint32)

@@ -1279,6 +1279,31 @@ u15h_dequant_affine(u15h_ctx* ctx, u15h_stream stream, const u15h_qweight* w,
                   "dequant_affine");
 }
 
+// Plans the mid-size tiles' direct read of a pack into `b` where they are
+// the product's tiles anyway and that beats the expansion: to 384 rows at 8
+// bits, 256 at 4.  Every row tile dequantises the weights again, and the
+// expansion costs 17 us for 16 million of them.  Expansion / direct, us in a
+// graph, K = 4096 (N = 4096 | 6144 | 12288) and K = 12288 (N = 4096): w8g64
+// 129 rows 34.3/24.8 | 46.2/31.8 | 75.2/49.5 and 74.1/42.0; 300 rows 40.6/31.7
+// | 53.1/48.9 | 79.5/71.7 and 86.4/68.0; 384 rows 45.0/32.9 | 54.4/50.7 |
+// 82.5/74.5 and 93.6/70.6; 512 rows 42.4/40.2 | 53.1/61.5 | 91.8/82.4 and
+// 102/81.  w4g32 256 rows 37.0/28.1 | 47.2/37.3 | 60.0/57.3 and 77.1/50.1;
+// 384 rows 39.9/33.8 | 46.4/47.7 | 71.7/70.7 and 81.7/68.6.
+static bool
+plan_pack(const u15h_ctx* ctx, const u15h_qweight* w, int M, int K, GemmBatch& b)
+{
+  const uintptr_t at = reinterpret_cast<uintptr_t>(w->scales) |
+                       reinterpret_cast<uintptr_t>(w->biases);
+  if (ctx->q_min_m_set || K % 64 != 0 || at % 2 != 0 || M > (w->bits == 8 ? 384 : 256) ||
+      skinny_fits(ctx, b, Epi::kBf16)) {
+    return false;
+  }
+  pick_tiles(ctx, b, Epi::kBf16);
+  b.p[0].qs = w->scales;
+  b.p[0].qb = w->biases;
+  return b.bn == u15h::kMidBN;
+}
+
 u15h_status
 u15h_linear_q(u15h_ctx* ctx, u15h_stream stream, const u15h_bf16* x,
               const u15h_qweight* w, const u15h_bf16* bias, u15h_bf16* y,
@@ -1313,6 +1338,18 @@ u15h_linear_q(u15h_ctx* ctx, u15h_stream stream, const u15h_bf16* x,
     if (skinny_fits(ctx, b, Epi::kBf16)) {
       return skinny_launch(ctx, b, Epi::kBf16, as_stream(stream), false,
                            take_profile_event(ctx), w);
+    }
+  }
+  if (!int8) {
+    GemmBatch b = empty_batch(K * 2);
+    add_problem(b, x, w->codes, nullptr, y, bias, nullptr, nullptr, M, N, N,
+                u15h::tile_cols(Epi::kBf16));
+    if (plan_pack(ctx, w, M, K, b)) {
+      if ((st = plan_split(ctx, b, Epi::kBf16)) != U15H_OK) { return st; }
+      return launched(ctx,
+                      u15h::launch_gemm_pack(b, w->bits, w->group, ctx->gemm,
+                                             as_stream(stream), take_profile_event(ctx)),
+                      "gemm_pack");
     }
   }
   if ((st = ensure_deq_scratch(ctx, stream, (size_t)N * K * 2)) != U15H_OK) {

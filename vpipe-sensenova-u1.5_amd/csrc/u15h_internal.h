@@ -37,6 +37,8 @@ struct GemmProblem {
   const uint16_t* bias;   // bf16 [n] or null
   const float*    sa;     // per-row scale [rows] (kDequantBf16)
   const float*    sw;     // per-column scale [n] (kDequantBf16)
+  const uint16_t* qs;     // affine pack (w its codes): scales, biases
+  const uint16_t* qb;     //   bf16 [n][K / group]
   int rows;               // activation rows of this problem
   int n;                  // output columns of this problem
   int wld;                // bytes between consecutive weight rows
@@ -98,6 +100,10 @@ struct GemmEvents {
   hipEvent_t red_after = nullptr;     // its end
 };
 hipError_t launch_gemm_bf16(const GemmBatch& b, Epi epi, const GemmShape& g,
+                            hipStream_t s, const GemmEvents& ev);
+// One problem whose weight is an affine pack, on the mid-size tiles (b.bn ==
+// kMidBN): K % 64 == 0, at group 32 scales and biases 4-byte aligned.
+hipError_t launch_gemm_pack(const GemmBatch& b, int bits, int group, const GemmShape& g,
                             hipStream_t s, const GemmEvents& ev);
 
 // The skinny bf16 GEMM for problems of at most kSkinnyMaxRows rows: one

@@ -1277,6 +1277,220 @@ mid_tile(const GemmBatch& B, char* const (&ring)[RING], float* scl, int item)
   gemm_epilogue<Mma, E, WN, BM, BN>(B, P, t, wm, wn, lane, acc, half, scl);
 }
 
+// mid_tile on an affine pack (QB bits, groups of GRP).  Each wave
+// dequantises 16 of the 128 weight rows' K-block, as the expansion does (a
+// multiply, then an add, then bf16), one stage ahead into one of two LDS
+// buffers laid out as mid_tile's weights; tiles, K order and sums are the
+// dense kernel's, so the result equals it on the expansion bit for bit.  A
+// lane holds 16 codes of one row and their scale and bias, loaded RING
+// stages ahead into registers.  What it saves is the expansion: its launch and
+// 2 x 2 bytes a weight through memory.  300 rows, K = N = 4096, w8g64: 40.6 us
+// expanded, 31.7 here (the dense product alone 24).  The codes copied to LDS
+// and every wave dequantising its own fragments (each weight once per row half
+// and tile) was bound by that: 38.8.
+template <int BM, int RING, int QB, int GRP>
+__device__ __forceinline__ void
+mid_pack_tile(const GemmBatch& B, char* const (&ring)[RING], char* const (&wbuf)[2], int item)
+{
+  using Mma = MmaBf16x16;
+  constexpr Epi E = Epi::kBf16;
+  constexpr int BN = kMidBN, KB = kKB, WN = kMidWN;
+  constexpr int kWaves = 2 * WN;
+  constexpr int HM = BM / 2, NW = BN / WN;
+  constexpr int FI = NW / Mma::kF, FJ = HM / Mma::kF;
+  constexpr int LA = BM / 8 / kWaves;               // activation copies per wave
+  constexpr int LB = LA + 3;                        // loads per wave and stage
+  constexpr int kSub = KB / Mma::kKBytes;
+  constexpr int kGroups = 64 / Mma::kF;
+  const int kbytes = B.kbytes;
+  const int nk = (kbytes + KB - 1) / KB;
+  const TileWork t = tile_work<E, BM, BN>(B, nk, item);
+  const GemmProblem& P = B.p[t.prob];
+  constexpr int TC = tile_cols(E, BN);
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave / WN;
+  const int wn = wave % WN;
+
+  const __amdgpu_buffer_rsrc_t ra =
+      make_rsrc(static_cast<const char*>(P.a) + (size_t)t.row0 * kbytes,
+                min(BM, P.rows - t.row0) * kbytes);
+  // codes, scales and biases of the tile's rows (rows past n read zero)
+  const int nrow = min(TC, P.n - t.col0);
+  const int cpitch = kbytes / 2 * QB / 8;
+  const int spitch = kbytes / 2 / GRP * 2;
+  const __amdgpu_buffer_rsrc_t rw =
+      make_rsrc(static_cast<const char*>(P.w) + (size_t)t.col0 * cpitch, nrow * cpitch);
+  const __amdgpu_buffer_rsrc_t rs = make_rsrc(
+      reinterpret_cast<const char*>(P.qs) + (size_t)t.col0 * spitch, nrow * spitch);
+  const __amdgpu_buffer_rsrc_t rb = make_rsrc(
+      reinterpret_cast<const char*>(P.qb) + (size_t)t.col0 * spitch, nrow * spitch);
+
+  // lane l of a block: row l / 8, landing position l % 8, which holds chunk
+  // (l % 8) ^ key(row); the block's parity is the wave's
+  const int lrow = lane >> 3;
+  const int chunk = (lane & 7) ^ (((8 * (wave & 1) + lrow) >> 1) & 7);
+  const int a_off = (8 * wave + lrow) * kbytes + (chunk << 4);
+  // codes: lane l holds 16 of row 16 wave + l / 4
+  const int crow = wave * 16 + (lane >> 2), cq = lane & 3;
+  const int c_off = crow * cpitch + cq * 2 * QB;
+  const int s_off = crow * spitch + cq * 16 / GRP * 2;
+  const int lr = lane % Mma::kF;
+  const int lh = lane / Mma::kF;
+  // (fixed sizes: a lambda capturing an array of template-dependent size
+  // loses the kernel's host-side launch stub)
+  uint32_t sreg[4], breg[4];
+  u32x4_t creg[4];
+  auto issue_loads = [&](char* stage, int slot, int ktl) {
+    const int kt = min(t.kbeg + ktl, nk - 1);
+    const int oob = ktl >= t.nst ? kOobOffset : 0;
+    const int so = __builtin_amdgcn_readfirstlane(kt * (64 / GRP) * 2);
+    const int co = __builtin_amdgcn_readfirstlane(kt * 8 * QB);
+    const int ko = __builtin_amdgcn_readfirstlane(kt * KB);
+    if constexpr (QB == 8) {
+      creg[slot] = __builtin_amdgcn_raw_buffer_load_b128(rw, c_off + oob, co, 0);
+    } else {
+      const u32x2_t c = __builtin_amdgcn_raw_buffer_load_b64(rw, c_off + oob, co, 0);
+      creg[slot] = u32x4_t{c[0], c[1], 0, 0};
+    }
+    sreg[slot] = __builtin_amdgcn_raw_buffer_load_b16(rs, s_off + oob, so, 0);
+    breg[slot] = __builtin_amdgcn_raw_buffer_load_b16(rb, s_off + oob, so, 0);
+#pragma unroll
+    for (int b = 0; b < LA; ++b) {
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          ra, (__attribute__((address_space(3))) void*)(stage + (wave + kWaves * b) * 1024), 16,
+          a_off + b * 64 * kbytes + oob, ko, 0, 0);
+    }
+  };
+
+  int rd[kSub];
+#pragma unroll
+  for (int s = 0; s < kSub; ++s) {
+    rd[s] = lr * KB + (((kGroups * s + lh) ^ ((lr >> 1) & 7)) << 4);
+  }
+  const int abase = wm * HM * KB;
+  const int wbase = wn * NW * KB;
+  typename Mma::acc_t acc[FI][FJ];
+#pragma unroll
+  for (int i = 0; i < FI; ++i) {
+#pragma unroll
+    for (int j = 0; j < FJ; ++j) { acc[i][j] = typename Mma::acc_t{}; }
+  }
+  i32x4_t fa[2][FI], fb[2][FJ];
+  auto read_frags = [&](const char* base, const char* wb, int s, int buf) {
+#pragma unroll
+    for (int i = 0; i < FI; ++i) {
+      fa[buf][i] = *reinterpret_cast<const i32x4_t*>(wb + wbase + i * 16 * KB + rd[s]);
+    }
+#pragma unroll
+    for (int j = 0; j < FJ; ++j) {
+      fb[buf][j] = *reinterpret_cast<const i32x4_t*>(base + abase + j * 16 * KB + rd[s]);
+    }
+  };
+  // the codes of a slot, dequantised into chunks 2 cq and 2 cq + 1 of the row
+  auto dequant = [&](int slot, char* wb) {
+    // opaque here, so that nothing of the conversion moves up to where it
+    // would wait for the loads just issued
+    uint32_t sb = sreg[slot], bb = breg[slot];
+    u32x4_t cc = creg[slot];
+    asm volatile("" : "+v"(sb), "+v"(bb), "+v"(cc));
+    const float sc = __uint_as_float(sb << 16);
+    const float bi = __uint_as_float(bb << 16);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      u32x4_t o;
+#pragma unroll
+      for (int e = 0; e < 8; e += 2) {
+        const uint32_t c = QB == 8 ? cc[2 * h + (e >> 2)] : cc[h];
+        const int at = QB == 8 ? (e & 3) * 8 : e * 4;
+        float p0 = sc * (float)((c >> at) & ((1u << QB) - 1));
+        float p1 = sc * (float)((c >> (at + QB)) & ((1u << QB) - 1));
+        asm("" : "+v"(p0), "+v"(p1));   // the products stay rounded: no fma
+        o[e >> 1] = pack_bf16x2(p0 + bi, p1 + bi);
+      }
+      *reinterpret_cast<u32x4_t*>(wb + crow * KB +
+                                  (((2 * cq + h) ^ ((crow >> 1) & 7)) << 4)) = o;
+    }
+  };
+  auto mma_step = [&](int buf) {
+#pragma unroll
+    for (int i = 0; i < FI; ++i) {
+#pragma unroll
+      for (int j = 0; j < FJ; ++j) {
+        acc[i][j] = Mma::run(fa[buf][i], fb[buf][j], acc[i][j]);
+      }
+    }
+  };
+  // past the last stage the loads fetch nothing and the reads are unused
+  auto stage = [&](char* cur, const char* nxt, char* wcur, char* wnxt, int slot, int ktl) {
+    read_frags(cur, wcur, 1, 1);
+    mma_step(0);
+    dequant((slot + 1) % RING, wnxt);
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((RING - 2) * LB) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    issue_loads(cur, slot, ktl + RING);
+    read_frags(nxt, wnxt, 0, 0);
+    mma_step(1);
+  };
+#pragma unroll
+  for (int r = 0; r < RING; ++r) { issue_loads(ring[r], r, r); }
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"((RING - 1) * LB) : "memory");
+  dequant(0, wbuf[0]);
+  lds_barrier();
+  read_frags(ring[0], wbuf[0], 0, 0);
+  // (stages run to a multiple of both the ring and the two weight buffers)
+  constexpr int kUn = RING == 3 ? 6 : 4;
+  const int nst_pad = (t.nst + kUn - 1) / kUn * kUn;
+  for (int ktl = 0; ktl < nst_pad; ktl += kUn) {
+#pragma unroll
+    for (int r = 0; r < kUn; ++r) {
+      stage(ring[r % RING], ring[(r + 1) % RING], wbuf[r % 2], wbuf[(r + 1) % 2], r % RING,
+            ktl + r);
+    }
+  }
+  // no load may still be writing LDS when the epilogue reuses it
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  char* const half[2] = {ring[0], ring[1]};
+  gemm_epilogue<Mma, E, WN, BM, BN>(B, P, t, wm, wn, lane, acc, half, nullptr);
+}
+
+template <int BM, int RING, int QB, int GRP>
+__global__ __launch_bounds__(128 * kMidWN, 1) void
+mid_pack_kernel(const GemmBatch B)
+{
+  constexpr int kBytes = BM * kKB;
+  __shared__ __attribute__((aligned(1024))) char lds0[kBytes];
+  __shared__ __attribute__((aligned(1024))) char lds1[kBytes];
+  __shared__ __attribute__((aligned(1024))) char lds2[kBytes];
+  __shared__ __attribute__((aligned(1024))) char lds3[RING == 4 ? kBytes : 16];
+  __shared__ __attribute__((aligned(1024))) char w0[kMidBN * kKB];
+  __shared__ __attribute__((aligned(1024))) char w1[kMidBN * kKB];
+  char* const wbuf[2] = {w0, w1};
+  const int items = grid_blocks(B);
+  const int G = gridDim.x;
+  const int b = blockIdx.x;
+  for (int base = 0; base < items; base += G) {
+    const int R = min(G, items - base);
+    int w = base + b;
+    if (G % 8 == 0) {
+      const int x = b % 8, i = b / 8;
+      const int lo = x * R / 8, hi = (x + 1) * R / 8;
+      if (i >= hi - lo) { break; }
+      w = base + lo + i;
+    } else if (b >= R) {
+      break;
+    }
+    if constexpr (RING == 4) {
+      char* const ring[4] = {lds0, lds1, lds2, lds3};
+      mid_pack_tile<BM, 4, QB, GRP>(B, ring, wbuf, w);
+    } else {
+      char* const ring[3] = {lds0, lds1, lds2};
+      mid_pack_tile<BM, 3, QB, GRP>(B, ring, wbuf, w);
+    }
+  }
+}
+
 template <class Mma, Epi E, int BM, int RING>
 __global__ __launch_bounds__(128 * kMidWN, 1) void
 mid_gemm_kernel(const GemmBatch B)
@@ -4054,6 +4268,35 @@ launch_mid(const GemmBatch& b, int cus, hipStream_t s, const GemmEvents& ev)
   return hipGetLastError();
 }
 
+template <int BM, int RING, int QB, int GRP>
+hipError_t
+launch_mid_pack(const GemmBatch& b, int cus, hipStream_t s, const GemmEvents& ev)
+{
+  const int items = grid_blocks(b);
+  const int grid = (cus > 0 && cus < items) ? cus : items;
+  launch_timed(mid_pack_kernel<BM, RING, QB, GRP>, dim3(grid), dim3(128 * kMidWN), s, ev.before,
+               ev.after, b);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess || b.split_begin >= b.total_tiles) { return e; }
+  constexpr int kRows = 256 / (kMidBN / 4) * kReduceRowsPerThread;
+  launch_timed(split_reduce_kernel<false, Epi::kBf16, kMidWN, BM, kMidBN>,
+               dim3((b.total_tiles - b.split_begin) * (BM / kRows)), dim3(256), s,
+               ev.red_before, ev.red_after, b);
+  return hipGetLastError();
+}
+
+template <int QB, int GRP>
+hipError_t
+launch_mid_pack_bm(const GemmBatch& b, int cus, hipStream_t s, const GemmEvents& ev)
+{
+  switch (b.bm) {
+    case 128: return launch_mid_pack<128, 4, QB, GRP>(b, cus, s, ev);
+    case 192: return launch_mid_pack<192, 3, QB, GRP>(b, cus, s, ev);
+    case 256: return launch_mid_pack<256, 3, QB, GRP>(b, cus, s, ev);
+    default: return hipErrorInvalidValue;
+  }
+}
+
 template <class Mma, Epi E>
 hipError_t
 launch_mid_bm(const GemmBatch& b, int cus, hipStream_t s, const GemmEvents& ev)
@@ -4242,6 +4485,20 @@ launch_gemm_bf16(const GemmBatch& b, Epi epi, const GemmShape& g,
       return launch_gemm_waves<MmaBf16, Epi::kSwiglu>(b, g, s, ev);
     default: return hipErrorInvalidValue;
   }
+}
+
+hipError_t
+launch_gemm_pack(const GemmBatch& b, int bits, int group, const GemmShape& g, hipStream_t s,
+                 const GemmEvents& ev)
+{
+  if (b.total_tiles <= 0) { return hipSuccess; }
+  if (b.bn != kMidBN || b.kbytes % 128 != 0) { return hipErrorInvalidValue; }
+  if (bits == 8) {
+    return group == 64 ? launch_mid_pack_bm<8, 64>(b, g.cus, s, ev)
+                       : launch_mid_pack_bm<8, 32>(b, g.cus, s, ev);
+  }
+  return group == 64 ? launch_mid_pack_bm<4, 64>(b, g.cus, s, ev)
+                     : launch_mid_pack_bm<4, 32>(b, g.cus, s, ev);
 }
 
 hipError_t
@@ -4825,6 +5082,18 @@ kernels_loadable()
       reinterpret_cast<const void*>(&narrow_pack_kernel<8, 64, 4, true>),
       reinterpret_cast<const void*>(&narrow_pack_kernel<8, 64, 8, true>),
       reinterpret_cast<const void*>(&narrow_pack_kernel<8, 64, 8, false>),
+      reinterpret_cast<const void*>(&mid_pack_kernel<128, 4, 4, 32>),
+      reinterpret_cast<const void*>(&mid_pack_kernel<192, 3, 4, 32>),
+      reinterpret_cast<const void*>(&mid_pack_kernel<256, 3, 4, 32>),
+      reinterpret_cast<const void*>(&mid_pack_kernel<128, 4, 4, 64>),
+      reinterpret_cast<const void*>(&mid_pack_kernel<192, 3, 4, 64>),
+      reinterpret_cast<const void*>(&mid_pack_kernel<256, 3, 4, 64>),
+      reinterpret_cast<const void*>(&mid_pack_kernel<128, 4, 8, 32>),
+      reinterpret_cast<const void*>(&mid_pack_kernel<192, 3, 8, 32>),
+      reinterpret_cast<const void*>(&mid_pack_kernel<256, 3, 8, 32>),
+      reinterpret_cast<const void*>(&mid_pack_kernel<128, 4, 8, 64>),
+      reinterpret_cast<const void*>(&mid_pack_kernel<192, 3, 8, 64>),
+      reinterpret_cast<const void*>(&mid_pack_kernel<256, 3, 8, 64>),
       reinterpret_cast<const void*>(&skinny_reduce_kernel<kElBf16, false>),
       reinterpret_cast<const void*>(&skinny_reduce_kernel<kElBf16, true>),
   };
