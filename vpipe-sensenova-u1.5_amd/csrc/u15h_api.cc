@@ -1284,11 +1284,13 @@ u15h_dequant_affine(u15h_ctx* ctx, u15h_stream stream, const u15h_qweight* w,
 // bits, 256 at 4.  Every row tile dequantises the weights again, and the
 // expansion costs 17 us for 16 million of them.  Expansion / direct, us in a
 // graph, K = 4096 (N = 4096 | 6144 | 12288) and K = 12288 (N = 4096): w8g64
-// 129 rows 34.3/24.8 | 46.2/31.8 | 75.2/49.5 and 74.1/42.0; 300 rows 40.6/31.7
-// | 53.1/48.9 | 79.5/71.7 and 86.4/68.0; 384 rows 45.0/32.9 | 54.4/50.7 |
-// 82.5/74.5 and 93.6/70.6; 512 rows 42.4/40.2 | 53.1/61.5 | 91.8/82.4 and
-// 102/81.  w4g32 256 rows 37.0/28.1 | 47.2/37.3 | 60.0/57.3 and 77.1/50.1;
-// 384 rows 39.9/33.8 | 46.4/47.7 | 71.7/70.7 and 81.7/68.6.
+// 129 rows 34.3/22.0 | 46.2/30.8 | 75.2/48.6 and 74.1/43.7; 300 rows 40.6/29.6
+// | 53.1/46.3 | 79.5/70.4 and 86.4/66.9; 384 rows 45.0/31.5 | 54.4/47.8 |
+// 82.5/71.7 and 93.6/68.5.  w4g32 129 rows 33.0/23.8 | 38.9/29.5 | 61.6/45.2
+// and 62.7/40.9; 256 rows 37.0/26.7 | 47.2/35.7 | 60.0/56.0 and 77.1/48.2.
+// Above, with three stages in flight instead of four, some lost: w8g64 512
+// rows 42.4/40.2 | 53.1/61.5 | 91.8/82.4 and 102/81; w4g32 384 rows 39.9/33.8
+// | 46.4/47.7 | 71.7/70.7 and 81.7/68.6.
 static bool
 plan_pack(const u15h_ctx* ctx, const u15h_qweight* w, int M, int K, GemmBatch& b)
 {

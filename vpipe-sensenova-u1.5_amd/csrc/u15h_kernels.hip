@@ -1282,15 +1282,18 @@ mid_tile(const GemmBatch& B, char* const (&ring)[RING], float* scl, int item)
 // multiply, then an add, then bf16), one stage ahead into one of two LDS
 // buffers laid out as mid_tile's weights; tiles, K order and sums are the
 // dense kernel's, so the result equals it on the expansion bit for bit.  A
-// lane holds 16 codes of one row and their scale and bias, loaded RING
+// lane holds 16 codes of one row and their scale and bias, loaded four
 // stages ahead into registers.  What it saves is the expansion: its launch and
 // 2 x 2 bytes a weight through memory.  300 rows, K = N = 4096, w8g64: 40.6 us
-// expanded, 31.7 here (the dense product alone 24).  The codes copied to LDS
+// expanded, 29.6 here (the dense product alone 24).  The codes copied to LDS
 // and every wave dequantising its own fragments (each weight once per row half
-// and tile) was bound by that: 38.8.
-template <int BM, int RING, int QB, int GRP>
+// and tile) was bound by that: 38.8.  Four stages in flight at every size (at
+// 256 rows the ring and the weight buffers fill the 160 KB): three, as the
+// dense tiles of 192 and 256 rows have, leave the codes, which are wanted a
+// stage earlier, one stage short: 31.7.
+template <int BM, int QB, int GRP>
 __device__ __forceinline__ void
-mid_pack_tile(const GemmBatch& B, char* const (&ring)[RING], char* const (&wbuf)[2], int item)
+mid_pack_tile(const GemmBatch& B, char* const (&ring)[4], char* const (&wbuf)[2], int item)
 {
   using Mma = MmaBf16x16;
   constexpr Epi E = Epi::kBf16;
@@ -1300,6 +1303,7 @@ mid_pack_tile(const GemmBatch& B, char* const (&ring)[RING], char* const (&wbuf)
   constexpr int FI = NW / Mma::kF, FJ = HM / Mma::kF;
   constexpr int LA = BM / 8 / kWaves;               // activation copies per wave
   constexpr int LB = LA + 3;                        // loads per wave and stage
+  constexpr int RING = 4;
   constexpr int kSub = KB / Mma::kKBytes;
   constexpr int kGroups = 64 / Mma::kF;
   const int kbytes = B.kbytes;
@@ -1439,14 +1443,11 @@ mid_pack_tile(const GemmBatch& B, char* const (&ring)[RING], char* const (&wbuf)
   dequant(0, wbuf[0]);
   lds_barrier();
   read_frags(ring[0], wbuf[0], 0, 0);
-  // (stages run to a multiple of both the ring and the two weight buffers)
-  constexpr int kUn = RING == 3 ? 6 : 4;
-  const int nst_pad = (t.nst + kUn - 1) / kUn * kUn;
-  for (int ktl = 0; ktl < nst_pad; ktl += kUn) {
+  const int nst_pad = (t.nst + RING - 1) / RING * RING;
+  for (int ktl = 0; ktl < nst_pad; ktl += RING) {
 #pragma unroll
-    for (int r = 0; r < kUn; ++r) {
-      stage(ring[r % RING], ring[(r + 1) % RING], wbuf[r % 2], wbuf[(r + 1) % 2], r % RING,
-            ktl + r);
+    for (int r = 0; r < RING; ++r) {
+      stage(ring[r], ring[(r + 1) % RING], wbuf[r % 2], wbuf[(r + 1) % 2], r, ktl + r);
     }
   }
   // no load may still be writing LDS when the epilogue reuses it
@@ -1455,7 +1456,7 @@ mid_pack_tile(const GemmBatch& B, char* const (&ring)[RING], char* const (&wbuf)
   gemm_epilogue<Mma, E, WN, BM, BN>(B, P, t, wm, wn, lane, acc, half, nullptr);
 }
 
-template <int BM, int RING, int QB, int GRP>
+template <int BM, int QB, int GRP>
 __global__ __launch_bounds__(128 * kMidWN, 1) void
 mid_pack_kernel(const GemmBatch B)
 {
@@ -1463,7 +1464,7 @@ mid_pack_kernel(const GemmBatch B)
   __shared__ __attribute__((aligned(1024))) char lds0[kBytes];
   __shared__ __attribute__((aligned(1024))) char lds1[kBytes];
   __shared__ __attribute__((aligned(1024))) char lds2[kBytes];
-  __shared__ __attribute__((aligned(1024))) char lds3[RING == 4 ? kBytes : 16];
+  __shared__ __attribute__((aligned(1024))) char lds3[kBytes];
   __shared__ __attribute__((aligned(1024))) char w0[kMidBN * kKB];
   __shared__ __attribute__((aligned(1024))) char w1[kMidBN * kKB];
   char* const wbuf[2] = {w0, w1};
@@ -1481,13 +1482,8 @@ mid_pack_kernel(const GemmBatch B)
     } else if (b >= R) {
       break;
     }
-    if constexpr (RING == 4) {
-      char* const ring[4] = {lds0, lds1, lds2, lds3};
-      mid_pack_tile<BM, 4, QB, GRP>(B, ring, wbuf, w);
-    } else {
-      char* const ring[3] = {lds0, lds1, lds2};
-      mid_pack_tile<BM, 3, QB, GRP>(B, ring, wbuf, w);
-    }
+    char* const ring[4] = {lds0, lds1, lds2, lds3};
+    mid_pack_tile<BM, QB, GRP>(B, ring, wbuf, w);
   }
 }
 
@@ -4268,13 +4264,13 @@ launch_mid(const GemmBatch& b, int cus, hipStream_t s, const GemmEvents& ev)
   return hipGetLastError();
 }
 
-template <int BM, int RING, int QB, int GRP>
+template <int BM, int QB, int GRP>
 hipError_t
 launch_mid_pack(const GemmBatch& b, int cus, hipStream_t s, const GemmEvents& ev)
 {
   const int items = grid_blocks(b);
   const int grid = (cus > 0 && cus < items) ? cus : items;
-  launch_timed(mid_pack_kernel<BM, RING, QB, GRP>, dim3(grid), dim3(128 * kMidWN), s, ev.before,
+  launch_timed(mid_pack_kernel<BM, QB, GRP>, dim3(grid), dim3(128 * kMidWN), s, ev.before,
                ev.after, b);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || b.split_begin >= b.total_tiles) { return e; }
@@ -4290,9 +4286,9 @@ hipError_t
 launch_mid_pack_bm(const GemmBatch& b, int cus, hipStream_t s, const GemmEvents& ev)
 {
   switch (b.bm) {
-    case 128: return launch_mid_pack<128, 4, QB, GRP>(b, cus, s, ev);
-    case 192: return launch_mid_pack<192, 3, QB, GRP>(b, cus, s, ev);
-    case 256: return launch_mid_pack<256, 3, QB, GRP>(b, cus, s, ev);
+    case 128: return launch_mid_pack<128, QB, GRP>(b, cus, s, ev);
+    case 192: return launch_mid_pack<192, QB, GRP>(b, cus, s, ev);
+    case 256: return launch_mid_pack<256, QB, GRP>(b, cus, s, ev);
     default: return hipErrorInvalidValue;
   }
 }
@@ -5082,18 +5078,18 @@ kernels_loadable()
       reinterpret_cast<const void*>(&narrow_pack_kernel<8, 64, 4, true>),
       reinterpret_cast<const void*>(&narrow_pack_kernel<8, 64, 8, true>),
       reinterpret_cast<const void*>(&narrow_pack_kernel<8, 64, 8, false>),
-      reinterpret_cast<const void*>(&mid_pack_kernel<128, 4, 4, 32>),
-      reinterpret_cast<const void*>(&mid_pack_kernel<192, 3, 4, 32>),
-      reinterpret_cast<const void*>(&mid_pack_kernel<256, 3, 4, 32>),
-      reinterpret_cast<const void*>(&mid_pack_kernel<128, 4, 4, 64>),
-      reinterpret_cast<const void*>(&mid_pack_kernel<192, 3, 4, 64>),
-      reinterpret_cast<const void*>(&mid_pack_kernel<256, 3, 4, 64>),
-      reinterpret_cast<const void*>(&mid_pack_kernel<128, 4, 8, 32>),
-      reinterpret_cast<const void*>(&mid_pack_kernel<192, 3, 8, 32>),
-      reinterpret_cast<const void*>(&mid_pack_kernel<256, 3, 8, 32>),
-      reinterpret_cast<const void*>(&mid_pack_kernel<128, 4, 8, 64>),
-      reinterpret_cast<const void*>(&mid_pack_kernel<192, 3, 8, 64>),
-      reinterpret_cast<const void*>(&mid_pack_kernel<256, 3, 8, 64>),
+      reinterpret_cast<const void*>(&mid_pack_kernel<128, 4, 32>),
+      reinterpret_cast<const void*>(&mid_pack_kernel<192, 4, 32>),
+      reinterpret_cast<const void*>(&mid_pack_kernel<256, 4, 32>),
+      reinterpret_cast<const void*>(&mid_pack_kernel<128, 4, 64>),
+      reinterpret_cast<const void*>(&mid_pack_kernel<192, 4, 64>),
+      reinterpret_cast<const void*>(&mid_pack_kernel<256, 4, 64>),
+      reinterpret_cast<const void*>(&mid_pack_kernel<128, 8, 32>),
+      reinterpret_cast<const void*>(&mid_pack_kernel<192, 8, 32>),
+      reinterpret_cast<const void*>(&mid_pack_kernel<256, 8, 32>),
+      reinterpret_cast<const void*>(&mid_pack_kernel<128, 8, 64>),
+      reinterpret_cast<const void*>(&mid_pack_kernel<192, 8, 64>),
+      reinterpret_cast<const void*>(&mid_pack_kernel<256, 8, 64>),
       reinterpret_cast<const void*>(&skinny_reduce_kernel<kElBf16, false>),
       reinterpret_cast<const void*>(&skinny_reduce_kernel<kElBf16, true>),
   };
