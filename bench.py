@@ -241,6 +241,23 @@ def kernel_label(int8, max_rows=None):
     return f"mot_gemm_kernel<{mma}, {epi}, 4>"
 
 
+def step_kernel(int8, max_rows):
+    """kernel_label for the kernels a step of these rows runs: int8 batches of
+    at most 128 rows per problem take the skinny kernels' int8 form, and
+    from there to ~2000 rows the planner picks the 256 x 256 or the mid-size
+    tiles per launch."""
+    label = kernel_label(int8, max_rows)
+    if not label.startswith("mot_gemm_kernel") or max_rows is None:
+        return label
+    if max_rows <= 128:
+        if not int8 or os.environ.get("U15H_SKINNY", "") == "0":
+            return label
+        return "narrow_dma_kernel (int8)" if max_rows <= 16 else "narrow_lds_kernel (int8)"
+    if max_rows <= 2048 and os.environ.get("U15H_MID", "") != "0":
+        return label + " | mid_gemm_kernel"
+    return label
+
+
 def copy_probe():
     import torch
     src = torch.empty(COPY_PROBE_BYTES // 2, dtype=torch.bfloat16, device="cuda")
@@ -526,7 +543,7 @@ def tier_result(work, ms, k, steps, int8, traffic):
     gbps = nbytes / (kern_ms * 1e-3) / 1e9
     peak, unit = (PEAK_I8, "TOPS") if int8 else (PEAK_BF16, "TFLOP/s")
     roof = dict(_roof(flop_launch, nbytes, rate, gbps, peak, unit),
-                traffic=traffic, kernel=kernel_label(int8, work.get("max_rows")),
+                traffic=traffic, kernel=step_kernel(int8, work.get("max_rows")),
                 avg_launch_ms=round(kern_ms, 5), flop_per_launch=flop_launch,
                 alg_bytes_per_launch=int(nbytes), achieved_GBps=round(gbps, 1),
                 split_reduce_ms_per_step=round(k["post_ms"] / steps, 5))
@@ -755,7 +772,7 @@ def m_sweep(torch, u15h, ops, gen, rounds):
     """The three routes of one projection (K=4096, N=6144, the reference's
     sweep shape, src/u15-metal-ops.h:436-448, 486-502) over row counts:
     dense bf16 (u15h_linear), the w8g64 pack through u15h_linear_q (read
-    directly below the 96-row floor, dequantised once then the dense GEMM
+    directly to 384 rows, above them dequantised once then the dense GEMM
     from it on), and the int8 GEMM on pre-quantised weights (activation
     quantiser included).  Each route rotates enough weight copies to exceed
     twice the Infinity Cache; medians of interleaved rounds.  GB/s counts
@@ -807,7 +824,7 @@ def m_sweep(torch, u15h, ops, gen, rounds):
             wbytes = N * K * (1 if name == "int8" else 2)
             row[name] = {"us_per_call": round(us, 2),
                          "weight_GBps": round(wbytes / (us * 1e-6) / 1e9, 1)}
-        row["linear_q_route"] = "direct" if M < 96 else "dequant_once"
+        row["linear_q_route"] = "direct" if M <= 384 else "dequant_once"
         row["linear_q_over_dense"] = round(row["linear_q"]["us_per_call"]
                                            / row["dense"]["us_per_call"], 3)
         rows.append(row)
