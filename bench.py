@@ -772,8 +772,8 @@ def m_sweep(torch, u15h, ops, gen, rounds):
     """The three routes of one projection (K=4096, N=6144, the reference's
     sweep shape, src/u15-metal-ops.h:436-448, 486-502) over row counts:
     dense bf16 (u15h_linear), the w8g64 pack through u15h_linear_q (read
-    directly to 384 rows, above them dequantised once then the dense GEMM
-    from it on), and the int8 GEMM on pre-quantised weights (activation
+    directly to 384 rows, above them dequantised once then the dense
+    GEMM), and the int8 GEMM on pre-quantised weights (activation
     quantiser included).  Each route rotates enough weight copies to exceed
     twice the Infinity Cache; medians of interleaved rounds.  GB/s counts
     the bf16 weight bytes (N x K x 2; N x K for int8) whatever the route
