@@ -139,13 +139,23 @@ def test_packs_on_the_mid_tiles(ops, contexts, bits, group, M, K, N, bm):
     """Packs of more than 128 rows, read by the tiles (to 256 rows at 4 bits,
     384 at 8) or expanded, with bias: bit-equal to u15h_linear on the
     expansion, at tile edges, one K stage, odd stage counts and splits."""
+    pack_equals_expansion(ops if bm is None else contexts[bm], bits, group, M, K, N)
+
+
+@pytest.mark.parametrize("bits,group,M,K,N", [(4, 32, 224, 87488, 256), (8, 64, 192, 210624, 128)])
+def test_packs_of_long_k(ops, bits, group, M, K, N):
+    """Sizes where the mid-size and the 256 x 256 tiles' estimates are close:
+    the tiles are picked once."""
+    pack_equals_expansion(ops, bits, group, M, K, N)
+
+
+def pack_equals_expansion(o, bits, group, M, K, N):
     rng = np.random.default_rng(M + K + bits + group)
     codes = rng.integers(0, 1 << 32, (N, K * bits // 32), dtype=np.uint64).astype(np.uint32)
     sc, bi = (dev_bf16(rand_bf16_bits(rng, (N, K // group), 0.01)) for _ in range(2))
     qw = (torch.from_numpy(codes.view(np.int32)).cuda(), sc, bi, bits, group)
     x, b = dev_bf16(rand_bf16_bits(rng, (M, K))), dev_bf16(rand_bf16_bits(rng, (N,), 0.5))
     w = torch.empty(N, K, dtype=torch.bfloat16, device="cuda")
-    o = ops if bm is None else contexts[bm]
     o.dequant_affine(qw, N, K, w)
     y, t = (torch.full((M, N), 7.0, dtype=torch.bfloat16, device="cuda") for _ in range(2))
     o.linear_q(x, qw, b, y, M, K, N)

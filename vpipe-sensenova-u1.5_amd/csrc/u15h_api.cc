@@ -274,7 +274,7 @@ pick_tiles(const u15h_ctx* ctx, GemmBatch& b, Epi epi)
   }
 }
 
-// Chooses the tiles and the split-K tail of a batch.  With T
+// Chooses the split-K tail of a batch whose tiles are chosen.  With T
 // tiles on C compute units, the last T % C tiles would run as a last,
 // partial round that leaves most units idle; instead each is cut into
 // S = C / (T % C) shares of its K stages (so the shares fill about one
@@ -282,9 +282,8 @@ pick_tiles(const u15h_ctx* ctx, GemmBatch& b, Epi epi)
 // the context's workspace (allocated on first use), or with `noalloc` to
 // the static scratch, which allocates nothing.
 u15h_status
-plan_split(u15h_ctx* ctx, GemmBatch& b, Epi epi, bool noalloc = false)
+plan_split(u15h_ctx* ctx, GemmBatch& b, bool noalloc = false)
 {
-  pick_tiles(ctx, b, epi);
   b.split = 1;
   b.split_begin = b.total_tiles;
   b.ws = nullptr;
@@ -481,12 +480,13 @@ skinny_launch(u15h_ctx* ctx, const GemmBatch& b, Epi epi, hipStream_t s, bool no
   return launched(ctx, u15h::launch_skinny_bf16(k, s, ev), "skinny_gemm_bf16");
 }
 
-// One launch of the tiled kernel on a planned batch.
+// One launch of the tiled kernel on a batch counted on 256 x 256 tiles.
 u15h_status
 tiled_launch(u15h_ctx* ctx, GemmBatch& b, Epi epi, hipStream_t s, bool noalloc,
              const u15h::GemmEvents& ev, const char* what)
 {
-  const u15h_status st = plan_split(ctx, b, epi, noalloc);
+  pick_tiles(ctx, b, epi);
+  const u15h_status st = plan_split(ctx, b, noalloc);
   if (st != U15H_OK) { return st; }
   const bool int8 = epi == Epi::kI32 || epi == Epi::kDequantBf16;
   return launched(ctx,
@@ -1279,10 +1279,10 @@ u15h_dequant_affine(u15h_ctx* ctx, u15h_stream stream, const u15h_qweight* w,
                   "dequant_affine");
 }
 
-// Plans the mid-size tiles' direct read of a pack into `b` where they are
-// the product's tiles anyway and that beats the expansion: to 384 rows at 8
-// bits, 256 at 4.  Every row tile dequantises the weights again, and the
-// expansion costs 17 us for 16 million of them.  Expansion / direct, us in a
+// Picks the tiles of `b`, a product with a pack, and whether they read the
+// pack directly: where they are mid-size ones and that beats the expansion,
+// to 384 rows at 8 bits, 256 at 4.  Every row tile dequantises the weights
+// again, and the expansion costs 17 us for 16 million of them.  Expansion / direct, us in a
 // graph, K = 4096 (N = 4096 | 6144 | 12288) and K = 12288 (N = 4096): w8g64
 // 129 rows 34.3/22.0 | 46.2/30.8 | 75.2/48.6 and 74.1/43.7; 300 rows 40.6/29.6
 // | 53.1/46.3 | 79.5/70.4 and 86.4/66.9; 384 rows 45.0/31.5 | 54.4/47.8 |
@@ -1347,7 +1347,7 @@ u15h_linear_q(u15h_ctx* ctx, u15h_stream stream, const u15h_bf16* x,
     add_problem(b, x, w->codes, nullptr, y, bias, nullptr, nullptr, M, N, N,
                 u15h::tile_cols(Epi::kBf16));
     if (plan_pack(ctx, w, M, K, b)) {
-      if ((st = plan_split(ctx, b, Epi::kBf16)) != U15H_OK) { return st; }
+      if ((st = plan_split(ctx, b)) != U15H_OK) { return st; }
       return launched(ctx,
                       u15h::launch_gemm_pack(b, w->bits, w->group, ctx->gemm,
                                              as_stream(stream), take_profile_event(ctx)),
