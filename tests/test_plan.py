@@ -58,3 +58,29 @@ def test_packs_keep_the_tiles_of_the_dense_product(plan, cus):
                 p = [re.sub("^pack ", "tiled ", s) for s in p]
             assert p == d, (bits, shape)
         assert direct > len(shapes) // 4
+
+
+def test_attention_splits_where_it_gains(plan):
+    """Key shares of an attention call: none where its partial sums cost more
+    than the keys they spread (times measured unsplit / split in each
+    remark)."""
+    calls = {                                    # hq hkv tq tk d q_offset mode
+        "attn 32 8 600 728 64 128 0": False,     # 12.9 / 20.4
+        "attn 32 8 600 728 128 128 0": False,    # 19.0 / 29.0
+        "attn 64 8 256 756 128 500 0": False,    # 18.3 / 28.0
+        "attn 16 4 1024 1024 64 0 0": False,     # 15.2 / 21.6
+        "attn 32 8 700 828 32 128 0": False,     # 11.2 / 15.7
+        "attn 32 8 333 933 128 600 1": False,    # 21.5 / 25.3
+        "attn 32 8 700 1700 64 1000 1": False,   # 23.3 / 27.1
+        "attn 32 8 512 1212 64 700 2": False,    # 22.2 / 25.4
+        "attn 32 8 1 201 128 200 1": False,
+        "attn 32 8 1 1501 128 1500 1": True,     # 27.5 / 10.1
+        "attn 32 8 41 2345 128 2304 1": True,    # 39.0 / 16.9
+        "attn 32 8 128 3128 128 3000 1": True,   # 50.6 / 27.0
+        "attn 32 8 333 2637 128 2304 0": True,   # 45.5 / 33.6
+        "attn 32 8 600 5600 128 5000 0": True,   # 89.8 / 67.3
+        "attn 16 2 1500 1800 128 300 2": True,   # 61.3 / 45.8
+    }
+    for call, steps in zip(calls, plan(list(calls))):
+        shares = int(launches(steps)[0].split("shares=")[1])
+        assert (shares > 1) == calls[call], (call, steps)

@@ -1510,12 +1510,19 @@ u15h_repack_affine_i8(u15h_ctx* ctx, u15h_stream stream,
 // from measured calls (32 query heads over 8, d = 128, us in a graph, not
 // split / split): 1 query over 200 keys 8.8 / 9.4, over 1500 27.5 / 10.1,
 // over 4000 63.5 / 11.4; 41 over 2345 40.2 / 16.3; 128 over 3128 52.5 /
-// 25.1; 333 over 2333 42.5 / 30.4; 512 over 512 causal 15.0 / 21.3; 700
-// over 1700 50.4 / 48.1.
+// 25.1; 512 over 512 causal 15.0 / 21.3.
 //  - at least 12 key tiles (of the mean query, for the causal masks);
 //  - unsplit workgroups on at most 3/4 of the CUs;
 //  - shares of 1 tile or more (one-wave workgroups, at most 32 shares), 3
-//    (two waves) or 4 (four), two workgroups per CU at most.
+//    (two waves) or 4 (four), two workgroups per CU at most;
+//  - with four waves (more than 64 rows of a kv head), whose partials are
+//    megabytes, the estimate below.  Of 4779 such calls that the lines above
+//    split (10 head shapes, 1-1900 queries after 0-8000 keys, three masks)
+//    368 were slower split, by up to 10 us and 58% (32 heads over 8,
+//    bidirectional, 600 queries over 728 keys: d = 128 19.0 / 29.0, d = 64
+//    12.9 / 20.4, d = 32 10.6 / 14.1); with the estimate 7 are, by at most
+//    2.2 us, and 91 that gained, by 12.4 us at most, stay unsplit.  Of the
+//    1402 calls of fewer rows none was slower.
 static int
 attention_shares(const u15h_ctx* ctx, u15h::AttnArgs a)
 {
@@ -1525,7 +1532,8 @@ attention_shares(const u15h_ctx* ctx, u15h::AttnArgs a)
   const long long blocks = (long long)a.hkv * ((rows + 32 * waves - 1) / (32 * waves));
   long long S = ctx->attn_split;
   if (S < 0) {
-    const long long seen = a.mode == 0 ? a.tk : std::min<long long>(a.tk, a.q_offset + a.tq / 2);
+    const long long seen =
+        a.mode == 0 ? a.tk : std::min<long long>(a.tk, (long long)a.q_offset + a.tq / 2);
     const long long tiles = (seen + 63) / 64;
     if (tiles < 12 || 4LL * a.hq * ((a.tq + 127) / 128) > 3LL * ctx->num_cu) { return 1; }
     S = std::min(waves == 1 ? std::min(tiles, 32LL) : tiles / (waves == 2 ? 3 : 4),
@@ -1534,9 +1542,23 @@ attention_shares(const u15h_ctx* ctx, u15h::AttnArgs a)
   S = std::min<long long>(S, (a.tk + 63) / 64);
   for (; S > 1; --S) {
     a.shares = (int)S;
-    if (u15h::attn_split_ws_bytes(a) <= kAttnWsBytes) { return (int)S; }
+    if (u15h::attn_split_ws_bytes(a) <= kAttnWsBytes) { break; }
   }
-  return 1;
+  if (S > 1 && waves == 4 && ctx->attn_split < 0) {
+    // us, fitted to those calls: the longest workgroup's tiles unsplit (longer
+    // under the block-causal mask), against its share of them at 1.6 times
+    // the cost and the partials' round trip
+    const double tile = a.d == 128 ? 0.9 : a.d == 64 ? 0.62 : 0.52;
+    const double per_mb = a.d == 128 ? 0.45 : 0.8;
+    const long long last =
+        a.mode == 0 ? a.tk : std::min<long long>(a.tk, (long long)a.q_offset + a.tq);
+    const long long T = (last + 63) / 64;
+    const double whole = tile * T * (a.mode != 2 ? 1.0 : a.d == 32 ? 1.2 : 1.3);
+    const double split = 1.6 * tile * ((T + S - 1) / S) +
+                         per_mb * 1e-6 * u15h::attn_split_ws_bytes(a);
+    if (split >= whole) { return 1; }
+  }
+  return (int)std::max(S, 1LL);
 }
 
 static u15h_status
