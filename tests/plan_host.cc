@@ -7,7 +7,9 @@
 //   swiglu M_und M_gen K I | i8 M_und M_gen K N |
 //   attn hq hkv tq tk d q_offset mode
 // each on a context of its own, and prints a line per call: its launches (and
-// device allocations after u15h_create), separated by " ; ", then the status.
+// device allocations after u15h_create, "malloc relaxed" where the thread's
+// capture mode lets a capturing stream's caller allocate), separated by
+// " ; ", then the status.
 // A batch that the kernels would refuse, or whose partial sums do not fit the
 // scratch, is answered as they answer it: with hipErrorInvalidValue.  The
 // first argument is the number of CUs.
@@ -20,6 +22,7 @@ namespace {
 
 int g_cus = 256;
 bool g_created = false;
+hipStreamCaptureMode g_mode = hipStreamCaptureModeGlobal;
 std::string g_out;
 
 void
@@ -195,12 +198,20 @@ hipError_t hipGetLastError(void) { return hipSuccess; }
 hipError_t
 hipMalloc(void** p, size_t)
 {
-  if (g_created) { emit("malloc"); }
+  if (g_created) {
+    emit(g_mode == hipStreamCaptureModeRelaxed ? "malloc relaxed" : "malloc");
+  }
   *p = fake<void>();
   return hipSuccess;
 }
 hipError_t hipSetDevice(int) { return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t
+hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode* mode)
+{
+  std::swap(*mode, g_mode);
+  return hipSuccess;
+}
 
 }  // extern "C"
 

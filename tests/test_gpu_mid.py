@@ -162,3 +162,51 @@ def pack_equals_expansion(o, bits, group, M, K, N):
     o.linear(x, w, b, t, M, K, N)
     torch.cuda.synchronize()
     assert torch.equal(y.view(torch.int16), t.view(torch.int16))
+
+
+@pytest.mark.parametrize("call,Mu,Mg,K,N", [
+    ("linear", 0, 2800, 4096, 3072), ("linear", 333, 1, 2048, 12288),
+    ("swiglu", 333, 1, 2048, 6144), ("i8", 333, 257, 8192, 10240)])
+def test_first_call_of_a_context_under_capture(ops, call, Mu, Mg, K, N):
+    """Mid-size tiles with a split tail where the 256 x 256 ones have none:
+    such a call, captured as a context's first, allocates nothing.  Replays
+    with eager work between them equal the eager result."""
+    g = torch.Generator(device="cuda").manual_seed(Mu + Mg + K)
+    M = Mu + Mg
+
+    def rnd(*shape):
+        return torch.empty(*shape, dtype=torch.bfloat16, device="cuda").normal_(generator=g)
+
+    def codes(*shape):
+        return torch.randint(-127, 128, shape, generator=g, dtype=torch.int8, device="cuda")
+    y = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
+    if call == "i8":
+        xq, q0, q1 = codes(M, K), codes(N, K), codes(N, K)
+        sx, s0, s1 = (torch.rand(n, generator=g, device="cuda") for n in (M, N, N))
+
+        def run(o):
+            o.mot_gemm_i8(xq, sx, Mu, Mg, K, [dict(wq_und=q0, wq_gen=q1, sw_und=s0, sw_gen=s1,
+                                                   y=y)])
+    else:
+        x, w = rnd(M, K), [rnd(N, K) for _ in range(4 if call == "swiglu" else 2)]
+
+        def run(o):
+            if call == "swiglu":
+                o.mot_gate_up_swiglu(x, Mu, Mg, K, *w, y)
+            else:
+                o.mot_linear(x, Mu, Mg, K, [dict(w_und=w[0], w_gen=w[1], y=y)])
+    run(ops)
+    torch.cuda.synchronize()
+    want = y.clone()
+    o = u15h.Ops(0)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        run(o)
+    for _ in range(3):
+        y.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y.view(torch.int16), want.view(torch.int16))
+        run(ops)
+    torch.cuda.synchronize()
+    o.close()

@@ -45,7 +45,8 @@ struct u15h_ctx {
   hipEvent_t prof_quant[2] = {nullptr, nullptr};
   u15h::GemmEvents prof_gemm;
   // Partial-sum workspace of split tiles: at most num_cu K shares of one
-  // 256x256 tile each (allocated on first use, kept until destroy).
+  // 256x256 tile each (allocated on first use, also under stream capture;
+  // kept until destroy).
   void* split_ws = nullptr;
   // The device address of the static split-K scratch that
   // u15h_mot_linear_noalloc uses instead (looked up at create; null if the
@@ -208,6 +209,23 @@ split_ws_capacity(const u15h_ctx* ctx)
   return (size_t)ctx->num_cu * u15h::kBM * u15h::kBN * 4;
 }
 
+// Allocates the context's split-K workspace if it has none.  The first call
+// that splits may be one that a graph is captured from, where hipMalloc is
+// refused and ends the capture unless the thread is in relaxed mode.  The
+// allocation is no stream operation: the graph records the address only.
+u15h_status
+ensure_split_ws(u15h_ctx* ctx)
+{
+  if (ctx->split_ws != nullptr) { return U15H_OK; }
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  const bool relaxed = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+  const hipError_t e = hipMalloc(&ctx->split_ws, split_ws_capacity(ctx));
+  if (relaxed) { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  if (e == hipSuccess) { return U15H_OK; }
+  ctx->split_ws = nullptr;
+  return fail(ctx, U15H_ENOMEM, "split-K workspace of %zu bytes", split_ws_capacity(ctx));
+}
+
 // K shares of a last round of `rem` tiles over C compute units.
 int
 tail_shares(const u15h_ctx* ctx, int rem, int nk)
@@ -309,13 +327,8 @@ plan_split(u15h_ctx* ctx, GemmBatch& b, bool noalloc = false)
     b.ws = ctx->noalloc_ws;
     return U15H_OK;
   }
-  if (ctx->split_ws == nullptr) {
-    if (hipMalloc(&ctx->split_ws, split_ws_capacity(ctx)) != hipSuccess) {
-      ctx->split_ws = nullptr;
-      return fail(ctx, U15H_ENOMEM, "split-K workspace of %zu bytes",
-                  split_ws_capacity(ctx));
-    }
-  }
+  const u15h_status st = ensure_split_ws(ctx);
+  if (st != U15H_OK) { return st; }
   b.ws = ctx->split_ws;
   return split_ws_bytes(b) <= split_ws_capacity(ctx)
              ? U15H_OK
@@ -460,12 +473,8 @@ skinny_launch(u15h_ctx* ctx, const GemmBatch& b, Epi epi, hipStream_t s, bool no
       }
       k.ws = static_cast<float*>(ctx->noalloc_ws);
     } else {
-      if (ctx->split_ws == nullptr &&
-          hipMalloc(&ctx->split_ws, split_ws_capacity(ctx)) != hipSuccess) {
-        ctx->split_ws = nullptr;
-        return fail(ctx, U15H_ENOMEM, "split-K workspace of %zu bytes",
-                    split_ws_capacity(ctx));
-      }
+      const u15h_status st = ensure_split_ws(ctx);
+      if (st != U15H_OK) { return st; }
       k.ws = static_cast<float*>(ctx->split_ws);
     }
     size_t off = 0;
