@@ -80,8 +80,8 @@ def test_exact_sums_equal_the_256_tiles(contexts, bm, Mu, Mg, K, N):
 
 @pytest.mark.parametrize("M,K,N", [(130, 4096, 1032), (333, 4096, 4096), (1100, 1024, 2056)])
 def test_planned_tiles(ops, contexts, M, K, N):
-    """The default context's choice (a mid-size tile at these shapes) on
-    random operands, with bias, at the reference's bars."""
+    """The default context's choice (a mid-size tile at these shapes:
+    test_plan.py) on random operands, with bias, at the reference's bars."""
     rng = np.random.default_rng(M + K + N)
     xb, wb = rand_bf16_bits(rng, (M, K)), rand_bf16_bits(rng, (N, K), 0.02)
     bb = rand_bf16_bits(rng, (N,), 0.5)
@@ -101,8 +101,8 @@ def test_planned_tiles(ops, contexts, M, K, N):
                                        (50, 4096, 320, 4096)])
 def test_few_rows_apart_from_whole_rounds(ops, contexts, Mu, Mg, K, N):
     """A group of at most 128 rows beside one whose 256 x 256 tiles fill whole
-    rounds of 256 CUs runs in a launch of its own: equal bits on exact sums
-    to the one grouped launch, for every epilogue, and in the
+    rounds of 256 CUs runs in a launch of its own (test_plan.py): equal bits
+    on exact sums to the one grouped launch, for every epilogue, and in the
     allocation-free call."""
     rng = np.random.default_rng(Mu + Mg + K)
     M = Mu + Mg

@@ -95,3 +95,39 @@ def test_the_split_workspace_is_allocated_under_capture_too(plan):
     steps = plan(calls)
     assert all(s[-1] == "ok" and "malloc" not in s for s in steps)
     assert sum("malloc relaxed" in s for s in steps) > len(calls) // 3
+
+
+@pytest.mark.parametrize("M,K,N", [(130, 4096, 1032), (333, 4096, 4096), (1100, 1024, 2056)])
+def test_mid_size_tiles_are_planned(plan, M, K, N):
+    """The shapes of test_gpu_mid.py's test_planned_tiles."""
+    (steps,) = plan([f"linear {M} {K} {N}"])
+    (one,) = launches(steps)
+    assert re.match("tiled bf16 (128|192|256)x128 ", one), steps
+
+
+@pytest.mark.parametrize("Mu,Mg,K,N", [(128, 4096, 256, 4096), (1, 2048, 192, 8192),
+                                       (50, 4096, 320, 4096)])
+def test_few_rows_are_planned_apart(plan, Mu, Mg, K, N):
+    """The shapes of test_gpu_mid.py's test of the same name: the larger
+    group's whole rounds, then the few rows on the skinny route.  With a
+    partial last round, or the smaller group above 128 rows, one launch."""
+    calls = ["mot", "swiglu"] + (["i8"] if K % 128 == 0 else [])
+    for steps in plan([f"{c} {Mu} {Mg} {K} {N}" for c in calls]):
+        many, few = launches(steps)
+        assert many.startswith("tiled") and " 256x256 " in many and "tail=0" in many, steps
+        assert few.startswith("skinny") and f"rows={Mu} " in few, steps
+    for steps in plan([f"{c} {mu} {mg} {K} {N}" for c in calls
+                       for mu, mg in ((Mu, Mg - 256), (129, Mg), (Mu, Mg + 1))]):
+        assert len(launches(steps)) == 1, steps
+
+
+@pytest.mark.parametrize("cus", [256, 208, 64, 8])
+def test_every_plan_is_accepted(plan, cus):
+    """Row, column and K counts over the range of the entry points: batches
+    that the kernels take, with partial sums that fit the workspace."""
+    calls = [f"{c} {mu} {mg} {K} {N}" for c in ("mot", "swiglu", "i8")
+             for mu, mg in ((1, 0), (16, 0), (17, 0), (128, 0), (129, 0), (1, 700), (128, 4096),
+                            (0, 1900), (0, 16640), (333, 333))
+             for K in (128, 4096, 12288, 65536, 131072) for N in (8, 264, 4096, 24576, 1 << 20)]
+    for call, steps in zip(calls, plan(calls, cus)):
+        assert steps[-1] == "ok" and launches(steps), (call, steps)
