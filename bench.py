@@ -208,7 +208,8 @@ def step_work(m_und, m_gen, layers):
     quant_bytes = (3 * in_elems + 4 * 4 * M) * layers        # bf16 in, int8 + scale out
     return {"flop": flop, "bf16_bytes": bf16_bytes, "i8_bytes": i8_bytes,
             "quant_bytes": quant_bytes, "gemm_launches": 4 * layers,
-            "quant_launches": 4 * layers, "max_rows": max(m_und, m_gen)}
+            "quant_launches": 4 * layers, "max_rows": max(m_und, m_gen),
+            "few_rows": min(m_und, m_gen)}
 
 
 def kernel_label(int8, max_rows=None):
@@ -241,21 +242,60 @@ def kernel_label(int8, max_rows=None):
     return f"mot_gemm_kernel<{mma}, {epi}, 4>"
 
 
-def step_kernel(int8, max_rows):
+def mid_size_on():
+    """Whether the library plans mid-size tiles (read at u15h_create)."""
+    return (os.environ.get("U15H_MID", "") != "0"
+            and os.environ.get("U15H_WAVES", "") in ("", "8")
+            and os.environ.get("U15H_MFMA16", "") in ("", "1"))
+
+
+def few_rows_apart(max_rows, few_rows, cus=256):
+    """The step's launches that run their smaller group apart, on a skinny
+    kernel inside the same profiled span: the larger group's 256 x 256 tiles
+    fill whole rounds of the CUs."""
+    env = os.environ.get
+    if (not 0 < few_rows <= 128 < max_rows or not mid_size_on()
+            or env("U15H_MID", "") in ("128", "192", "256")
+            or env("U15H_SKINNY", "") == "0" or env("U15H_SPLIT", "") == "0"):
+        return []
+    bands = -(-max_rows // 256)
+    cols = (("q|k|v", NQ + 2 * NKV), ("o", HIDDEN), ("gate|up", 2 * INTER), ("down", HIDDEN))
+    return [name for name, n in cols if bands * (n // 256) % cus == 0]
+
+
+def step_kernel(int8, max_rows, few_rows=0):
     """kernel_label for the kernels a step of these rows runs: int8 batches of
-    at most 128 rows per problem take the skinny kernels' int8 form, and
-    from there to ~2000 rows the planner picks the 256 x 256 or the mid-size
-    tiles per launch."""
+    at most 128 rows per problem take the skinny kernels' int8 form, from
+    there to ~2000 rows the planner picks the 256 x 256 or the mid-size
+    tiles per launch, and few rows beside whole rounds run apart."""
     label = kernel_label(int8, max_rows)
     if not label.startswith("mot_gemm_kernel") or max_rows is None:
         return label
+    skinny = "narrow" if int8 else "skinny"
     if max_rows <= 128:
         if not int8 or os.environ.get("U15H_SKINNY", "") == "0":
             return label
         return "narrow_dma_kernel (int8)" if max_rows <= 16 else "narrow_lds_kernel (int8)"
-    if max_rows <= 2048 and os.environ.get("U15H_MID", "") != "0":
-        return label + " | mid_gemm_kernel"
+    if max_rows <= 2048 and mid_size_on():
+        label += " | mid_gemm_kernel"
+    apart = few_rows_apart(max_rows, few_rows)
+    if apart:
+        build = "dma" if few_rows <= 16 else "lds"
+        label += f" + {skinny}_{build}_kernel ({', '.join(apart)}: the {few_rows} rows)"
     return label
+
+
+def linear_q_route(M):
+    """How u15h_linear_q takes the sweep's w8g64 pack at M rows: read
+    directly on the skinny kernels to 128 rows and on the mid-size tiles to
+    384 (which the planner picks at that N and K), else expanded."""
+    skinny = os.environ.get("U15H_SKINNY", "") != "0"
+    floor = os.environ.get("U15H_Q_MIN_M", "")
+    if floor:
+        return "direct" if skinny and M < min(int(floor), 129) else "dequant_once"
+    if (M <= 128 and skinny) or (M <= 384 and mid_size_on()):
+        return "direct"
+    return "dequant_once"
 
 
 def copy_probe():
@@ -543,7 +583,7 @@ def tier_result(work, ms, k, steps, int8, traffic):
     gbps = nbytes / (kern_ms * 1e-3) / 1e9
     peak, unit = (PEAK_I8, "TOPS") if int8 else (PEAK_BF16, "TFLOP/s")
     roof = dict(_roof(flop_launch, nbytes, rate, gbps, peak, unit),
-                traffic=traffic, kernel=step_kernel(int8, work.get("max_rows")),
+                traffic=traffic, kernel=step_kernel(int8, work.get("max_rows"), work.get("few_rows", 0)),
                 avg_launch_ms=round(kern_ms, 5), flop_per_launch=flop_launch,
                 alg_bytes_per_launch=int(nbytes), achieved_GBps=round(gbps, 1),
                 split_reduce_ms_per_step=round(k["post_ms"] / steps, 5))
@@ -824,7 +864,7 @@ def m_sweep(torch, u15h, ops, gen, rounds):
             wbytes = N * K * (1 if name == "int8" else 2)
             row[name] = {"us_per_call": round(us, 2),
                          "weight_GBps": round(wbytes / (us * 1e-6) / 1e9, 1)}
-        row["linear_q_route"] = "direct" if M <= 384 else "dequant_once"
+        row["linear_q_route"] = linear_q_route(M)
         row["linear_q_over_dense"] = round(row["linear_q"]["us_per_call"]
                                            / row["dense"]["us_per_call"], 3)
         rows.append(row)

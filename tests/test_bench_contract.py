@@ -172,6 +172,31 @@ def test_kernel_label_names_the_skinny_route(monkeypatch):
     assert bench.kernel_label(False, 128) == "mot_gemm_kernel<MmaBf16x16, kBf16, 4>"
 
 
+def test_step_kernel_and_pack_route_name_what_runs(monkeypatch):
+    """The few rows that run apart from whole rounds are named beside the
+    tiled kernel, and the pack's route follows the knobs."""
+    for k in ("U15H_WAVES", "U15H_MFMA16", "U15H_SKINNY", "U15H_MID", "U15H_SPLIT",
+              "U15H_Q_MIN_M"):
+        monkeypatch.delenv(k, raising=False)
+    w = bench.step_work(128, 4096, 1)
+    label = bench.step_kernel(False, w["max_rows"], w["few_rows"])
+    assert label == ("mot_gemm_kernel<MmaBf16x16, kBf16, 4> + skinny_lds_kernel "
+                     "(o, gate|up, down: the 128 rows)")
+    assert bench.step_kernel(True, 4096, 9).endswith(
+        " + narrow_dma_kernel (o, gate|up, down: the 9 rows)")
+    assert bench.step_kernel(False, 3584, 128) == bench.kernel_label(False)
+    assert bench.step_kernel(False, 4096, 129) == bench.kernel_label(False)
+    assert bench.step_kernel(False, 1024, 128) == (bench.kernel_label(False)
+                                                   + " | mid_gemm_kernel")
+    routes = [bench.linear_q_route(M) for M in (1, 128, 384, 512)]
+    assert routes == ["direct"] * 3 + ["dequant_once"]
+    monkeypatch.setenv("U15H_MID", "0")
+    assert [bench.linear_q_route(M) for M in (128, 129)] == ["direct", "dequant_once"]
+    assert bench.step_kernel(False, 4096, 128) == bench.kernel_label(False)
+    monkeypatch.setenv("U15H_Q_MIN_M", "96")
+    assert [bench.linear_q_route(M) for M in (95, 96)] == ["direct", "dequant_once"]
+
+
 def test_small_m_rotates_past_the_cache():
     """Below the ridge a pass cycles more than twice the 256 MB Infinity
     Cache of weights; above it one layer is the step."""
