@@ -98,7 +98,7 @@ def test_planned_tiles(ops, contexts, M, K, N):
 
 
 @pytest.mark.parametrize("Mu,Mg,K,N", [(128, 4096, 256, 4096), (1, 2048, 192, 8192),
-                                       (50, 4096, 320, 4096)])
+                                       (50, 4096, 320, 4096), (77, 4096, 256, 4096)])
 def test_few_rows_apart_from_whole_rounds(ops, contexts, Mu, Mg, K, N):
     """A group of at most 128 rows beside one whose 256 x 256 tiles fill whole
     rounds of 256 CUs runs in a launch of its own (test_plan.py): equal bits

@@ -106,12 +106,19 @@ def test_mid_size_tiles_are_planned(plan, M, K, N):
 
 
 @pytest.mark.parametrize("Mu,Mg,K,N", [(128, 4096, 256, 4096), (1, 2048, 192, 8192),
-                                       (50, 4096, 320, 4096)])
+                                       (50, 4096, 320, 4096), (77, 4096, 256, 4096),
+                                       (128, 4096, 1024, 4096)])
 def test_few_rows_are_planned_apart(plan, Mu, Mg, K, N):
     """The shapes of test_gpu_mid.py's test of the same name: the larger
     group's whole rounds, then the few rows on the skinny route.  With a
-    partial last round, or the smaller group above 128 rows, one launch."""
-    calls = ["mot", "swiglu"] + (["i8"] if K % 128 == 0 else [])
+    partial last round, or the smaller group above 128 rows, one launch; int8
+    of a short K with more than 96 rows too, which were slower apart."""
+    calls = ["mot", "swiglu"]
+    if K % 128 == 0 and (Mu <= 96 or K >= 1024):
+        calls.append("i8")
+    elif K % 128 == 0:
+        (steps,) = plan([f"i8 {Mu} {Mg} {K} {N}"])
+        assert len(launches(steps)) == 1, steps
     for steps in plan([f"{c} {Mu} {Mg} {K} {N}" for c in calls]):
         many, few = launches(steps)
         assert many.startswith("tiled") and " 256x256 " in many and "tail=0" in many, steps

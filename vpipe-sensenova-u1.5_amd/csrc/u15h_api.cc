@@ -508,10 +508,15 @@ tiled_launch(u15h_ctx* ctx, GemmBatch& b, Epi epi, hipStream_t s, bool noalloc,
 // the former fill whole rounds of 256 x 256 tiles by themselves and the latter
 // fit the skinny route: the few rows' half-empty tiles would be a split tail
 // of their own, whose every CU streams their weights at once.  4096 + 128
-// rows, together / apart (us in a graph): o 121 / 114.5, gate|up 646 / 641,
-// with SwiGLU 642 / 633, down 332 / 331, int8 down 175 / 167, int8 o 71.5 /
-// 70.9; where the larger problems leave a partial round (q|k|v 178 / 196,
-// every projection at 1024 + 128) the grouped launch is the faster one.
+// rows, together / apart (us in a graph, K = 4096 unless said): o 118.9 /
+// 114.3, gate|up 646 / 641, with SwiGLU 642 / 640, N = 12288 328 / 322, down
+// (K = 12288) 329 / 331, int8 o 72.6 / 72.1, N = 12288 187 / 183, int8 down
+// 173 / 166-170; 1024 + 128, N = 16384, K = 1024 53.9 / 45.5.  Where the
+// larger problems leave a partial round (q|k|v 178 / 196, every projection at
+// 1024 + 128) the grouped launch is the faster one, and so it is for int8
+// below K = 1024, whose grouped tail is one short round, with more than 96
+// rows (128 + 1024, N = 16384, K = 256 20.6 / 21.7; 128 + 4096, N = 12288, K
+// = 512 54.7 / 56.0; 77 rows gain).
 bool
 few_rows_apart(const u15h_ctx* ctx, const GemmBatch& b, Epi epi, GemmBatch* many,
                GemmBatch* few)
@@ -526,6 +531,11 @@ few_rows_apart(const u15h_ctx* ctx, const GemmBatch& b, Epi epi, GemmBatch* many
     to->p[to->nprob++] = b.p[i];
   }
   if (many->nprob == 0 || few->nprob == 0 || !skinny_fits(ctx, *few, epi)) { return false; }
+  if ((epi == Epi::kI32 || epi == Epi::kDequantBf16) && b.kbytes < 1024) {
+    for (int i = 0; i < few->nprob; ++i) {
+      if (few->p[i].rows > 96) { return false; }
+    }
+  }
   set_tiles(*many, epi, u15h::kBM, u15h::kBN);
   set_tiles(*few, epi, u15h::kBM, u15h::kBN);
   return many->total_tiles % ctx->gemm_cus == 0;
