@@ -164,6 +164,39 @@ def pack_equals_expansion(o, bits, group, M, K, N):
     assert torch.equal(y.view(torch.int16), t.view(torch.int16))
 
 
+@pytest.mark.parametrize("bm", [128, 192, 256])
+@pytest.mark.parametrize("M,K,N", [(129, 320, 1000), (200, 4096, 136)])
+@pytest.mark.parametrize("bits,group", [(4, 32), (4, 64), (8, 32), (8, 64)])
+def test_packs_with_odd_scales(contexts, bits, group, M, K, N, bm):
+    """Scales and biases off dword alignment, and an infinite scale and a NaN
+    bias: the same bits as u15h_linear on the expansion, NaN where it has
+    NaN."""
+    rng = np.random.default_rng(M + K + bits + group)
+    codes = rng.integers(0, 1 << 32, (N, K * bits // 32), dtype=np.uint64).astype(np.uint32)
+    sc = rng.random((N, K // group)).astype(np.float32) * 0.01
+    bi = rng.standard_normal((N, K // group)).astype(np.float32) * 0.1
+    sc[3, -1], bi[5, 0] = np.inf, np.nan
+
+    def dev(a):
+        flat = torch.zeros(a.size + 8, dtype=torch.bfloat16, device="cuda")
+        t = flat[1:1 + a.size].view(a.shape)
+        t.copy_(dev_bf16(oracle.f32_to_bf16(a)))
+        return t
+    qw = (torch.from_numpy(codes.view(np.int32)).cuda(), dev(sc), dev(bi), bits, group)
+    x = dev_bf16(rand_bf16_bits(rng, (M, K)))
+    w = torch.empty(N, K, dtype=torch.bfloat16, device="cuda")
+    o = contexts[bm]
+    o.dequant_affine(qw, N, K, w)
+    y, t = (torch.full((M, N), 7.0, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    o.linear_q(x, qw, None, y, M, K, N)
+    o.linear(x, w, None, t, M, K, N)
+    torch.cuda.synchronize()
+    nan = torch.isnan(t)
+    assert torch.equal(torch.isnan(y), nan) and bool(nan[:, [3, 5]].all())
+    assert int(nan.sum()) == 2 * M
+    assert torch.equal(y.view(torch.int16)[~nan], t.view(torch.int16)[~nan])
+
+
 @pytest.mark.parametrize("call,Mu,Mg,K,N", [
     ("linear", 0, 2800, 4096, 3072), ("linear", 333, 1, 2048, 12288),
     ("swiglu", 333, 1, 2048, 6144), ("i8", 333, 257, 8192, 10240)])

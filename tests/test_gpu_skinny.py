@@ -163,12 +163,12 @@ def _pack_dev(codes, sc, bi, bits, group):
 @pytest.mark.parametrize("bits,group", [(8, 64), (8, 32), (4, 64), (4, 32)])
 @pytest.mark.parametrize("M", [1, 16, 17, 64, 95, 96])
 def test_linear_q_direct_route(ops, bits, group, M):
-    """Below the row floor (96, the reference's _mma_q_min_m) u15h_linear_q
-    reads the affine pack directly (the reference's steel qmm route,
+    """To 128 rows (the reference: below its row floor of 96, _mma_q_min_m)
+    u15h_linear_q reads the affine pack directly (the reference's steel qmm route,
     src/u15-metal-ops.cc:402-431), dequantising in registers to the
     expansion's bf16 weights: bit-equal to u15h_linear on the expansion
     (which at these rows runs the same skinny kernel), and within the bars
-    of the oracle.  At 96 rows it is dequant-once + the dense route."""
+    of the oracle."""
     K, N = 2048, 328
     w = oracle.randn_mt(bits * 100 + group + M, N * K, 0.05).reshape(N, K)
     codes, sc, bi, _ = oracle.pack_affine(w, bits, group)

@@ -102,7 +102,7 @@ struct GemmEvents {
 hipError_t launch_gemm_bf16(const GemmBatch& b, Epi epi, const GemmShape& g,
                             hipStream_t s, const GemmEvents& ev);
 // One problem whose weight is an affine pack, on the mid-size tiles (b.bn ==
-// kMidBN): K % 64 == 0, at group 32 scales and biases 4-byte aligned.
+// kMidBN): K % 64 == 0, scales and biases 2-byte aligned.
 hipError_t launch_gemm_pack(const GemmBatch& b, int bits, int group, const GemmShape& g,
                             hipStream_t s, const GemmEvents& ev);
 

@@ -572,7 +572,7 @@ gemm_epilogue_staged(const GemmProblem& P, const TileWork& t, int wm, int wn,
     }
   }
   __syncthreads();
-  // Read back: wave w stores tile rows [RW w, RW w + RW) (RW = 256 / waves);
+  // Read back: wave w stores tile rows [RW w, RW w + RW) (RW = BM / waves);
   // 64 / CH rows per instruction, CH lanes per row.
   constexpr int RW = BM / (2 * WN);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -2550,19 +2550,18 @@ sum_halves(float v)
 
 constexpr float kLazy = 8.0f;
 
-// Waves (32 queries each) per attention workgroup.  The causal masks run 4:
-// a workgroup runs to the last key its last query sees, and 256-query
-// workgroups waste more masked keys (causal 12% slower with 8).
-// Bidirectional, a K/V tile in LDS serves 256 queries with 8 waves (one
+// Waves (32 queries each) per workgroup of bidirectional attention; the
+// causal masks run 4: a workgroup runs to the last key its last query sees,
+// and 256-query workgroups waste more masked keys (causal 12% slower with 8).
+// A K/V tile in LDS serves 256 queries with 8 waves (one
 // workgroup per CU) and 128 with 4 (two per CU).  A pair of 4-wave
 // workgroups takes ~1.06 times an 8-wave one's time, a 4-wave one alone on
 // its CU ~0.77 times, so the rounds decide (us, 32 heads, d = 128, queries
 // over queries + 128 keys, 8 / 4 waves): 1024 34.5 / 26.0, 1500 46.5 /
 // 50.3, 2048 72.1 / 74.3, 3000 169.8 / 152.1, 4096 256.1 / 262.4.
 inline int
-attn_waves(int mode, int hq, int tq, int cus)
+attn_waves(int hq, int tq, int cus)
 {
-  if (mode != 0) { return 4; }
   const long long n8 = (long long)hq * ((tq + 255) / 256), n4 = (long long)hq * ((tq + 127) / 128);
   const long long r4 = n4 % (2 * cus);
   const double t8 = (double)((n8 + cus - 1) / cus);
@@ -4379,7 +4378,10 @@ launch_skinny_q(const SkinnyBatch& b, hipStream_t s, const GemmEvents& ev)
   }
 }
 
-// SwiGLU pairs (bf16; b.cols output columns of 2 weight rows each).
+// SwiGLU pairs (bf16; b.cols output columns of 2 weight rows each) and, below,
+// int8.  Above 16 rows a stage of the ring is 2 KiB per 16 rows and 8 KiB of
+// weights per CW: four stages, or three where those leave a CU room for two
+// workgroups (80 KiB each) and four do not.
 hipError_t
 launch_skinny_swiglu(const SkinnyBatch& b, hipStream_t s, const GemmEvents& ev)
 {
@@ -4785,7 +4787,7 @@ launch_attention_d(const AttnArgs& a, hipStream_t s)
     return launch_attention_split<D, MODE, 4>(a, s);
   }
   if constexpr (MODE == 0) {
-    if (attn_waves(MODE, a.hq, a.tq, a.cus) == 8) {
+    if (attn_waves(a.hq, a.tq, a.cus) == 8) {
       hipLaunchKernelGGL((attention_kernel<D, MODE, 8>), dim3(a.hq * ((a.tq + 255) / 256)),
                          dim3(512), 0, s, a);
       return hipGetLastError();
