@@ -370,6 +370,35 @@ def test_keys_split_over_workgroups(hq, hkv, d, tq, prefix, mode, shares):
     assert rel_l2(host_f32(head), ref) < BAR
 
 
+@pytest.mark.parametrize("mode", [0, 1, 2])
+@pytest.mark.parametrize("tq,key", [(1, 5), (9, 300), (33, 640), (70, 699)])
+def test_scores_that_overflow_in_one_share(tq, key, mode):
+    """One key whose scores are past f32's range, or so large that it takes
+    the whole row, in one share of ten: NaN in the rows where the unsplit
+    kernel has NaN, and the other rows as close to its as two orders of the
+    keys are (each within BAR of the exact result)."""
+    hq, hkv, d, prefix = 8, 2, 128, 700
+    tk = prefix + tq
+    g = torch.Generator(device="cuda").manual_seed(tq + key)
+    q, k, v = (torch.empty(*s, dtype=torch.bfloat16, device="cuda").normal_(generator=g)
+               for s in ((tq, hq * d), (hkv, tk, d), (hkv, tk, d)))
+    k[:, key] = 0
+    k[:, key, 0] = 3e38
+    t = torch.arange(tk, dtype=torch.int32, device="cuda")
+    outs = []
+    for shares in (0, 10):
+        o = ctx_with(shares)
+        out = torch.full_like(q, 7.0)
+        o.attention_token_major(q, k, v, out, hq, hkv, tk, mode, t if mode == 2 else None, prefix)
+        torch.cuda.synchronize()
+        o.close()
+        outs.append(out)
+    nan = torch.isnan(outs[0])
+    assert bool(nan.any()) and not bool(nan.all())
+    assert torch.equal(torch.isnan(outs[1]), nan)
+    assert rel_l2(host_f32(outs[1][~nan]), host_f32(outs[0][~nan])) < 2 * BAR
+
+
 @pytest.mark.parametrize("hq,tq", [(4, 1), (4, 127), (4, 128), (4, 129), (4, 257),
                                    (256, 255), (128, 257)])
 def test_bidirectional_workgroup_sizes(ops, hq, tq):

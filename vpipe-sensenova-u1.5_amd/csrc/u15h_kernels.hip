@@ -2993,7 +2993,7 @@ attention_kernel(const AttnArgs A)
     // lane-major: every store writes 1 KiB of consecutive bytes
     const SplitRows ws = split_rows(A.ws, (kvh * ntq + qt) * NWV + wave, share, A.shares, D);
     if (half == 0) { ws.ml[lq] = make_float2(m, l); }
-    if (!qvalid || l == 0.0f) { return; }
+    if (!qvalid || (l == 0.0f && m == -INFINITY)) { return; }
 #pragma unroll
     for (int i = 0; i < D / 8; ++i) {
       const int g = 4 * (i & 3);
@@ -3023,7 +3023,9 @@ attention_kernel(const AttnArgs A)
 // (chunk i of D / 8) of the 32 rows of one row group, lane (half, lq)
 // holding columns 8 i + 4 half .. + 3 of row lq as the kernel's accumulators
 // do.  out = sum_s w_s O_s / sum_s w_s l_s, w_s = exp2((m_s - max m) *
-// scale).  A share that saw no key of a row (l = 0) left no output for it.
+// scale).  A share that saw no key of a row (max -inf, sum 0) left no output
+// for it.  A sum of 0 under a finite max counts: the exponential of a largest
+// score near f32's range can round to 0, and the unsplit kernel's row is then 0.
 // The partials come from the other XCDs' writes, a round trip past L2 each,
 // so the shares are dealt over the W waves (up to kCombineAhead each), whose
 // loads all go out before the first is used; the waves' sums meet in LDS.
@@ -3051,11 +3053,11 @@ attention_combine_kernel(const AttnArgs A, int groups_per_head)
   const int tok = row / G;
   const bool valid = tok < A.tq;
   const float scale = 1.4426950408889634f * rsqrtf((float)D);
-  // adds (m1, l1, o1) to (m, l, o); a share without keys has l = 0
+  // adds (m1, l1, o1) to (m, l, o) unless it saw no key
   auto add = [&](float& m, float& l, f32x4_t& o, float m1, float l1, f32x4_t o1) {
-    if (l1 == 0.0f) { return; }
-    const float mx = l == 0.0f ? m1 : fmaxf(m, m1);
-    const float w0 = l == 0.0f ? 0.0f : __builtin_amdgcn_exp2f((m - mx) * scale);
+    if (l1 == 0.0f && m1 == -INFINITY) { return; }
+    const float mx = fmaxf(m, m1);
+    const float w0 = __builtin_amdgcn_exp2f((m - mx) * scale);   // 0 while m is -inf
     const float w1 = __builtin_amdgcn_exp2f((m1 - mx) * scale);
     l = l * w0 + l1 * w1;
 #pragma unroll
@@ -3070,7 +3072,7 @@ attention_combine_kernel(const AttnArgs A, int groups_per_head)
 #pragma unroll
     for (int j = 0; j < kCombineAhead; ++j) {
       const int s = s0 + j * W;
-      ml[j] = make_float2(0.0f, 0.0f);
+      ml[j] = make_float2(-INFINITY, 0.0f);
       o[j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
       if (s < A.shares && valid) {
         const SplitRows ws = split_rows(A.ws, rg, s, A.shares, D);
