@@ -1539,8 +1539,8 @@ u15h_repack_affine_i8(u15h_ctx* ctx, u15h_stream stream,
 //    split (10 head shapes, 1-1900 queries after 0-8000 keys, three masks)
 //    368 were slower split, by up to 10 us and 58% (32 heads over 8,
 //    bidirectional, 600 queries over 728 keys: d = 128 19.0 / 29.0, d = 64
-//    12.9 / 20.4, d = 32 10.6 / 14.1); with the estimate 7 are, by at most
-//    2.2 us, and 91 that gained, by 12.4 us at most, stay unsplit.  Of the
+//    12.9 / 20.4, d = 32 10.6 / 14.1); with the estimate 12 are, by at most
+//    2.5 us, and 52 that gained, by at most 4.9 us, stay unsplit.  Of the
 //    1402 calls of fewer rows none was slower.
 static int
 attention_shares(const u15h_ctx* ctx, u15h::AttnArgs a)
@@ -1564,17 +1564,21 @@ attention_shares(const u15h_ctx* ctx, u15h::AttnArgs a)
     if (u15h::attn_split_ws_bytes(a) <= kAttnWsBytes) { break; }
   }
   if (S > 1 && waves == 4 && ctx->attn_split < 0) {
-    // us, fitted to those calls: the longest workgroup's tiles unsplit (longer
-    // under the block-causal mask), against its share of them at 1.6 times
-    // the cost and the partials' round trip
-    const double tile = a.d == 128 ? 0.9 : a.d == 64 ? 0.62 : 0.52;
-    const double per_mb = a.d == 128 ? 0.45 : 0.8;
+    // us, fitted to those calls: the longest workgroup's tiles unsplit, longer
+    // under the block-causal mask and more so those that it cuts, against its
+    // share of them, dearer with two workgroups on a CU, and the partials'
+    // round trip
+    const double tile = a.d == 128 ? 0.92 : a.d == 64 ? 0.63 : 0.515;
     const long long last =
         a.mode == 0 ? a.tk : std::min<long long>(a.tk, (long long)a.q_offset + a.tq);
     const long long T = (last + 63) / 64;
-    const double whole = tile * T * (a.mode != 2 ? 1.0 : a.d == 32 ? 1.2 : 1.3);
-    const double split = 1.6 * tile * ((T + S - 1) / S) +
-                         per_mb * 1e-6 * u15h::attn_split_ws_bytes(a);
+    const double cut = std::max(0.0, T - a.q_offset / 64.0);
+    const double whole = tile * (a.mode == 2 ? 1.3 * T + 0.2 * cut : 1.0 * T);
+    const double share =
+        tile * (1.1 + (blocks * S > ctx->num_cu ? 0.4 : 0.0) + (a.mode == 2 ? 0.2 : 0.0));
+    const double per_mb = a.d == 128 ? 0.45 : 0.65;
+    const double split =
+        1.5 + share * ((T + S - 1) / S) + per_mb * 1e-6 * u15h::attn_split_ws_bytes(a);
     if (split >= whole) { return 1; }
   }
   return (int)std::max(S, 1LL);
