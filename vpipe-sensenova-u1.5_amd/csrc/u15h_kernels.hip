@@ -2580,7 +2580,7 @@ vswz(int r)
 
 // One share's partial results of 32 rows (row group rg) in the split
 // attention's scratch: O as [D / 8][64 lanes] float4, then the rows' running
-// max and sum.
+// max and sum (-1 where the share saw no key of the row).
 struct SplitRows {
   f32x4_t* o;
   float2* ml;
@@ -2992,8 +2992,9 @@ attention_kernel(const AttnArgs A)
   if constexpr (SPLIT) {
     // lane-major: every store writes 1 KiB of consecutive bytes
     const SplitRows ws = split_rows(A.ws, (kvh * ntq + qt) * NWV + wave, share, A.shares, D);
-    if (half == 0) { ws.ml[lq] = make_float2(m, l); }
-    if (!qvalid || (l == 0.0f && m == -INFINITY)) { return; }
+    const bool none = l == 0.0f && m == -INFINITY;    // no key of the share seen
+    if (half == 0) { ws.ml[lq] = make_float2(m, none ? -1.0f : l); }
+    if (!qvalid || none) { return; }
 #pragma unroll
     for (int i = 0; i < D / 8; ++i) {
       const int g = 4 * (i & 3);
@@ -3023,8 +3024,8 @@ attention_kernel(const AttnArgs A)
 // (chunk i of D / 8) of the 32 rows of one row group, lane (half, lq)
 // holding columns 8 i + 4 half .. + 3 of row lq as the kernel's accumulators
 // do.  out = sum_s w_s O_s / sum_s w_s l_s, w_s = exp2((m_s - max m) *
-// scale).  A share that saw no key of a row (max -inf, sum 0) left no output
-// for it.  A sum of 0 under a finite max counts: the exponential of a largest
+// scale).  A share that saw no key of a row left no output for it and a sum of
+// -1.  A sum of 0 under a finite max counts: the exponential of a largest
 // score near f32's range can round to 0, and the unsplit kernel's row is then 0.
 // The partials come from the other XCDs' writes, a round trip past L2 each,
 // so the shares are dealt over the W waves (up to kCombineAhead each), whose
@@ -3053,15 +3054,16 @@ attention_combine_kernel(const AttnArgs A, int groups_per_head)
   const int tok = row / G;
   const bool valid = tok < A.tq;
   const float scale = 1.4426950408889634f * rsqrtf((float)D);
-  // adds (m1, l1, o1) to (m, l, o) unless it saw no key
+  // adds (m1, l1, o1) to (m, l, o) unless it saw no key (the fused operations
+  // are spelled out so that every use rounds alike)
   auto add = [&](float& m, float& l, f32x4_t& o, float m1, float l1, f32x4_t o1) {
-    if (l1 == 0.0f && m1 == -INFINITY) { return; }
+    if (l1 < 0.0f) { return; }
     const float mx = fmaxf(m, m1);
     const float w0 = __builtin_amdgcn_exp2f((m - mx) * scale);   // 0 while m is -inf
     const float w1 = __builtin_amdgcn_exp2f((m1 - mx) * scale);
-    l = l * w0 + l1 * w1;
+    l = __builtin_fmaf(l, w0, l1 * w1);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) { o[e] = o[e] * w0 + o1[e] * w1; }
+    for (int e = 0; e < 4; ++e) { o[e] = __builtin_fmaf(o1[e], w1, o[e] * w0); }
     m = mx;
   };
   float m = -INFINITY, l = 0.0f;
@@ -3072,7 +3074,7 @@ attention_combine_kernel(const AttnArgs A, int groups_per_head)
 #pragma unroll
     for (int j = 0; j < kCombineAhead; ++j) {
       const int s = s0 + j * W;
-      ml[j] = make_float2(-INFINITY, 0.0f);
+      ml[j] = make_float2(0.0f, -1.0f);
       o[j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
       if (s < A.shares && valid) {
         const SplitRows ws = split_rows(A.ws, rg, s, A.shares, D);
@@ -3085,7 +3087,7 @@ attention_combine_kernel(const AttnArgs A, int groups_per_head)
   }
   if constexpr (W > 1) {
     so[wave][lane] = acc;
-    sml[wave][lane] = make_float2(m, l);
+    sml[wave][lane] = make_float2(m, l == 0.0f && m == -INFINITY ? -1.0f : l);
     __syncthreads();
     if (part != 0) { return; }
 #pragma unroll
