@@ -138,3 +138,16 @@ def test_every_plan_is_accepted(plan, cus):
              for K in (128, 4096, 12288, 65536, 131072) for N in (8, 264, 4096, 24576, 1 << 20)]
     for call, steps in zip(calls, plan(calls, cus)):
         assert steps[-1] == "ok" and launches(steps), (call, steps)
+
+
+def test_waves_and_shares_of_few_rows(plan):
+    """The plans of at most 16 rows around the lines of the rule."""
+    calls = {"linear 1 12288 4096": "waves=8 shares=1", "linear 1 12288 4104": "waves=4 shares=1",
+             "linear 1 4096 4104": "waves=4 shares=1", "linear 16 12288 4352": "waves=4 shares=1",
+             "linear 1 4096 1024": "waves=8 shares=1", "linear 8 8192 512": "waves=4 shares=4",
+             "linear 1 8192 768": "waves=4 shares=4", "linear 1 8192 784": "waves=4 shares=2",
+             "linear 1 16384 256": "waves=4 shares=8", "linear 1 16384 264": "waves=4 shares=4",
+             "swiglu 16 0 8192 4352": "waves=4 shares=1"}
+    for call, steps in zip(calls, plan(list(calls))):
+        (one,) = launches(steps)
+        assert one.endswith(calls[call]), (call, steps)

@@ -356,25 +356,30 @@ skinny_fits(const u15h_ctx* ctx, const GemmBatch& b, Epi epi)
 // At most 16 rows: waves per workgroup and K shares of `cb` workgroups of 16
 // columns over nkb K-blocks of 128 bytes.  A share's partial sums cost a
 // second launch (~2.5 us), so shares come only where the columns leave most
-// CUs idle over a long K; eight waves where four would keep too few loads in
-// flight.  Measured in a graph (us, bf16 1 / 16 rows; W x S waves and shares;
-// the earlier rule took 4 waves and shares of at least 32 K-blocks):
+// CUs idle over a long K, more of them the fewer the columns; eight waves
+// where four would keep too few loads in flight and every workgroup has a CU
+// to itself (bf16, 1 row, 4x1 / 8x1 us: N = 4096, K = 12288 23.9 / 21.2, N =
+// 4352 24.2 / 28.9).  Measured in a graph (us, bf16 1 / 16 rows; W x S waves
+// and shares; the earlier rule took 4 waves and shares of at least 32
+// K-blocks):
 //   N = 1024, K = 4096   4x1 6.0 / 7.5  8x1 5.2 / 7.8  4x2 6.8 / 8.0
 //   N = 4096, K = 4096   4x1 10.5 / 10.4  8x1 9.2 / 10.5  4x2 12.0 / 12.6
 //   N = 4096, K = 12288  4x1 23.9 / 24.0  8x1 21.2 / 24.3  4x2 23.5 / 26.1
+//   N = 512, K = 8192    4x2 8.1 (4 rows 8.4)  4x4 6.4 (7.1)
 //   N = 1024, K = 8192   8x1 7.2 / 12.1  4x2 8.1 / 10.2  4x4 8.7 / 9.4
 //   N = 1024, K = 12288  8x1 13.0 / 20.0  4x2 13.7 / 14.9  4x4 10.9 / 11.7
+//   N = 256, K = 16384   4x4 8.1 / 10.2  4x8 5.9 / 7.9
 //   N = 1024, K = 1024   4x1 2.9 / 3.6  8x1 3.1 / 3.8
 // 16 waves were slower than 8 at every shape.
 void
 narrow_plan(const u15h_ctx* ctx, int rows, int nkb, int cb, int* waves, int* shares)
 {
+  const int most = cb <= ctx->num_cu / 16 && nkb >= 256 ? 8 : 4;
+  const int keep = rows > 8 || cb <= 3 * ctx->num_cu / 16 ? 48 : 64;
   int S = 1;
-  while (nkb > 64 && S < 4 && nkb / S > (rows > 8 ? 48 : 64) && 2 * S * cb <= ctx->num_cu) {
-    S *= 2;
-  }
-  const bool few = 3 * cb < 4 * ctx->num_cu;
-  const bool eight = S == 1 && few && nkb >= 64 && (rows <= 4 || 8 * cb >= 5 * ctx->num_cu);
+  while (nkb > 64 && S < most && nkb / S > keep && 2 * S * cb <= ctx->num_cu) { S *= 2; }
+  const bool eight = S == 1 && cb <= ctx->num_cu && nkb >= 64 &&
+                     (rows <= 4 || 8 * cb >= 5 * ctx->num_cu);
   *waves = eight ? 8 : 4;
   *shares = S;
 }
@@ -1307,9 +1312,12 @@ u15h_dequant_affine(u15h_ctx* ctx, u15h_stream stream, const u15h_qweight* w,
 // | 53.1/46.3 | 79.5/70.4 and 86.4/66.9; 384 rows 45.0/31.5 | 54.4/47.8 |
 // 82.5/71.7 and 93.6/68.5.  w4g32 129 rows 33.0/23.8 | 38.9/29.5 | 61.6/45.2
 // and 62.7/40.9; 256 rows 37.0/26.7 | 47.2/35.7 | 60.0/56.0 and 77.1/48.2.
-// Above, with three stages in flight instead of four, some lost: w8g64 512
-// rows 42.4/40.2 | 53.1/61.5 | 91.8/82.4 and 102/81; w4g32 384 rows 39.9/33.8
-// | 46.4/47.7 | 71.7/70.7 and 81.7/68.6.
+// Above, where the product keeps mid-size tiles: w8g64 385 rows 39.9/33.0 |
+// 44.1/49.4 | 83.0/66.5, 512 rows 38.5/36.9 | 44.8/51.4 | 85.4/67.2 and
+// 94.8/70.9, 1024 rows 45.2/54.5 | 63.9/67.3; w4g32 384 rows 34.3/30.3 |
+// 42.5/41.7 | 62.0/58.7 and 65.3/59.2, 512 rows 35.0/36.9 | 44.9/50.4 |
+// 70.6/66.8 and 77.7/69.4, 640 rows, N = 12288 85.3/101.1.  The row counts
+// keep clear of every loss; they leave some gains.
 static bool
 plan_pack(const u15h_ctx* ctx, const u15h_qweight* w, int M, int K, GemmBatch& b)
 {
