@@ -4341,12 +4341,18 @@ launch_narrow_pack_waves(const SkinnyBatch& b, bool wide, hipStream_t s, const G
 
 // Affine packs at most 16 rows.  Scales and biases are loaded by dwords
 // where every row starts on one: 4-byte aligned, an even number of groups.
+// 4-bit packs to K = 1024 stay on the register kernel: four waves then have a
+// stage or two each, and the copies' latency is all there is (w4g32, 1 row,
+// us by lines / into registers: K = 256 N = 1024 4.5 / 3.9, K = 512 N = 12288
+// 8.1 / 6.4; K = 2048 N = 4096 5.8 / 6.8; w4g64, K = 1024 N = 8192, 16 rows
+// 8.5 / 8.0).
 template <int QB>
 hipError_t
 launch_narrow_pack(const SkinnyBatch& b, hipStream_t s, const GemmEvents& ev)
 {
   const uintptr_t at = reinterpret_cast<uintptr_t>(b.p[0].qs) | reinterpret_cast<uintptr_t>(b.p[0].qb);
-  const bool wide = at % 4 == 0 && b.kbytes / 2 / b.qgroup % 2 == 0;
+  const bool wide = at % 4 == 0 && b.kbytes / 2 / b.qgroup % 2 == 0 &&
+                    (QB != 4 || b.kbytes > 2048);
   if (b.qgroup == 32) {
     return b.waves == 4 ? launch_narrow_pack_waves<QB, 32, 4>(b, wide, s, ev)
                         : launch_narrow_pack_waves<QB, 32, 8>(b, wide, s, ev);
