@@ -265,9 +265,10 @@ def few_rows_apart(max_rows, few_rows, cus=256):
 
 def step_kernel(int8, max_rows, few_rows=0):
     """kernel_label for the kernels a step of these rows runs: int8 batches of
-    at most 128 rows per problem take the skinny kernels' int8 form, from
-    there to ~2000 rows the planner picks the 256 x 256 or the mid-size
-    tiles per launch, and few rows beside whole rounds run apart."""
+    at most 128 rows per problem take the skinny kernels' int8 form (above 16
+    rows, that or the mid-size tiles per launch), from there to ~2000 rows the
+    planner picks the 256 x 256 or the mid-size tiles per launch, and few rows
+    beside whole rounds run apart."""
     label = kernel_label(int8, max_rows)
     if not label.startswith("mot_gemm_kernel") or max_rows is None:
         return label
@@ -275,7 +276,9 @@ def step_kernel(int8, max_rows, few_rows=0):
     if max_rows <= 128:
         if not int8 or os.environ.get("U15H_SKINNY", "") == "0":
             return label
-        return "narrow_dma_kernel (int8)" if max_rows <= 16 else "narrow_lds_kernel (int8)"
+        if max_rows <= 16:
+            return "narrow_dma_kernel (int8)"
+        return "narrow_lds_kernel (int8)" + (" | mid_gemm_kernel" if mid_size_on() else "")
     if max_rows <= 2048 and mid_size_on():
         label += " | mid_gemm_kernel"
     apart = few_rows_apart(max_rows, few_rows)

@@ -1,7 +1,8 @@
 """At most 128 rows per weight set through the SwiGLU and int8 forms of the
 skinny kernels (narrow_dma_kernel to 16 rows, narrow_lds_kernel to 128) and
-the workgroups of the 16-row kernels, against the tiled GEMM of a
-context built with U15H_SKINNY=0.  int32 accumulators and dequantised
+the workgroups of the 16-row kernels, on a context built with U15H_SKINNY=2
+(every batch that fits them), against the tiled GEMM of one built with
+U15H_SKINNY=0.  int32 accumulators and dequantised
 outputs are equal bit for bit (exact sums, the same epilogue arithmetic);
 bf16 sums run in another order, so outputs meet the reference's bars
 (max-rel <= 1e-2, rel-L2 < 4e-3, tests/u15-kernels-test.cc:55), and equal
@@ -22,17 +23,30 @@ MAX_REL = 1e-2
 REF_BAR = 4e-3
 
 
-@pytest.fixture(scope="module")
-def tiled():
+def ctx_with(skinny):
+    """A context created with U15H_SKINNY=skinny (read at create)."""
     old = os.environ.get("U15H_SKINNY")
-    os.environ["U15H_SKINNY"] = "0"
+    os.environ["U15H_SKINNY"] = str(skinny)
     try:
-        o = u15h.Ops(0)
+        return u15h.Ops(0)
     finally:
         if old is None:
             del os.environ["U15H_SKINNY"]
         else:
             os.environ["U15H_SKINNY"] = old
+
+
+@pytest.fixture(scope="module")
+def tiled():
+    o = ctx_with(0)
+    yield o
+    torch.cuda.synchronize()
+    o.close()
+
+
+@pytest.fixture(scope="module")
+def ops():
+    o = ctx_with(2)
     yield o
     torch.cuda.synchronize()
     o.close()

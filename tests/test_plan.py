@@ -151,3 +151,25 @@ def test_waves_and_shares_of_few_rows(plan):
     for call, steps in zip(calls, plan(list(calls))):
         (one,) = launches(steps)
         assert one.endswith(calls[call]), (call, steps)
+
+
+def test_swiglu_and_int8_take_the_faster_route(plan):
+    """17 to 128 rows: the skinny kernels or the tiles, whichever is faster
+    (us skinny / tiles, as measured); 16 rows and bf16 stay skinny."""
+    calls = {
+        "swiglu 97 0 1536 128": "tiled",       # 19.2 / 10.9
+        "swiglu 97 0 12288 4352": "tiled",     # 75.0 / 56.0
+        "swiglu 128 0 3072 1024": "tiled",
+        "swiglu 97 0 768 2048": "skinny",      # 12.0 / 12.9
+        "swiglu 17 0 8192 512": "skinny",
+        "swiglu 16 0 8192 128": "skinny",
+        "i8 97 0 3072 128": "tiled",           # 15.8 / 10.4
+        "i8 128 0 16384 4352": "tiled",
+        "i8 97 0 1536 4096": "skinny",         # 10.7 / 12.9
+        "i8 17 0 4096 4096": "skinny",
+        "i8 16 0 3072 128": "skinny",
+        "mot 97 0 3072 128": "skinny",
+    }
+    for call, steps in zip(calls, plan(list(calls))):
+        (one,) = launches(steps)
+        assert one.startswith(calls[call]), (call, steps)

@@ -23,8 +23,10 @@ struct u15h_ctx {
   int num_cu = 256;
   int gemm_cus = 256;        // CUs the tiled GEMM's rounds are planned for
   bool split_on = true;      // env U15H_SPLIT=0 turns the split-K tail off
-  // env U15H_SKINNY=0 keeps batches of <= 128-row problems on the tiled GEMM
+  // env U15H_SKINNY=0 keeps batches of <= 128-row problems on the tiled GEMM,
+  // 2 runs every batch that fits the skinny kernels on them
   bool skinny_on = true;
+  bool skinny_always = false;
   // heads of one token per thread in u15h_mot_attention_prologue (1, 2 or
   // 4; env U15H_PROLOGUE_RPT).  At config 2 (4224 tokens, 32 + 8 + 8
   // heads of 128) 2 measured 21.6-21.9 us against 22.9-24.5 (1) and
@@ -384,17 +386,15 @@ narrow_plan(const u15h_ctx* ctx, int rows, int nkb, int cb, int* waves, int* sha
   *shares = S;
 }
 
-// Launches a batch that skinny_fits on the skinny kernels.
+// The plan of a batch that skinny_fits on the skinny kernels.
 // At most 16 rows: narrow_plan's workgroups.
 // Above: K shares S (a power of two) are added while the
 // workgroups stay within what the CUs hold at once, each share keeps enough
 // K-blocks to fill its waves' prefetch, and the 4-byte partial sums (written
 // and read once) stay at most half the weight bytes: S * rows * 16 <= K
-// bytes.  The partials go to the split-K workspace (or, with `noalloc`, the
-// static scratch); a batch whose partials would not fit takes fewer shares.
-u15h_status
-skinny_launch(u15h_ctx* ctx, const GemmBatch& b, Epi epi, hipStream_t s, bool noalloc,
-              const u15h::GemmEvents& ev, const u15h_qweight* q = nullptr)
+// bytes; a batch whose partials would not fit the scratch takes fewer shares.
+u15h::SkinnyBatch
+plan_skinny(const u15h_ctx* ctx, const GemmBatch& b, Epi epi, const u15h_qweight* q = nullptr)
 {
   u15h::SkinnyBatch k;
   std::memset(&k, 0, sizeof k);
@@ -470,6 +470,16 @@ skinny_launch(u15h_ctx* ctx, const GemmBatch& b, Epi epi, hipStream_t s, bool no
     if (S == 1 || u15h::skinny_ws_floats(k) * 4 <= cap) { break; }
     S /= 2;
   }
+  return k;
+}
+
+// Launches a plan of plan_skinny; its partial sums go to the split-K
+// workspace (or, with `noalloc`, the static scratch).
+u15h_status
+skinny_launch(u15h_ctx* ctx, u15h::SkinnyBatch& k, Epi epi, hipStream_t s, bool noalloc,
+              const u15h::GemmEvents& ev)
+{
+  const int S = k.split;
   if (S > 1) {
     if (noalloc) {
       if (ctx->noalloc_ws == nullptr) {
@@ -546,12 +556,68 @@ few_rows_apart(const u15h_ctx* ctx, const GemmBatch& b, Epi epi, GemmBatch* many
   return many->total_tiles % ctx->gemm_cus == 0;
 }
 
+// Whether a batch of SwiGLU or int8 problems runs faster on its skinny plan
+// than on tiles (bf16 and packs always take it).  To 16 rows it does.  Above,
+// the skinny workgroups of few columns walk a long K by themselves, and just
+// past a step of their K shares half the CUs idle, while the 128-row tiles
+// split K as finely as the CUs allow: at 65-128 rows every second size off
+// the model's widths was faster on tiles (97 rows, us, skinny / tiles: SwiGLU
+// N = 128, K = 1536 19.2 / 10.9, N = 4352, K = 12288 75.0 / 56.0, but N =
+// 2048, K = 768 12.0 / 12.9; int8 N = 128, K = 3072 15.8 / 10.4, but N =
+// 4096, K = 1536 10.7 / 12.9).  The estimates are fitted to
+// 3388 sizes each (17-128 rows, K 128-16384, N 16-12288), to 6% (skinny) and
+// 8% (tiles); the route taken is within 0.5% (SwiGLU) and 0.3% (int8) of the
+// better one on the mean, where the skinny one alone was 7% and 4% off.
+//   skinny: per K-block of a share and workgroup on a CU, a second launch and
+//   the partial sums with K shares, and the weights' bytes;
+//   tiles: per K stage of a round, the reduction (its partial sums, and for
+//   SwiGLU each share), and the weights' bytes.
+bool
+skinny_faster(const u15h_ctx* ctx, const u15h::SkinnyBatch& k, const GemmBatch& b, Epi epi)
+{
+  if (epi == Epi::kBf16 || k.max_rows <= 16 || ctx->skinny_always || !ctx->mid_on ||
+      ctx->mid_bm != 0 || !ctx->split_on) {
+    return true;
+  }
+  const bool sw = epi == Epi::kSwiglu;
+  const double r = (k.max_rows + 31) / 32;
+  double mb = 0;                                   // the weights'
+  for (int i = 0; i < b.nprob; ++i) { mb += 1e-6 * b.kbytes * b.p[i].n * (sw ? 2 : 1); }
+  const int load = (k.total_cb * k.split + ctx->num_cu - 1) / ctx->num_cu;
+  const double walk = (double)(b.kbytes / 128) / k.split * load;
+  const double part = 4e-6 * u15h::skinny_ws_floats(k);
+  const double skinny =
+      sw ? 3.35 + 0.55 * r + (0.11 + 0.11 * r) * walk + 0.12 * part +
+               (load > 1 ? 0.125 : 0.065) * mb + (k.split > 1 ? 3.1 : 0.0)
+         : 3.1 + 0.8 * r + (0.06 + 0.07 * r) * walk + 0.17 * part + 0.07 * mb +
+               (k.split > 1 ? 1.7 : 0.0);
+  GemmBatch t = b;
+  pick_tiles(ctx, t, epi);
+  const int nk = (b.kbytes + u15h::kKB - 1) / u15h::kKB;
+  const int full = t.total_tiles / ctx->gemm_cus, rem = t.total_tiles % ctx->gemm_cus;
+  const int S = tail_shares(ctx, rem, nk);
+  const double stages = full * nk + (rem > 0 ? (nk + S - 1) / S : 0);
+  const bool mid = t.bn == u15h::kMidBN;
+  double tiles = sw ? 5.8 + (mid ? 0.05 : 0.54) * stages + 0.16 * mb
+                    : 6.05 + (mid ? 0.12 : 2.8) * stages + 0.1 * mb;
+  if (S > 1) {
+    const double sums = 4e-6 * rem * S * t.bn * k.max_rows;
+    tiles += sw ? 0.43 + 0.54 * r + 0.35 * sums + 0.44 * S
+                : 1.84 + 0.32 * r + 0.53 * sums + 0.05 * S;
+  }
+  return skinny <= tiles;
+}
+
 // The route of every GEMM entry point's checked, bound batch.
 u15h_status
 run_gemm(u15h_ctx* ctx, GemmBatch& b, Epi epi, hipStream_t s, bool noalloc, const char* what)
 {
   const u15h::GemmEvents ev = take_profile_event(ctx);
-  if (skinny_fits(ctx, b, epi)) { return skinny_launch(ctx, b, epi, s, noalloc, ev); }
+  if (skinny_fits(ctx, b, epi)) {
+    u15h::SkinnyBatch k = plan_skinny(ctx, b, epi);
+    if (skinny_faster(ctx, k, b, epi)) { return skinny_launch(ctx, k, epi, s, noalloc, ev); }
+    return tiled_launch(ctx, b, epi, s, noalloc, ev, what);
+  }
   GemmBatch many, few;
   if (few_rows_apart(ctx, b, epi, &many, &few)) {
     // the profiling pair spans both kernels; the larger problems' whole
@@ -560,7 +626,9 @@ run_gemm(u15h_ctx* ctx, GemmBatch& b, Epi epi, hipStream_t s, bool noalloc, cons
     first.before = ev.before;
     second.before = nullptr;
     const u15h_status st = tiled_launch(ctx, many, epi, s, noalloc, first, what);
-    return st != U15H_OK ? st : skinny_launch(ctx, few, epi, s, noalloc, second);
+    if (st != U15H_OK) { return st; }
+    u15h::SkinnyBatch k = plan_skinny(ctx, few, epi);
+    return skinny_launch(ctx, k, epi, s, noalloc, second);
   }
   return tiled_launch(ctx, b, epi, s, noalloc, ev, what);
 }
@@ -740,6 +808,7 @@ u15h_create(int device, u15h_ctx** out)
   ctx->num_cu = prop.multiProcessorCount > 0 ? prop.multiProcessorCount : 256;
   ctx->split_on = env_int("U15H_SPLIT", 1) != 0;
   ctx->skinny_on = env_int("U15H_SKINNY", 1) != 0;
+  ctx->skinny_always = env_int("U15H_SKINNY", 1) == 2;
   ctx->prologue_rpt = env_int("U15H_PROLOGUE_RPT", 2);
   ctx->q_min_m = std::max(0, std::min(u15h::kSkinnyMaxRows + 1, env_int("U15H_Q_MIN_M", 96)));
   const char* floor = std::getenv("U15H_Q_MIN_M");
@@ -1365,8 +1434,9 @@ u15h_linear_q(u15h_ctx* ctx, u15h_stream stream, const u15h_bf16* x,
     add_problem(b, x, w->codes, nullptr, y, bias, nullptr, nullptr, M, N, N,
                 u15h::tile_cols(Epi::kBf16));
     if (skinny_fits(ctx, b, Epi::kBf16)) {
-      return skinny_launch(ctx, b, Epi::kBf16, as_stream(stream), false,
-                           take_profile_event(ctx), w);
+      u15h::SkinnyBatch k = plan_skinny(ctx, b, Epi::kBf16, w);
+      return skinny_launch(ctx, k, Epi::kBf16, as_stream(stream), false,
+                           take_profile_event(ctx));
     }
   }
   if (!int8) {
