@@ -182,8 +182,9 @@ u15h_status u15h_dequant_affine(u15h_ctx* ctx, u15h_stream stream,
  * qualifies (the reference's linear_mma_q_ re-enters linear_mma_,
  * src/u15-metal-ops.cc:291-300, 393-399).  With the default floor, calls of
  * at most 128 rows that the interception does not take still read the pack
- * directly, and so do calls of at most 384 rows at 8 bits or 256 at 4 where
- * u15h_linear takes a mid-size tile (the same results, faster). */
+ * directly unless it is small, and so do calls of at most 384 rows at 8 bits
+ * or 256 at 4 where u15h_linear takes a mid-size tile (the same results,
+ * faster). */
 u15h_status u15h_linear_q(u15h_ctx* ctx, u15h_stream stream,
                           const u15h_bf16* x, const u15h_qweight* w,
                           const u15h_bf16* bias, u15h_bf16* y,

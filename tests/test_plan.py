@@ -173,3 +173,22 @@ def test_swiglu_and_int8_take_the_faster_route(plan):
     for call, steps in zip(calls, plan(list(calls))):
         (one,) = launches(steps)
         assert one.startswith(calls[call]), (call, steps)
+
+
+def test_small_packs_of_96_rows_and_more_are_expanded(plan):
+    """From the reference's floor of 96 rows small weights are expanded and
+    larger ones read directly; below it all are read directly."""
+    calls = {
+        "pack 4 32 97 1536 256": "expand",     # us 16.7, direct 19.9
+        "pack 8 64 97 3072 128": "expand",     # 18.7, 21.0
+        "pack 4 32 96 1024 512": "expand",
+        "pack 4 32 95 1536 256": "skinny pack",
+        "pack 4 32 97 256 256": "skinny pack",
+        "pack 4 32 128 4096 6144": "skinny pack",
+        "pack 8 64 128 4096 1024": "skinny pack",
+        "pack 8 64 128 4096 12288": "skinny pack",
+    }
+    for call, steps in zip(calls, plan(list(calls))):
+        first, *rest = launches(steps)
+        assert first.startswith(calls[call]), (call, steps)
+        assert [r.split()[0] for r in rest] == (["skinny"] if first == "expand" else [])

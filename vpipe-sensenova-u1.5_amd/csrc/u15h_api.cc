@@ -1372,6 +1372,21 @@ u15h_dequant_affine(u15h_ctx* ctx, u15h_stream stream, const u15h_qweight* w,
                   "dequant_affine");
 }
 
+// Whether a pack of 96 to 128 rows is read directly rather than expanded: the
+// expansion costs a launch and the weights' bytes, dequantising while the
+// product runs ~0.1 us per K-block that a workgroup walks.  Of 2464 sizes each
+// (96-128 rows, K 128-16384, N 16-12288, both groups) 350 were slower direct
+// at 4 bits and 174 at 8 (us, expansion / direct, 97 rows: w4g32 N = 256, K =
+// 1536 16.7 / 19.9, w8g64 N = 128, K = 3072 18.7 / 21.0); with this line, the
+// sizes' own, 16 and 17 are.
+static bool
+pack_direct(const u15h_ctx* ctx, const u15h::SkinnyBatch& k, int K, int N)
+{
+  const int load = (k.total_cb * k.split + ctx->num_cu - 1) / ctx->num_cu;
+  const double walk = (double)(k.kbytes / 128) / k.split * load;
+  return ctx->skinny_always || walk <= 12.5 + (k.qbits == 4 ? 3.1e-6 : 6e-6) * K * N;
+}
+
 // Picks the tiles of `b`, a product with a pack, and whether they read the
 // pack directly: where they are mid-size ones and that beats the expansion,
 // to 384 rows at 8 bits, 256 at 4.  Every row tile dequantises the weights
@@ -1424,10 +1439,10 @@ u15h_linear_q(u15h_ctx* ctx, u15h_stream stream, const u15h_bf16* x,
   // dequantises each weight in registers to exactly the expansion's bf16
   // value, so the product equals u15h_linear on the expansion bit for bit.
   // From the floor to the skinny kernels' 128 rows it is still the faster
-  // way (128 rows, K = 4096, us in a graph, expansion / direct: w8g64 N = 4096
-  // 28.6 / 21.7, N = 12288 73.0 / 53.5; w4g32 N = 6144 34.8 / 32.0), and is
-  // taken where the expansion would go to the bf16 GEMM and the floor is the
-  // default one.
+  // way for all but small weights (128 rows, K = 4096, us in a graph,
+  // expansion / direct: w8g64 N = 4096 28.6 / 21.7, N = 12288 73.0 / 53.5;
+  // w4g32 N = 6144 34.8 / 32.0; pack_direct), and is taken where the expansion
+  // would go to the bf16 GEMM and the floor is the default one.
   const bool int8 = ctx->i8_on && M >= ctx->i8_min_m && K % 128 == 0;
   if (M < ctx->q_min_m || (!ctx->q_min_m_set && !int8)) {
     GemmBatch b = empty_batch(K * 2);
@@ -1435,8 +1450,10 @@ u15h_linear_q(u15h_ctx* ctx, u15h_stream stream, const u15h_bf16* x,
                 u15h::tile_cols(Epi::kBf16));
     if (skinny_fits(ctx, b, Epi::kBf16)) {
       u15h::SkinnyBatch k = plan_skinny(ctx, b, Epi::kBf16, w);
-      return skinny_launch(ctx, k, Epi::kBf16, as_stream(stream), false,
-                           take_profile_event(ctx));
+      if (M < ctx->q_min_m || pack_direct(ctx, k, K, N)) {
+        return skinny_launch(ctx, k, Epi::kBf16, as_stream(stream), false,
+                             take_profile_event(ctx));
+      }
     }
   }
   if (!int8) {
