@@ -6,7 +6,7 @@
 //   linear M K N | pack bits group M K N | mot M_und M_gen K N |
 //   swiglu M_und M_gen K I | i8 M_und M_gen K N |
 //   attn hq hkv tq tk d q_offset mode
-// each on a context of its own, and prints a line per call: its launches (and
+// ("captured" before it: on a capturing stream), each on a context of its own, and prints a line per call: its launches (and
 // device allocations after u15h_create, "malloc relaxed" where the thread's
 // capture mode lets a capturing stream's caller allocate), separated by
 // " ; ", then the status.
@@ -23,6 +23,7 @@ namespace {
 int g_cus = 256;
 bool g_created = false;
 hipStreamCaptureMode g_mode = hipStreamCaptureModeGlobal;
+bool g_capturing = false;
 std::string g_out;
 
 void
@@ -207,6 +208,12 @@ hipMalloc(void** p, size_t)
 hipError_t hipSetDevice(int) { return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t
+hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* status)
+{
+  *status = g_capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
+  return hipSuccess;
+}
+hipError_t
 hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode* mode)
 {
   std::swap(*mode, g_mode);
@@ -224,6 +231,8 @@ main(int argc, char** argv)
     std::istringstream in(line);
     std::string call;
     in >> call;
+    g_capturing = call == "captured";
+    if (g_capturing) { in >> call; }
     int v[7] = {};
     for (int& x : v) { in >> x; }
     g_out.clear();

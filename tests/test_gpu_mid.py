@@ -199,11 +199,13 @@ def test_packs_with_odd_scales(contexts, bits, group, M, K, N, bm):
 
 @pytest.mark.parametrize("call,Mu,Mg,K,N", [
     ("linear", 0, 2800, 4096, 3072), ("linear", 333, 1, 2048, 12288),
-    ("swiglu", 333, 1, 2048, 6144), ("i8", 333, 257, 8192, 10240)])
+    ("swiglu", 333, 1, 2048, 6144), ("i8", 333, 257, 8192, 10240),
+    ("swiglu", 97, 0, 1536, 128), ("i8", 97, 0, 3072, 128), ("pack", 97, 0, 1536, 256)])
 def test_first_call_of_a_context_under_capture(ops, call, Mu, Mg, K, N):
-    """Mid-size tiles with a split tail where the 256 x 256 ones have none:
-    such a call, captured as a context's first, allocates nothing.  Replays
-    with eager work between them equal the eager result."""
+    """Mid-size tiles with a split tail where the 256 x 256 ones have none, few
+    rows on tiles, and a pack that is expanded when not captured: captured as
+    a context's first call.  Replays with eager work between them equal the
+    eager result."""
     g = torch.Generator(device="cuda").manual_seed(Mu + Mg + K)
     M = Mu + Mg
 
@@ -213,7 +215,14 @@ def test_first_call_of_a_context_under_capture(ops, call, Mu, Mg, K, N):
     def codes(*shape):
         return torch.randint(-127, 128, shape, generator=g, dtype=torch.int8, device="cuda")
     y = torch.empty(M, N, dtype=torch.bfloat16, device="cuda")
-    if call == "i8":
+    if call == "pack":
+        rows = torch.randint(-2**31, 2**31 - 1, (N, K // 8), generator=g, dtype=torch.int32,
+                             device="cuda")
+        x, qw = rnd(M, K), (rows, rnd(N, K // 32), rnd(N, K // 32), 4, 32)
+
+        def run(o):
+            o.linear_q(x, qw, None, y, M, K, N)
+    elif call == "i8":
         xq, q0, q1 = codes(M, K), codes(N, K), codes(N, K)
         sx, s0, s1 = (torch.rand(n, generator=g, device="cuda") for n in (M, N, N))
 

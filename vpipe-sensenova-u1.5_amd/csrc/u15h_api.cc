@@ -1379,12 +1379,18 @@ u15h_dequant_affine(u15h_ctx* ctx, u15h_stream stream, const u15h_qweight* w,
 // at 4 bits and 174 at 8 (us, expansion / direct, 97 rows: w4g32 N = 256, K =
 // 1536 16.7 / 19.9, w8g64 N = 128, K = 3072 18.7 / 21.0); with this line, the
 // sizes' own, 16 and 17 are.
+// Under stream capture it is read directly too where the expansion's scratch
+// would have to grow, which a capturing stream refuses (the results are the
+// same either way).
 static bool
-pack_direct(const u15h_ctx* ctx, const u15h::SkinnyBatch& k, int K, int N)
+pack_direct(const u15h_ctx* ctx, const u15h::SkinnyBatch& k, int K, int N, hipStream_t s)
 {
   const int load = (k.total_cb * k.split + ctx->num_cu - 1) / ctx->num_cu;
   const double walk = (double)(k.kbytes / 128) / k.split * load;
-  return ctx->skinny_always || walk <= 12.5 + (k.qbits == 4 ? 3.1e-6 : 6e-6) * K * N;
+  if (ctx->skinny_always || walk <= 12.5 + (k.qbits == 4 ? 3.1e-6 : 6e-6) * K * N) { return true; }
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  return ctx->w_deq_bytes < (size_t)N * K * 2 &&
+         (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone);
 }
 
 // Picks the tiles of `b`, a product with a pack, and whether they read the
@@ -1450,7 +1456,7 @@ u15h_linear_q(u15h_ctx* ctx, u15h_stream stream, const u15h_bf16* x,
                 u15h::tile_cols(Epi::kBf16));
     if (skinny_fits(ctx, b, Epi::kBf16)) {
       u15h::SkinnyBatch k = plan_skinny(ctx, b, Epi::kBf16, w);
-      if (M < ctx->q_min_m || pack_direct(ctx, k, K, N)) {
+      if (M < ctx->q_min_m || pack_direct(ctx, k, K, N, as_stream(stream))) {
         return skinny_launch(ctx, k, Epi::kBf16, as_stream(stream), false,
                              take_profile_event(ctx));
       }
